@@ -207,3 +207,47 @@ def tolerance(case):
     if case["kind"] == "layer":
         return {"rel": 1.5e-3, "max": 8e-3}
     return {"rel": 8e-4, "max": 2e-3}
+
+
+def _dense64(container, device):
+    """The weight of host arrays [k/32][q][n], in 64 bits: W [k][n]."""
+    bits = torch.from_numpy(container["bW"].view("<i4").copy()).to(device)
+    alpha = torch.from_numpy(container["alpha"]).to(device).double()
+    k, n, groups = container["k"], container["n"], container["num_groups"]
+    shifts = torch.arange(32, device=device, dtype=torch.int32).view(1, 32, 1)
+    W = torch.zeros(groups, k // groups, n, dtype=torch.float64, device=device)
+    for b in range(container["q"]):
+        signs = ((bits[:, b, None, :] >> shifts) & 1).view(groups, k // groups, n)
+        W += alpha[:, b, None, :] * (2 * signs - 1)
+        del signs
+    if container["q_bias"] is not None:
+        W += torch.from_numpy(container["q_bias"]).to(device).double()[:, None, :]
+    return W.view(k, n)
+
+
+def exact(case, seed):
+    """What run returns for the inputs of prepare(case, seed), in 64 bits and plain torch."""
+    dev = torch.device("cuda", torch.cuda.current_device())
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(seed)
+    kind, m, shapes = case["kind"], case.get("m", 1), _shapes(case)
+
+    def activations(rows, k):
+        return torch.randn(rows, k, device=dev, generator=gen).half().double()
+
+    if kind == "load":
+        return _dense64(_container(case, case["k"], case["n"], gen), dev).t()
+    if kind == "layer":
+        bias = (torch.randn(case["n"], device=dev, generator=gen) * 0.1).half().double()
+        W = _dense64(_container(case, case["k"], case["n"], gen), dev)
+        return activations(m, case["k"]) @ W + bias
+    if kind == "call":
+        W = _dense64(_container(case, case["k"], case["n"], gen), dev)
+        return activations(m, case["k"]) @ W
+    if kind == "cols":
+        W = _dense64(_container(case, case["k"], case["n"], gen), dev)
+        x = torch.randn(case["k"], m, device=dev, generator=gen).half().double()
+        return W.t() @ x
+    containers = [_container(case, k, n, gen) for k, n in (shapes if kind == "block" else shapes[:1])]
+    xs = [activations(m, k) for k, _ in shapes]
+    return [x @ _dense64(containers[i if kind == "block" else 0], dev) for i, x in enumerate(xs)]
