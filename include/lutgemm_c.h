@@ -83,17 +83,19 @@ int lutgemm_weight_info(const lutgemm_weight *w, lutgemm_weight_info_t *info);
 /* y[r][0..n) = x[r][0..k) * W for r < m, fp16 in / fp16 out, fp32 accumulation, asynchronous
  * on `stream` (a hipStream_t passed as void*, NULL = the default stream).  x and y are
  * device pointers, row-major [m][k] and [m][n], x 16-byte aligned.  The offset term is applied
- * iff the weight was created with q_bias.  No memset of y is needed and none is issued; the
- * call allocates nothing.  The result is deterministic (bit-identical from launch to launch).
+ * iff the weight was created with q_bias.  No memset of y is needed and none is issued; a
+ * call of up to 16 rows allocates nothing.  The result is deterministic (bit-identical from launch to launch).
  * Replaces lutGEMM::matmul(void* output, void* input, nQWeight_fp16&, int m, int algo)
  * (lutGEMM/include/kernels.h:27, lutGEMM/src/kernels.cu:64-71), which for m == 1 runs
  * kernel::nqmv (mv_fp16.hpp:121) or kernel::nqmv_bias (mv_fp16_bias.hpp:143) and for m > 1
  * dequantises the whole weight and calls a library GEMM (kernels.cu:73-79); here every
  * 1 <= m <= LUTGEMM_MAX_BATCH streams the packed weight: m == 1 and m == 2 through the table-lookup
- * kernels (a two-row pass gives each row bit-identical to its own one-row call), m >= 3 through
- * the batch kernel, which takes up to 16 rows per pass over the weight and contracts them on the
+ * kernels (a two-row pass gives each row bit-identical to its own one-row call), 3 to 16 rows through
+ * the batch kernel, which takes them in one pass over the weight and contracts them on the
  * matrix cores while a tile is in registers (any number of planes and any group size; weights of
- * more than four planes with workgroups of exactly eight wavefronts).  Batch results are deterministic and within
+ * more than four planes with workgroups of exactly eight wavefronts), and more rows through a kernel that contracts
+ * a tile with up to 64 of them.  A launch of more than 16 rows that splits k keeps partial sums in memory of the stream's set,
+ * allocated (up to 16 MiB) at the first such launch; under graph capture, where it cannot be, k is not split.  Batch results are deterministic and within
  * the same tolerance, but a row may differ in the last bit from its own one-row call (another order
  * of the fp32 additions).
  * Launches on one stream run one after the other and share one set of split-k accumulators of the
@@ -230,7 +232,7 @@ int lutgemm_weight_plan(const lutgemm_weight *w, int *workgroups, int *waves_per
                         int *k_splits, int *k_blocks_per_group);
 
 /* The same for the launches a call with m activation rows makes (m = 1: the plan above; m = 2:
- * the two-row plan; m >= 3: the batch kernel's plan for passes of min(m, 16) rows).  LUTGEMM_ERR_BAD_SHAPE for m outside
+ * the two-row plan; 3 <= m <= 16: the batch kernel's plan; beyond: that of the kernel for many rows).  LUTGEMM_ERR_BAD_SHAPE for m outside
  * 1..LUTGEMM_MAX_BATCH.  No counterpart in the reference. */
 int lutgemm_weight_plan_for(const lutgemm_weight *w, int m, int *workgroups, int *waves_per_group,
                             int *k_splits, int *k_blocks_per_group);
@@ -241,7 +243,8 @@ int lutgemm_weight_plan_for(const lutgemm_weight *w, int m, int *workgroups, int
  * (1..12 wavefronts per workgroup, 1..min(k/512 rounded up, 128) k-splits). */
 int lutgemm_weight_set_plan(lutgemm_weight *w, int waves_per_group, int k_splits);
 
-/* Override the batch kernel's launch plan (calls with 3 or more rows): 8..16 wavefronts per
+/* Override the batch kernel's launch plan (calls with 3 to 16 rows, and the passes of 16 rows that
+ * lutgemm_matvec_static makes of more): 8..16 wavefronts per
  * workgroup (exactly 8 for weights of more than four planes; fewer than 16 where four scale
  * groups per 128 k leave less LDS) and the k-splits; both 0: back to the automatic choice.
  * LUTGEMM_ERR_BAD_SHAPE if the request cannot be launched.  No launch on the handle may be in

@@ -48,6 +48,7 @@ constexpr int kBuildRounds = 8;  // table parts per k-block (kernels.hip: kBuild
 constexpr int kMaxSplits = 128;  // the split-k arrival count has 8 bits, the sum room for 128 addends
 constexpr int kStreamSlots = 4;  // sets of split-k words per handle: one per stream that launches on it
 constexpr int kRowsPerPass = lutgemm_kernels::kBatchRows;  // activation rows a launch can take (rows of split-k words per set)
+constexpr int kMaxRowsK = 1 << 24;  // the kernel for more rows addresses 64 of them with 32 bits
 constexpr int kTableRows = 2;    // rows per pass of the table-lookup kernels
 constexpr int kStagedColumns = 16;  // column-batched calls up to this m never allocate
 
@@ -72,6 +73,7 @@ struct StreamSet {
     unsigned long long *accum;   // kRowsPerPass x (padded outputs) split-k words, zero between launches
     void *xrows;                 // staging of column-batched activations: xrows_cols rows of k halves,
     int xrows_cols;              //   grown on demand
+    float *partials;             // sums of launches of more than 16 rows that split k: from the first such launch on
     hipEvent_t done;             // recorded behind the set's latest launch (only while done_valid)
     bool done_valid;
     unsigned long long last_use;
@@ -292,6 +294,56 @@ FusedPlan choose_fused_batch_plan(const Shape *const *shapes, const int *rows, i
     return best;
 }
 
+// Launch plan of the kernel for more than 16 rows (rows_body.h): output batches per workgroup (8, or 4 with the
+// wavefronts in two groups along k), row tiles of 16 per workgroup, workgroups along the rows and along k.
+struct RowsPlan { int nw, row_tiles, row_chunks, ntiles, blocks_per_split, k_splits; };
+
+// Sums that split k through memory come in units of 16 rows x 32 outputs (2 KiB).  A launch splits k to fill the
+// device, so some 256 workgroups of 8 batches x 4 row tiles bound what it needs: 16 MiB, less for narrow weights.
+constexpr size_t kPartialUnits = 8192, kPartialUnitBytes = 2048;
+constexpr int kMaxRowsSplits = 32, kMaxSplitChunks = 16;
+size_t partial_units(const Shape &s)
+{
+    const size_t most = (size_t)s.nb * 4 * kMaxSplitChunks * (s.ts < kMaxRowsSplits ? s.ts : kMaxRowsSplits);
+    return most < kPartialUnits ? most : kPartialUnits;
+}
+
+// Cost model in microseconds.  A workgroup's step is eight (batch, k-block) tiles on eight wavefronts.  Alone on its
+// compute unit a step takes 0.65 us per plane and row tile; with the whole device at work the matrix cores are
+// throttled to 0.95 us (both from the plans of four shapes, 7168 x 7168 to 12288 x 12288, two to five planes with the
+// offset counted as one, 17 to 256 rows).  A launch has a fixed part, more for every further round of workgroups, and
+// a k-split adds the exchange of the sums: a round trip, a load per partial sum and the traffic of both.  Over those shapes
+// the choice is within 6 % of the fastest measured plan.
+RowsPlan choose_rows_plan(const Shape &s, int cus, int m, bool may_split)
+{
+    const double kFixed = 8.0, kRound = 4.0, kAlone = 0.65, kThrottled = 0.95, kSplit = 3.0, kSplitEach = 0.3, kPartialBytesPerUs = 4.0e6;
+    const size_t units = partial_units(s);
+    RowsPlan best{};
+    double best_cost = 1e300;
+    for (int rt = lutgemm_kernels::kRowsTilesMin; rt <= lutgemm_kernels::kRowsTilesMax; rt++) {
+        if (rt > lutgemm_kernels::kRowsTilesMin && m <= 16 * (rt - 1)) break;   // an empty row tile
+        const int chunks = div_up(m, 16 * rt);
+        for (int nw = 8; nw >= 4; nw -= 4)
+            for (int ks = 1; ks <= s.ts && ks <= kMaxRowsSplits; ks++) {
+                const int bps = div_up(s.ts, ks);
+                const size_t need = (size_t)s.nb * chunks * rt * ks;
+                if (div_up(s.ts, bps) != ks) continue;   // the same plan as a smaller ks
+                if (ks > 1 && (!may_split || chunks > kMaxSplitChunks || need > units)) break;
+                const int ntiles = div_up(s.nb, nw);
+                const double groups = (double)ntiles * chunks * ks, step = (double)s.qo * rt;
+                const double steps = div_up(bps, lutgemm_kernels::kRowsWaves / nw), rounds = std::ceil(groups / cus);
+                const double alone = rounds * steps * step * kAlone, throttled = groups * steps * step * kThrottled / cus;
+                double cost = kFixed + (rounds - 1.0) * kRound + (alone > throttled ? alone : throttled);
+                if (ks > 1) cost += kSplit + kSplitEach * ks + 2.0 * (double)(need * kPartialUnitBytes) / kPartialBytesPerUs;
+                if (cost < best_cost) {
+                    best_cost = cost;
+                    best = RowsPlan{nw, rt, chunks, ntiles, bps, ks};
+                }
+            }
+    }
+    return best;
+}
+
 // A handle's device memory belongs to the device that was current when it was created.
 int check_device(const lutgemm_weight *w)
 {
@@ -346,11 +398,26 @@ int alloc_workspace(lutgemm_weight *w)
     return alloc_set(w, 0);
 }
 
+// The set's room for partial sums, allocated once (it never moves, so another call on the stream may hold it); null
+// where it is not there and cannot be had: under graph capture, or out of memory.  The caller then does not split k.
+float *partials_of(lutgemm_weight *w, int slot, void *stream)
+{
+    std::lock_guard<std::mutex> lock(w->slot_mutex);
+    StreamSet &t = w->set[slot];
+    if (!t.partials && !stream_capturing(stream) &&
+        hipMalloc((void **)&t.partials, partial_units(w->shape) * kPartialUnitBytes) != hipSuccess) {
+        (void)hipGetLastError();
+        t.partials = nullptr;
+    }
+    return t.partials;
+}
+
 size_t workspace_bytes(const lutgemm_weight *w)
 {
     size_t bytes = 0;
     for (int i = 0; i < kStreamSlots; i++) {
         if (w->set[i].accum) bytes += set_words(w) * sizeof(unsigned long long);
+        if (w->set[i].partials) bytes += partial_units(w->shape) * kPartialUnitBytes;
         if (w->set[i].xrows) bytes += (size_t)w->set[i].xrows_cols * w->shape.k * sizeof(uint16_t);
     }
     return bytes;
@@ -721,6 +788,30 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
     }
     a.x_row_stride = s.k;
     a.accum_row_stride = (long long)s.nb * kBatch;
+    // More rows than a pass of the batch kernel takes: one launch over all of them, except for the allocation-free entry
+    // point (its words hold no partial sums) and for a k beyond the kernel's 32-bit offsets.
+    if (m > kRowsPerPass && !static_ws && s.k <= kMaxRowsK) {
+        RowsPlan plan = choose_rows_plan(s, w->compute_units, m, true);
+        if (plan.k_splits > 1 && !(a.partials = partials_of(mw, slot, stream)))
+            plan = choose_rows_plan(s, w->compute_units, m, false);
+        a.ntiles = plan.ntiles;
+        a.k_splits = plan.k_splits;
+        a.blocks_per_split = plan.blocks_per_split;
+        a.rows = m;
+        a.x = xh;
+        a.y = yh;
+        a.y_stride = cols ? m : 1;   // y [n][m] or [m][n]
+        a.y_row_stride = cols ? 1 : s.n;
+        lutgemm_kernels::RowsGrid g{};
+        g.row_chunks = plan.row_chunks;
+        g.q = s.q;
+        g.gsub = s.gsub;
+        g.wide_y = !cols && s.n % 4 == 0 && ((uintptr_t)y & 7u) == 0;
+        hipError_t e = lutgemm_kernels::launch_rows(s.qo, plan.row_tiles, lutgemm_kernels::kRowsWaves / plan.nw, a, g, st);
+        if (e != hipSuccess) return hip_fail(e, "launch lut_rows_kernel");
+        lease.launched = true;
+        return LUTGEMM_OK;
+    }
     if (m >= 3) {
         // up to 16 rows per pass over the weight on the matrix cores
         const int pass_rows = m < kRowsPerPass ? m : kRowsPerPass;
@@ -1052,6 +1143,7 @@ int lutgemm_weight_destroy(lutgemm_weight *w)
     for (StreamSet &t : w->set) {
         ptrs.push_back(t.accum);
         ptrs.push_back(t.xrows);
+        ptrs.push_back(t.partials);
         if (t.done) (void)hipEventDestroy(t.done);
     }
     for (void *p : ptrs)
@@ -1343,7 +1435,10 @@ int lutgemm_weight_plan_for(const lutgemm_weight *w, int m, int *workgroups, int
     if (m < 1 || m > LUTGEMM_MAX_BATCH)
         return fail(LUTGEMM_ERR_BAD_SHAPE, "m=%d outside 1..%d", m, LUTGEMM_MAX_BATCH);
     Plan p = m == 1 ? w->plan : w->plan2;
-    if (m >= 3) {
+    if (m > kRowsPerPass && w->shape.k <= kMaxRowsK) {
+        const RowsPlan r = choose_rows_plan(w->shape, w->compute_units, m, true);
+        p = Plan{lutgemm_kernels::kRowsWaves, r.ntiles * r.row_chunks, r.blocks_per_split, r.k_splits};
+    } else if (m >= 3) {
         const int pass_rows = m < kRowsPerPass ? m : kRowsPerPass;
         p = w->batch_measured[pass_rows > 8] ? w->plan_batch[pass_rows > 8]
                                               : choose_batch_plan(w->shape, w->compute_units, pass_rows > 8 ? kRowsPerPass : 8);

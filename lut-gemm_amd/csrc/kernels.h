@@ -13,8 +13,9 @@ struct MatvecArgs {
     const uint16_t *scales; // scale tiles (layout.h)
     const void *x;          // fp16 activations, contiguous, 16-byte aligned
     void *y;                // fp16 outputs, element j at y[j * y_stride]
-    unsigned long long *accum;  // [2][nb*32] split-k accumulators (count | flags | fixed-point sum), zero
-                                // between launches; used when k_splits > 1
+    unsigned long long *accum;  // [rows][nb*32] split-k accumulators (count | flags | fixed-point sum), zero
+                                // between launches; used when k_splits > 1 (launch_rows: only counts)
+    float *partials;        // launch_rows with k_splits > 1: partial sums (no initial value)
     int k, n;
     int ts, nb;             // k-blocks, output batches
     int ntiles;             // column tiles = ceil(nb / waves)
@@ -87,6 +88,32 @@ hipError_t launch_batch(int q, int has_offset, int gsub, const MatvecArgs &a, in
 // workgroups = sum of the entries' ntiles * k_splits, entry i starting at first_block[i].
 hipError_t launch_batch_multi(int q, int has_offset, int gsub, const MultiMatvecArgs &m, int workgroups, int waves,
                               hipStream_t stream);
+
+// Many activation rows in one launch (rows_body.h): a workgroup of kRowsWaves wavefronts takes 16 rt rows and
+// kRowsWaves / kw output batches, its wavefronts in kw groups that share out the k-blocks; row_chunks workgroups share
+// a weight tile.  `planes` is q, one more with an offset (1 to 9); rt kRowsTilesMin .. kRowsTilesMax; kw 1 or 2.
+constexpr int kRowsWaves = 8;
+constexpr int kRowsTilesMin = 2, kRowsTilesMax = 4;
+struct RowsGrid {
+    int row_chunks;
+    int q, gsub;
+    int wide_y;   // four neighbouring outputs of a row are 8-byte aligned in y
+};
+// words of 32 k (for each of the four lane groups) that are staged in LDS at a time
+constexpr int rows_stage_words(int rt) { return rt == 2 ? 2 : 1; }
+// bytes of a quarter of one activation row of a stage: every value as the pair (-x, +x), 16 bytes of padding
+constexpr int rows_pitch(int rt) { return rows_stage_words(rt) * 128 + 16; }
+// rows staged by a k group: whole rounds of its wavefronts
+constexpr int rows_staged(int rt, int kw)
+{
+    const int per_round = kRowsWaves / kw * 64 / (16 * rows_stage_words(rt));
+    return (16 * rt + per_round - 1) / per_round * per_round;
+}
+// LDS of a workgroup: two stage buffers per k group and the sign staging of its wavefronts
+constexpr int rows_lds_bytes(int rt, int kw) { return kw * 2 * 4 * rows_staged(rt, kw) * rows_pitch(rt) + kRowsWaves * 1024; }
+static_assert(rows_lds_bytes(2, 2) <= 160 * 1024 && rows_lds_bytes(3, 2) <= 160 * 1024 && rows_lds_bytes(4, 2) <= 160 * 1024, "LDS of a compute unit");
+hipError_t launch_rows(int planes, int rt, int kw, const MatvecArgs &a, const RowsGrid &g, hipStream_t stream);
+hipError_t launch_rows_two_groups(int planes, int rt, const MatvecArgs &a, const RowsGrid &g, hipStream_t stream);   // kw == 2
 
 // words[0..count) = 0 (a fill kernel rather than a memset node, so that it can be captured)
 hipError_t launch_fill_zero(unsigned long long *words, size_t count, hipStream_t stream);

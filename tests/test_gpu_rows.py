@@ -1,0 +1,94 @@
+"""GPU parity of the kernel for more than 16 activation rows: the edges of its tiles (rows, outputs, k-blocks),
+every plane count with and without an offset, every scale layout, splits along k, both forms of the call."""
+import numpy as np
+import pytest
+
+from gpu_util import assert_within_tolerance, run_matvec
+from test_gpu_parity import make, say, truth_of
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # k, n, q, g, offset, rows
+    (32, 1, 1, 32, False, (17,)), (512, 31, 2, 512, True, (17, 32, 33)), (544, 33, 3, 32, True, (48, 49)),
+    (1056, 257, 4, 96, False, (64, 65)), (2048, 264, 5, 64, False, (31, 100)), (1536, 130, 5, 512, True, (50, 130)),
+    (1024, 512, 6, 128, True, (16 * 6 + 1,)), (4096, 100, 7, 32, False, (20, 64)), (2560, 70, 8, 128, True, (17, 40)),
+    (3072, 96, 8, 64, False, (80,)), (49152, 40, 3, 128, False, (18, 63)), (512, 8200, 1, 256, True, (24, 200)),
+]
+
+
+@pytest.mark.parametrize("k,n,q,g,offset,rows", CASES)
+def test_many_rows_kernel(lutgemm, oracle, device, k, n, q, g, offset, rows):
+    from lutgemm import synth
+    w, W = make(lutgemm, synth, k, n, q, g, offset=offset, seed=k + n)
+    x = synth.make_x(max(rows), k, seed=n)
+    truth = truth_of(oracle, w, x)
+    for m in rows:
+        say("case rows", k, n, q, g, offset, "m", m, W.plan(m))
+        y = run_matvec(lutgemm, W, x[:m], device)
+        assert_within_tolerance(y, truth[:m], "m=%d plan=%s" % (m, W.plan(m)))
+        # the same launch again, and the column form, bit for bit (the split-k counts are back at zero)
+        assert np.array_equal(y.view(np.uint16), run_matvec(lutgemm, W, x[:m], device).view(np.uint16))
+        assert np.array_equal(y.view(np.uint16), run_matvec(lutgemm, W, x[:m], device, cols=True).view(np.uint16))
+        # a call of up to 16 rows afterwards finds its split-k words at zero
+        assert_within_tolerance(run_matvec(lutgemm, W, x[:9], device), truth[:9], "9 rows after %d" % m)
+    W.close()
+
+
+@pytest.mark.parametrize("q,g", [(1, 128), (3, 128), (2, 32)])
+def test_many_rows_non_finite_activations(lutgemm, device, q, g):
+    """The pattern of infinities and NaNs is that of the batch kernel, and stays in the rows it belongs to."""
+    from lutgemm import synth
+    k, n, m = 4096, 96, 40
+    w, W = make(lutgemm, synth, k, n, q, g, seed=5)
+    x = synth.make_x(m, k, seed=5)
+    clean = run_matvec(lutgemm, W, x, device)
+    bad = x.copy()
+    bad[3, 700] = np.nan
+    bad[9, 5] = np.inf
+    bad[12, 5], bad[12, 3000] = np.inf, -np.inf
+    say("case rows non-finite", q, g, W.plan(m))
+    y = run_matvec(lutgemm, W, bad, device)
+    few = run_matvec(lutgemm, W, bad[:16], device)
+    for r in (3, 9, 12):
+        assert np.array_equal(np.isnan(y[r]), np.isnan(few[r])), r
+        inf = np.isinf(few[r])
+        assert np.array_equal(y[r][inf], few[r][inf]) and not np.isfinite(y[r]).any(), r
+    rest = [r for r in range(m) if r not in (3, 9, 12)]
+    assert np.array_equal(y[rest].view(np.uint16), clean[rest].view(np.uint16))
+    W.close()
+
+
+def test_many_rows_under_capture_and_on_two_streams(lutgemm, oracle, device):
+    """A capture on a stream whose set has no room for partial sums yet does not split k; once it has, eager launches,
+    replays and a second stream give the same bits."""
+    import torch
+    from lutgemm import synth
+    k, n, q, g, m = 8192, 512, 3, 128, 40
+    w, W = make(lutgemm, synth, k, n, q, g, seed=6)
+    assert W.plan(m)["k_splits"] > 1
+    xs = [torch.from_numpy(synth.make_x(m, k, seed=s)).to(device) for s in (6, 7)]
+    truth = [truth_of(oracle, w, x.cpu().numpy()) for x in xs]
+    static_x, out = xs[0].clone(), torch.zeros((m, n), dtype=torch.float16, device=device)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    for room in (False, True):
+        say("case rows capture", "after an eager call" if room else "first")
+        with torch.cuda.stream(side):
+            W.matvec(static_x.data_ptr(), out.data_ptr(), m if room else 1, side.cuda_stream)
+            side.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                W.matvec(static_x.data_ptr(), out.data_ptr(), m, side.cuda_stream)
+        for rep in range(2):
+            for x, t in zip(xs, truth):
+                static_x.copy_(x)
+                out.zero_()
+                torch.cuda.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert_within_tolerance(out.cpu().numpy(), t, "replay %d" % rep)
+                if room:
+                    eager = run_matvec(lutgemm, W, x.cpu().numpy(), device)
+                    assert np.array_equal(out.cpu().numpy().view(np.uint16), eager.view(np.uint16))
+    W.close()
