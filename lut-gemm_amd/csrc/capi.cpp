@@ -544,50 +544,64 @@ struct SetLease {
 // have left non-zero; the next call on that device clears them first.
 std::atomic<bool> g_static_dirty[lutgemm_kernels::kMaxDevices];
 
-// New handle for shape s on the current device from tiles already in the device layout
-// (host or device memory, `kind` says which).
-int create_from_tiles(const Shape &s, const void *signs, const void *scales, hipMemcpyKind kind,
-                      lutgemm_weight **out)
+// New handle for shape s on the current device, its tiles not yet filled in.
+int new_handle(const Shape &s, lutgemm_weight **out)
 {
     int count = 0;
     hipError_t e = hipGetDeviceCount(&count);
     if (e != hipSuccess || count <= 0)
         return fail(LUTGEMM_ERR_NO_DEVICE, "no HIP device available (%s)",
                     e == hipSuccess ? "device count is 0" : hipGetErrorString(e));
-    int dev = 0;
+    int dev = 0, units = 0;
     e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
-    hipDeviceProp_t prop;
-    e = hipGetDeviceProperties(&prop, dev);
-    if (e != hipSuccess) return hip_fail(e, "hipGetDeviceProperties");
+    e = hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return hip_fail(e, "hipDeviceGetAttribute");
 
     lutgemm_weight *w = new (std::nothrow) lutgemm_weight();
     if (!w) return fail(LUTGEMM_ERR_OUT_OF_MEMORY, "host allocation failed");
     w->shape = s;
     w->device = dev;
-    w->compute_units = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
+    w->compute_units = units > 0 ? units : 256;
 
-    const size_t sb = sign_bytes(s), cb = scale_bytes(s);
     int st = LUTGEMM_OK;
-    e = hipMalloc((void **)&w->d_signs, sb);
+    e = hipMalloc((void **)&w->d_signs, sign_bytes(s));
     if (e != hipSuccess) st = hip_fail(e, "hipMalloc(signs)");
     if (st == LUTGEMM_OK) {
-        e = hipMalloc((void **)&w->d_scales, cb);
+        e = hipMalloc((void **)&w->d_scales, scale_bytes(s));
         if (e != hipSuccess) st = hip_fail(e, "hipMalloc(scales)");
-    }
-    if (st == LUTGEMM_OK) {
-        e = hipMemcpy(w->d_signs, signs, sb, kind);
-        if (e != hipSuccess) st = hip_fail(e, "hipMemcpy(signs)");
-    }
-    if (st == LUTGEMM_OK) {
-        e = hipMemcpy(w->d_scales, scales, cb, kind);
-        if (e != hipSuccess) st = hip_fail(e, "hipMemcpy(scales)");
     }
     if (st == LUTGEMM_OK) {
         w->plan = w->plan2 = choose_plan(s, w->compute_units);
         w->batch_measured[0] = w->batch_measured[1] = false;
         st = alloc_workspace(w);
     }
+    if (st != LUTGEMM_OK) {
+        lutgemm_weight_destroy(w);
+        return st;
+    }
+    *out = w;
+    return LUTGEMM_OK;
+}
+
+int copy_tiles(lutgemm_weight *w, const void *signs, const void *scales, hipMemcpyKind kind)
+{
+    hipError_t e = hipMemcpy(w->d_signs, signs, sign_bytes(w->shape), kind);
+    if (e != hipSuccess) return hip_fail(e, "hipMemcpy(signs)");
+    e = hipMemcpy(w->d_scales, scales, scale_bytes(w->shape), kind);
+    if (e != hipSuccess) return hip_fail(e, "hipMemcpy(scales)");
+    return LUTGEMM_OK;
+}
+
+// New handle for shape s on the current device from tiles already in the device layout
+// (host or device memory, `kind` says which).
+int create_from_tiles(const Shape &s, const void *signs, const void *scales, hipMemcpyKind kind,
+                      lutgemm_weight **out)
+{
+    lutgemm_weight *w = nullptr;
+    int st = new_handle(s, &w);
+    if (st != LUTGEMM_OK) return st;
+    st = copy_tiles(w, signs, scales, kind);
     if (st != LUTGEMM_OK) {
         lutgemm_weight_destroy(w);
         return st;
@@ -634,17 +648,98 @@ int pack_to_host(const Shape &s, const uint32_t *bW, const uint16_t *alpha_h, co
     return LUTGEMM_OK;
 }
 
-int create_common(const uint32_t *bW, const uint16_t *alpha_h, const uint16_t *q_bias_h, int k, int n,
+// The tiles of w from the caller's arrays, re-tiled on the device (pack.hip).  *done stays false, with nothing to undo,
+// where the device has no room for the copies or the weight is beyond the kernels' grids.
+int pack_on_device(lutgemm_weight *w, const uint32_t *bW, const void *alpha, const void *q_bias, bool halves, bool *done)
+{
+    const Shape &s = w->shape;
+    const size_t item = halves ? 2 : 4, words = (size_t)(s.k / 32) * s.q * s.n * sizeof(uint32_t);
+    const size_t scales = (size_t)s.num_groups * s.q * s.n * item, offsets = q_bias ? (size_t)s.num_groups * s.n * item : 0;
+    auto aligned = [](size_t b) { return (b + 255) / 256 * 256; };
+    char *raw = nullptr;
+    *done = false;
+    if (hipMalloc((void **)&raw, aligned(words) + aligned(scales) + offsets) != hipSuccess) {
+        (void)hipGetLastError();
+        return LUTGEMM_OK;
+    }
+    char *d_alpha = raw + aligned(words), *d_offsets = d_alpha + aligned(scales);
+    int st = LUTGEMM_OK;
+    auto copy = [&](void *to, const void *from, size_t bytes) {
+        if (st != LUTGEMM_OK) return;
+        const hipError_t e = hipMemcpy(to, from, bytes, hipMemcpyHostToDevice);
+        if (e != hipSuccess) st = hip_fail(e, "hipMemcpy(weight arrays)");
+    };
+    copy(raw, bW, words);
+    copy(d_alpha, alpha, scales);
+    if (q_bias) copy(d_offsets, q_bias, offsets);
+    if (st == LUTGEMM_OK) {
+        lutgemm_kernels::PackArgs a{};
+        a.words = reinterpret_cast<const uint32_t *>(raw);
+        a.alpha = d_alpha;
+        a.offsets = q_bias ? d_offsets : nullptr;
+        a.halves = halves;
+        a.signs = w->d_signs;
+        a.scales = w->d_scales;
+        a.k = s.k;
+        a.n = s.n;
+        a.q = s.q;
+        a.gsub = s.gsub;
+        a.group_size = s.group_size;
+        a.ts = s.ts;
+        a.nb = s.nb;
+        hipError_t e = lutgemm_kernels::launch_pack(a, nullptr);
+        if (e == hipSuccess) {
+            e = hipStreamSynchronize(nullptr);   // the tiles are there when the call returns, for every stream
+            if (e != hipSuccess) st = hip_fail(e, "hipStreamSynchronize(pack)");
+            else *done = true;
+        } else if (e != hipErrorInvalidValue) {
+            st = hip_fail(e, "launch pack kernels");
+        }
+    }
+    (void)hipFree(raw);
+    return st;
+}
+
+// alpha and q_bias: fp16 bits (halves) or fp32
+int create_common(const uint32_t *bW, const void *alpha, const void *q_bias, bool halves, int k, int n,
                   int q, int num_groups, lutgemm_weight **out)
 {
     Shape s;
-    int st = shape_or_fail(k, n, q, num_groups, q_bias_h != nullptr, &s);
+    int st = shape_or_fail(k, n, q, num_groups, q_bias != nullptr, &s);
     if (st != LUTGEMM_OK) return st;
-    std::vector<uint8_t> signs;
-    std::vector<uint16_t> scales;
-    st = pack_to_host(s, bW, alpha_h, q_bias_h, &signs, &scales);
+    lutgemm_weight *w = nullptr;
+    st = new_handle(s, &w);
     if (st != LUTGEMM_OK) return st;
-    return create_from_tiles(s, signs.data(), scales.data(), hipMemcpyHostToDevice, out);
+    bool done = false;
+    st = pack_on_device(w, bW, alpha, q_bias, halves, &done);
+    if (st == LUTGEMM_OK && !done) {   // on the host
+        std::vector<uint8_t> signs;
+        std::vector<uint16_t> scales, ah, zh;
+        try {
+            if (!halves) {
+                ah.resize((size_t)num_groups * q * n);
+                if (q_bias) zh.resize((size_t)num_groups * n);
+            }
+        } catch (const std::bad_alloc &) {
+            st = fail(LUTGEMM_ERR_OUT_OF_MEMORY, "host allocation failed");
+        }
+        if (st == LUTGEMM_OK) {
+            if (!halves) {
+                lutgemm_packer::floats_to_halves(static_cast<const float *>(alpha), ah.data(), ah.size());
+                if (q_bias) lutgemm_packer::floats_to_halves(static_cast<const float *>(q_bias), zh.data(), zh.size());
+            }
+            const uint16_t *az = halves ? static_cast<const uint16_t *>(alpha) : ah.data();
+            const uint16_t *zz = !q_bias ? nullptr : halves ? static_cast<const uint16_t *>(q_bias) : zh.data();
+            st = pack_to_host(s, bW, az, zz, &signs, &scales);
+        }
+        if (st == LUTGEMM_OK) st = copy_tiles(w, signs.data(), scales.data(), hipMemcpyHostToDevice);
+    }
+    if (st != LUTGEMM_OK) {
+        lutgemm_weight_destroy(w);
+        return st;
+    }
+    *out = w;
+    return LUTGEMM_OK;
 }
 
 // Packed-weight file: 64-byte little-endian header, the sign tiles, the scale tiles.
@@ -1032,7 +1127,7 @@ int lutgemm_weight_create_f16(const uint32_t *bW, const uint16_t *alpha, const u
 {
     if (!bW || !alpha || !out) return fail(LUTGEMM_ERR_NULL_POINTER, "null argument to weight_create");
     *out = nullptr;
-    return create_common(bW, alpha, q_bias, k, n, q, num_groups, out);
+    return create_common(bW, alpha, q_bias, true, k, n, q, num_groups, out);
 }
 
 int lutgemm_weight_create(const uint32_t *bW, const float *alpha, const float *q_bias, int k, int n, int q,
@@ -1040,22 +1135,7 @@ int lutgemm_weight_create(const uint32_t *bW, const float *alpha, const float *q
 {
     if (!bW || !alpha || !out) return fail(LUTGEMM_ERR_NULL_POINTER, "null argument to weight_create");
     *out = nullptr;
-    Shape s;
-    if (!make_shape(k, n, q, num_groups, q_bias != nullptr, &s))
-        return fail(LUTGEMM_ERR_BAD_SHAPE,
-                    "bad shape k=%d n=%d q=%d num_groups=%d (need k%%32==0, 1<=q<=8, "
-                    "k%%num_groups==0, (k/num_groups)%%32==0)",
-                    k, n, q, num_groups);
-    std::vector<uint16_t> ah, zh;
-    try {
-        ah.resize((size_t)num_groups * q * n);
-        if (q_bias) zh.resize((size_t)num_groups * n);
-    } catch (const std::bad_alloc &) {
-        return fail(LUTGEMM_ERR_OUT_OF_MEMORY, "host allocation failed");
-    }
-    lutgemm_packer::floats_to_halves(alpha, ah.data(), ah.size());
-    if (q_bias) lutgemm_packer::floats_to_halves(q_bias, zh.data(), zh.size());
-    return create_common(bW, ah.data(), q_bias ? zh.data() : nullptr, k, n, q, num_groups, out);
+    return create_common(bW, alpha, q_bias, false, k, n, q, num_groups, out);
 }
 
 int lutgemm_weight_clone(const lutgemm_weight *w, lutgemm_weight **out)

@@ -41,6 +41,17 @@ struct MultiMatvecArgs {
     MatvecArgs entry[kMaxFused];
 };
 
+// Device copies of the arrays a weight is created from (packer.h's layout) and the tiles to make of them.
+struct PackArgs {
+    const uint32_t *words;  // [k/32][q][n]
+    const void *alpha;      // [groups][q][n], fp16 bits or fp32
+    const void *offsets;    // [groups][n], null for a weight without
+    int halves;             // the scales are fp16 bits
+    uint8_t *signs;
+    uint16_t *scales;
+    int k, n, q, gsub, group_size, ts, nb;
+};
+
 struct DequantArgs {
     const uint8_t *signs;
     const uint16_t *scales;
@@ -130,6 +141,9 @@ hipError_t static_split_k_words(int device, unsigned long long **words);
 
 // fp16 [k][m] -> [m][k]
 hipError_t launch_gather_columns(const void *cols, void *rows, int k, int m, hipStream_t stream);
+
+// hipErrorInvalidValue for a weight beyond the kernels' grids (2^31 threads)
+hipError_t launch_pack(const PackArgs &a, hipStream_t stream);
 
 hipError_t launch_dequantize(const DequantArgs &a, hipStream_t stream);
 
