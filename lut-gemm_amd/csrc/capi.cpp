@@ -811,7 +811,8 @@ int read_file(const char *path, Shape *s, std::vector<uint8_t> *signs, std::vect
 
 // `static_ws`: take the split-k words from the static device array instead of the handle's
 // per-stream sets (rows form only; nothing on this route allocates).
-int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *stream, bool cols, bool static_ws)
+int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *stream, bool cols, bool static_ws,
+               const void *bias = nullptr)
 {
     if (!w || !x || !y) return fail(LUTGEMM_ERR_NULL_POINTER, "null argument to matvec");
     if (m < 1 || m > LUTGEMM_MAX_BATCH)
@@ -826,6 +827,7 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
     a.n = s.n;
     a.ts = s.ts;
     a.nb = s.nb;
+    a.bias = bias;
     const uint16_t *xh = static_cast<const uint16_t *>(x);
     uint16_t *yh = static_cast<uint16_t *>(y);
     if (((uintptr_t)x & 15u) != 0)  // rows of x are k fp16 apart and k is a multiple of 32
@@ -886,8 +888,9 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
     // More rows than a pass of the batch kernel takes: one launch over all of them, except for the allocation-free entry
     // point (its words hold no partial sums) and for a k beyond the kernel's 32-bit offsets.
     if (m > kRowsPerPass && !static_ws && s.k <= kMaxRowsK) {
+        lutgemm_kernels::RowsGrid g{};
         RowsPlan plan = choose_rows_plan(s, w->compute_units, m, true);
-        if (plan.k_splits > 1 && !(a.partials = partials_of(mw, slot, stream)))
+        if (plan.k_splits > 1 && !(g.partials = partials_of(mw, slot, stream)))
             plan = choose_rows_plan(s, w->compute_units, m, false);
         a.ntiles = plan.ntiles;
         a.k_splits = plan.k_splits;
@@ -897,7 +900,6 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
         a.y = yh;
         a.y_stride = cols ? m : 1;   // y [n][m] or [m][n]
         a.y_row_stride = cols ? 1 : s.n;
-        lutgemm_kernels::RowsGrid g{};
         g.row_chunks = plan.row_chunks;
         g.q = s.q;
         g.gsub = s.gsub;
@@ -1245,6 +1247,12 @@ int lutgemm_weight_info(const lutgemm_weight *w, lutgemm_weight_info_t *info)
 int lutgemm_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *stream)
 {
     return run_matvec(w, x, y, m, stream, false, false);
+}
+
+int lutgemm_matvec_bias(const lutgemm_weight *w, const void *x, void *y, const void *bias, int m, void *stream)
+{
+    if (((uintptr_t)bias & 1u) != 0) return fail(LUTGEMM_ERR_BAD_SHAPE, "bias must be 2-byte aligned");
+    return run_matvec(w, x, y, m, stream, false, false, bias);
 }
 
 int lutgemm_matvec_static(const lutgemm_weight *w, const void *x, void *y, int m, void *stream)

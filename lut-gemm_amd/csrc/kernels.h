@@ -15,7 +15,7 @@ struct MatvecArgs {
     void *y;                // fp16 outputs, element j at y[j * y_stride]
     unsigned long long *accum;  // [rows][nb*32] split-k accumulators (count | flags | fixed-point sum), zero
                                 // between launches; used when k_splits > 1 (launch_rows: only counts)
-    float *partials;        // launch_rows with k_splits > 1: partial sums (no initial value)
+    const void *bias;       // fp16 [n] added to the fp32 sum of an output before its one rounding; null for none
     int k, n;
     int ts, nb;             // k-blocks, output batches
     int ntiles;             // column tiles = ceil(nb / waves)
@@ -108,6 +108,7 @@ constexpr int kRowsTilesMin = 2, kRowsTilesMax = 4;
 struct RowsGrid {
     int row_chunks;
     int q, gsub;
+    float *partials;   // k_splits > 1: partial sums (no initial value)
     int wide_y;   // four neighbouring outputs of a row are 8-byte aligned in y
 };
 // words of 32 k (for each of the four lane groups) that are staged in LDS at a time

@@ -525,8 +525,11 @@ __device__ __forceinline__ void matvec_workgroup(const MatvecArgs &a, int block)
         if (more) __syncthreads();
     }
 
+    const int out = nb * kBatch + (lane >> 1);
+    const bool valid = active && (lane & 1) == 0 && out < a.n;
+    const uint32_t bias = output_bias(a, out, valid);   // on its way during the reduction
     const float total = reduce_across_lanes(acc, lane);
-    finish_output(total, active, nb * kBatch + (lane >> 1), lane, reinterpret_cast<__half *>(a.y), a.accum, a);
+    finish_output(total, bias, valid, out, reinterpret_cast<__half *>(a.y), a.accum, a);
 }
 
 template <int Q, bool OFF, int GSUB>
@@ -665,13 +668,14 @@ __device__ __forceinline__ void matvec2_workgroup(const MatvecArgs &a, int block
 
     const int out = nb * kBatch + (lane >> 1);
     __half *y = reinterpret_cast<__half *>(a.y);
+    const bool valid0 = active && (lane & 1) == 0 && out < a.n, valid1 = valid0 && a.rows > 1;
+    const uint32_t bias = output_bias(a, out, valid0);
     const float total0 = reduce_across_lanes(acc0, lane);
     const float total1 = reduce_across_lanes(acc1, lane);
-    const bool valid0 = active && (lane & 1) == 0 && out < a.n, valid1 = valid0 && a.rows > 1;
     __half *y0 = y + (size_t)out * a.y_stride, *y1 = y0 + a.y_row_stride;
     if (a.k_splits == 1) {
-        if (valid0) *y0 = __float2half_rn(total0);
-        if (valid1) *y1 = __float2half_rn(total1);
+        if (valid0) *y0 = __float2half_rn(add_bias(total0, bias));
+        if (valid1) *y1 = __float2half_rn(add_bias(total1, bias));
         return;
     }
     // both atomics go out before the first answer is looked at
@@ -681,8 +685,8 @@ __device__ __forceinline__ void matvec2_workgroup(const MatvecArgs &a, int block
     // both answers are looked at before the first output is written (pinned by the empty asm statement)
     unsigned last = (unsigned)arrived_last(r0, valid0, a.k_splits) | ((unsigned)arrived_last(r1, valid1, a.k_splits) << 1);
     asm volatile("" : "+v"(last) : : "memory");
-    if (last & 1u) finish_last(r0, w0, y0, a.k_splits);
-    if (last & 2u) finish_last(r1, w1, y1, a.k_splits);
+    if (last & 1u) finish_last(r0, w0, y0, a.k_splits, bias);
+    if (last & 2u) finish_last(r1, w1, y1, a.k_splits, bias);
 }
 
 template <int Q, bool OFF, int GSUB>

@@ -286,13 +286,20 @@ __global__ __launch_bounds__(kRowsWaves * 64) void lut_rows_kernel(MatvecArgs a,
     if (a.k_splits > 1) {
         // sums over the workgroups of the tile in the order of their k ranges, by the wavefront that comes last
         const size_t unit = ((size_t)rc * a.nb + nb) * a.k_splits;
-        if (!sum_partials<2 * RT>(a.partials + unit * (2 * RT * 256), reinterpret_cast<unsigned *>(a.accum + ((size_t)rc * a.nb + nb)), ks,
+        if (!sum_partials<2 * RT>(g.partials + unit * (2 * RT * 256), reinterpret_cast<unsigned *>(a.accum + ((size_t)rc * a.nb + nb)), ks,
                                   a.k_splits, lane, [&](auto I) -> float4v & { return acc[I % 2][I / 2]; }))
             return;
     }
     __half *y = reinterpret_cast<__half *>(a.y);
+    float bias[2][4];
+    static_for<8>([&](auto I) {
+        const int out = nb * kBatch + 16 * (I / 4) + 4 * kappa + I % 4;
+        bias[I / 4][I % 4] = (float)__builtin_bit_cast(_Float16, (uint16_t)output_bias(a, out, out < a.n));
+    });
     static_for<2 * RT>([&](auto I) {
         constexpr int h = I % 2, t = I / 2;
+#pragma unroll
+        for (int v = 0; v < 4; v++) acc[h][t][v] += bias[h][v];
         const int row = row0 + 16 * t + j, out = nb * kBatch + 16 * h + 4 * kappa;
         if (row >= a.rows) return;
         __half *at = y + (size_t)row * a.y_row_stride + (size_t)out * a.y_stride;

@@ -26,7 +26,7 @@ MAX_BATCH = 4096
 # every symbol include/lutgemm_c.h declares
 EXPORTED = [
     "lutgemm_weight_create", "lutgemm_weight_create_f16", "lutgemm_weight_destroy", "lutgemm_weight_info",
-    "lutgemm_matvec", "lutgemm_matvec_cols", "lutgemm_matvec_many", "lutgemm_dequantize", "lutgemm_weight_unpack",
+    "lutgemm_matvec", "lutgemm_matvec_bias", "lutgemm_matvec_cols", "lutgemm_matvec_many", "lutgemm_dequantize", "lutgemm_weight_unpack",
     "lutgemm_weight_plan", "lutgemm_weight_plan_for", "lutgemm_weight_set_plan", "lutgemm_weight_set_batch_plan", "lutgemm_weight_autotune", "lutgemm_weight_device_ptrs", "lutgemm_packed_sizes",
     "lutgemm_pack_host", "lutgemm_unpack_host", "lutgemm_float_to_half", "lutgemm_last_error",
     "lutgemm_status_string", "lutgemm_version", "lutgemm_pack_file", "lutgemm_unpack_file", "lutgemm_weight_save",
@@ -79,6 +79,7 @@ def load():
     L.lutgemm_weight_destroy.argtypes = [vp]
     L.lutgemm_weight_info.argtypes = [vp, ctypes.POINTER(WeightInfo)]
     L.lutgemm_matvec.argtypes = [vp, vp, vp, i, vp]
+    L.lutgemm_matvec_bias.argtypes = [vp, vp, vp, vp, i, vp]
     L.lutgemm_matvec_cols.argtypes = [vp, vp, vp, i, vp]
     L.lutgemm_matvec_static.argtypes = [vp, vp, vp, i, vp]
     L.lutgemm_matvec_many.argtypes = [vp, vp, vp, vp, i, vp]
@@ -281,6 +282,10 @@ class BCQWeight:
 
     def matvec(self, x_ptr, y_ptr, m=1, stream=0):
         _check(load().lutgemm_matvec(self._h, x_ptr, y_ptr, m, stream or None))
+
+    def matvec_bias(self, x_ptr, y_ptr, bias_ptr, m=1, stream=0):
+        """matvec with an fp16 bias [n] (0 for none) added to the fp32 sums before they are rounded."""
+        _check(load().lutgemm_matvec_bias(self._h, x_ptr, y_ptr, bias_ptr or None, m, stream or None))
 
     def matvec_static(self, x_ptr, y_ptr, m=1, stream=0):
         """matvec with the split-k words in the library's static device array: allocates nothing."""
