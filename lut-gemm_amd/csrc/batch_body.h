@@ -524,15 +524,12 @@ __device__ __forceinline__ void batch_workgroup(const MatvecArgs &a, unsigned bl
             word[h][v] = a.accum + (size_t)row * a.accum_row_stride + out;
             yout[h][v] = y + (size_t)row * a.y_row_stride + (size_t)out * a.y_stride;
         }
-    uint32_t bias[2];
-#pragma unroll
-    for (int h = 0; h < 2; h++) bias[h] = output_bias(a, nb * kBatch + 16 * h + j, active && nb * kBatch + 16 * h + j < a.n);
     if (a.k_splits == 1) {
 #pragma unroll
         for (int h = 0; h < 2; h++)
 #pragma unroll
             for (int v = 0; v < 4; v++)
-                if (valid[h][v]) *yout[h][v] = __float2half_rn(add_bias(acc[h][v], bias[h]));
+                if (valid[h][v]) *yout[h][v] = __float2half_rn(acc[h][v]);
         return;
     }
     Arrival arrival[2][4];
@@ -553,7 +550,7 @@ __device__ __forceinline__ void batch_workgroup(const MatvecArgs &a, unsigned bl
     for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int v = 0; v < 4; v++)
-            if (last & (1u << (4 * h + v))) finish_last(arrival[h][v], word[h][v], yout[h][v], a.k_splits, bias[h]);
+            if (last & (1u << (4 * h + v))) finish_last(arrival[h][v], word[h][v], yout[h][v], a.k_splits);
 }
 
 

@@ -827,7 +827,7 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
     a.n = s.n;
     a.ts = s.ts;
     a.nb = s.nb;
-    a.bias = bias;
+    if (m == 1 || (m > kRowsPerPass && s.k <= kMaxRowsK)) a.bias = bias;   // the others get it behind their launches
     const uint16_t *xh = static_cast<const uint16_t *>(x);
     uint16_t *yh = static_cast<uint16_t *>(y);
     if (((uintptr_t)x & 15u) != 0)  // rows of x are k fp16 apart and k is a multiple of 32
@@ -885,6 +885,12 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
     }
     a.x_row_stride = s.k;
     a.accum_row_stride = (long long)s.nb * kBatch;
+    // The kernels of 2 to 16 rows take no bias (add_bias in tile_device.h): a small kernel follows them.
+    auto add_bias_behind = [&]() -> int {
+        if (!bias || a.bias) return LUTGEMM_OK;
+        const hipError_t e = lutgemm_kernels::launch_add_bias(y, bias, m, s.n, st);
+        return e == hipSuccess ? LUTGEMM_OK : hip_fail(e, "launch add_bias_kernel");
+    };
     // More rows than a pass of the batch kernel takes: one launch over all of them, except for the allocation-free entry
     // point (its words hold no partial sums) and for a k beyond the kernel's 32-bit offsets.
     if (m > kRowsPerPass && !static_ws && s.k <= kMaxRowsK) {
@@ -936,7 +942,7 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
             }
             lease.launched = true;
         }
-        return LUTGEMM_OK;
+        return add_bias_behind();
     }
     // two activation rows per pass over the weight, a last single row if m is odd
     for (int r = 0; r < m; r += 2) {
@@ -963,7 +969,7 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
         }
         lease.launched = true;
     }
-    return LUTGEMM_OK;
+    return add_bias_behind();
 }
 
 // ---- runs of independent entries that share one launch (lutgemm_matvec_many) ----------------

@@ -15,7 +15,8 @@ struct MatvecArgs {
     void *y;                // fp16 outputs, element j at y[j * y_stride]
     unsigned long long *accum;  // [rows][nb*32] split-k accumulators (count | flags | fixed-point sum), zero
                                 // between launches; used when k_splits > 1 (launch_rows: only counts)
-    const void *bias;       // fp16 [n] added to the fp32 sum of an output before its one rounding; null for none
+    const void *bias;       // one row (launch_matvec) and launch_rows: fp16 [n] added to the fp32 sum of an output before
+                            // its one rounding, null for none
     int k, n;
     int ts, nb;             // k-blocks, output batches
     int ntiles;             // column tiles = ceil(nb / waves)
@@ -139,6 +140,9 @@ hipError_t launch_fill_zero(unsigned long long *words, size_t count, hipStream_t
 constexpr size_t kStaticSplitKWords = (size_t)1 << 20;
 constexpr int kMaxDevices = 64;
 hipError_t static_split_k_words(int device, unsigned long long **words);
+
+// y [m][n] += bias [n], fp16
+hipError_t launch_add_bias(void *y, const void *bias, int m, int n, hipStream_t stream);
 
 // fp16 [k][m] -> [m][k]
 hipError_t launch_gather_columns(const void *cols, void *rows, int k, int m, hipStream_t stream);

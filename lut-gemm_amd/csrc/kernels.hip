@@ -448,7 +448,7 @@ __device__ __forceinline__ float reduce_across_lanes(float (&acc)[kBatch], int l
 }
 
 // Workgroup `block` of one matvec (the body of lut_matvec_kernel and of lut_matvec_multi_kernel).
-template <int Q, bool OFF, int GSUB>
+template <int Q, bool OFF, int GSUB, bool BIAS>
 __device__ __forceinline__ void matvec_workgroup(const MatvecArgs &a, int block)
 {
     constexpr int QO = Q + (OFF ? 1 : 0);
@@ -525,17 +525,14 @@ __device__ __forceinline__ void matvec_workgroup(const MatvecArgs &a, int block)
         if (more) __syncthreads();
     }
 
-    const int out = nb * kBatch + (lane >> 1);
-    const bool valid = active && (lane & 1) == 0 && out < a.n;
-    const uint32_t bias = output_bias(a, out, valid);   // on its way during the reduction
     const float total = reduce_across_lanes(acc, lane);
-    finish_output(total, bias, valid, out, reinterpret_cast<__half *>(a.y), a.accum, a);
+    finish_output<BIAS>(total, active, nb * kBatch + (lane >> 1), lane, reinterpret_cast<__half *>(a.y), a.accum, a);
 }
 
-template <int Q, bool OFF, int GSUB>
+template <int Q, bool OFF, int GSUB, bool BIAS>
 __global__ __launch_bounds__(768) void lut_matvec_kernel(MatvecArgs a)
 {
-    matvec_workgroup<Q, OFF, GSUB>(a, blockIdx.x);
+    matvec_workgroup<Q, OFF, GSUB, BIAS>(a, blockIdx.x);
 }
 
 // Several independent one-row matvecs in one launch: the workgroups of entry i follow those of
@@ -547,7 +544,7 @@ __global__ __launch_bounds__(768) void lut_matvec_multi_kernel(MultiMatvecArgs m
 {
     int i = 0;
     while (i + 1 < m.count && (int)blockIdx.x >= m.first_block[i + 1]) i++;   // scalar: at most 31 steps
-    matvec_workgroup<Q, OFF, GSUB>(m.entry[i], (int)blockIdx.x - m.first_block[i]);
+    matvec_workgroup<Q, OFF, GSUB, false>(m.entry[i], (int)blockIdx.x - m.first_block[i]);
 }
 
 // process_tile for two activation rows (tables of lookup8x2).
@@ -668,14 +665,13 @@ __device__ __forceinline__ void matvec2_workgroup(const MatvecArgs &a, int block
 
     const int out = nb * kBatch + (lane >> 1);
     __half *y = reinterpret_cast<__half *>(a.y);
-    const bool valid0 = active && (lane & 1) == 0 && out < a.n, valid1 = valid0 && a.rows > 1;
-    const uint32_t bias = output_bias(a, out, valid0);
     const float total0 = reduce_across_lanes(acc0, lane);
     const float total1 = reduce_across_lanes(acc1, lane);
+    const bool valid0 = active && (lane & 1) == 0 && out < a.n, valid1 = valid0 && a.rows > 1;
     __half *y0 = y + (size_t)out * a.y_stride, *y1 = y0 + a.y_row_stride;
     if (a.k_splits == 1) {
-        if (valid0) *y0 = __float2half_rn(add_bias(total0, bias));
-        if (valid1) *y1 = __float2half_rn(add_bias(total1, bias));
+        if (valid0) *y0 = __float2half_rn(total0);
+        if (valid1) *y1 = __float2half_rn(total1);
         return;
     }
     // both atomics go out before the first answer is looked at
@@ -685,8 +681,8 @@ __device__ __forceinline__ void matvec2_workgroup(const MatvecArgs &a, int block
     // both answers are looked at before the first output is written (pinned by the empty asm statement)
     unsigned last = (unsigned)arrived_last(r0, valid0, a.k_splits) | ((unsigned)arrived_last(r1, valid1, a.k_splits) << 1);
     asm volatile("" : "+v"(last) : : "memory");
-    if (last & 1u) finish_last(r0, w0, y0, a.k_splits, bias);
-    if (last & 2u) finish_last(r1, w1, y1, a.k_splits, bias);
+    if (last & 1u) finish_last(r0, w0, y0, a.k_splits);
+    if (last & 2u) finish_last(r1, w1, y1, a.k_splits);
 }
 
 template <int Q, bool OFF, int GSUB>
@@ -757,6 +753,14 @@ __global__ __launch_bounds__(256) void gather_columns_kernel(const uint16_t *col
     rows[idx] = cols[(size_t)i * m + r];
 }
 
+// y [m][n] += bias [n]
+__global__ __launch_bounds__(256) void add_bias_kernel(__half *y, const __half *bias, int n, size_t count)
+{
+    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= count) return;
+    y[idx] = __float2half_rn(__half2float(y[idx]) + __half2float(bias[idx % (size_t)n]));
+}
+
 __global__ __launch_bounds__(256) void fill_zero_kernel(unsigned long long *words, size_t count)
 {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x)
@@ -780,6 +784,17 @@ hipError_t allow_two_table_sets(Kernel kernel, std::atomic<unsigned long long> &
     return hipSuccess;
 }
 
+template <int Q, bool OFF, int GSUB, bool BIAS>
+hipError_t launch_one_row(const MatvecArgs &a, int workgroups, int threads, hipStream_t stream)
+{
+    static std::atomic<unsigned long long> allowed{0};
+    const hipError_t e = allow_two_table_sets(&lut_matvec_kernel<Q, OFF, GSUB, BIAS>, allowed);
+    if (e != hipSuccess) return e;
+    const size_t lds = (size_t)(a.blocks_per_split == 1 ? 1 : 2) * kTableFloats * sizeof(float);
+    hipLaunchKernelGGL((lut_matvec_kernel<Q, OFF, GSUB, BIAS>), dim3(workgroups), dim3(threads), lds, stream, a);
+    return hipGetLastError();
+}
+
 template <int Q, bool OFF, int GSUB>
 hipError_t launch_one(const MatvecArgs &a, int workgroups, int threads, hipStream_t stream)
 {
@@ -788,13 +803,8 @@ hipError_t launch_one(const MatvecArgs &a, int workgroups, int threads, hipStrea
     else if (a.rows > 1)
         hipLaunchKernelGGL((lut_matvec2_kernel<Q, OFF, GSUB>), dim3(workgroups), dim3(threads), 0, stream, a);
     else
-    {
-        static std::atomic<unsigned long long> allowed{0};
-        const hipError_t e = allow_two_table_sets(&lut_matvec_kernel<Q, OFF, GSUB>, allowed);
-        if (e != hipSuccess) return e;
-        const size_t lds = (size_t)(a.blocks_per_split == 1 ? 1 : 2) * kTableFloats * sizeof(float);
-        hipLaunchKernelGGL((lut_matvec_kernel<Q, OFF, GSUB>), dim3(workgroups), dim3(threads), lds, stream, a);
-    }
+        return a.bias ? launch_one_row<Q, OFF, GSUB, true>(a, workgroups, threads, stream)
+                      : launch_one_row<Q, OFF, GSUB, false>(a, workgroups, threads, stream);
     return hipGetLastError();
 }
 
@@ -909,6 +919,14 @@ hipError_t launch_fill_zero(unsigned long long *words, size_t count, hipStream_t
     const size_t blocks = (count + 255) / 256;
     hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)(blocks < 1024 ? blocks : 1024)), dim3(256), 0, stream, words,
                        count);
+    return hipGetLastError();
+}
+
+hipError_t launch_add_bias(void *y, const void *bias, int m, int n, hipStream_t stream)
+{
+    const size_t count = (size_t)m * n;
+    hipLaunchKernelGGL(add_bias_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, static_cast<__half *>(y),
+                       static_cast<const __half *>(bias), n, count);
     return hipGetLastError();
 }
 

@@ -68,19 +68,13 @@ __device__ __forceinline__ void load_tile(TileRegs<Q, QO, GSUB> &r, const NextTi
     for (int u = 0; u < 2 * Q; u++) r.sign[u] = __builtin_nontemporal_load(n.sign + u * n.sign_stride);
 }
 
-// The fp16 bits added to the sum of output `out`: its bias, or -0, which changes no value.
-__device__ __forceinline__ uint32_t output_bias(const MatvecArgs &a, int out, bool valid)
+// value + the bias of output `out` (in the kernels that take one; the bias is a template argument because even a test for
+// its absence at the end of a workgroup cost the batch kernel 2 to 7 %)
+template <bool BIAS>
+__device__ __forceinline__ float add_bias(const MatvecArgs &a, float value, int out)
 {
-    return a.bias && valid ? static_cast<const uint16_t *>(a.bias)[out] : 0x8000u;
-}
-
-// value + bias in one mixed-precision multiply-add (the product with 1 is exact).  Not for a value that comes straight out of a
-// matrix instruction: the compiler inserts the wait states for those only in front of instructions of its own.
-__device__ __forceinline__ float add_bias(float value, uint32_t bias)
-{
-    float sum;
-    asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(sum) : "v"(bias), "v"(value));
-    return sum;
+    if constexpr (BIAS) return value + __half2float(static_cast<const __half *>(a.bias)[out]);
+    else return value;
 }
 
 // Lane pair (2j, 2j+1) of a wavefront holds the k-range total of output `out`; the even lane
@@ -132,7 +126,9 @@ __device__ __forceinline__ bool arrived_last(const Arrival &r, bool valid, int k
     return valid && (r.old >> 56) == (unsigned long long)(k_splits - 1);
 }
 
-__device__ __forceinline__ void finish_last(const Arrival &r, unsigned long long *word, __half *yout, int k_splits, uint32_t bias)
+// `finish` makes the output's value of the sum
+template <typename F>
+__device__ __forceinline__ void finish_last(const Arrival &r, unsigned long long *word, __half *yout, int k_splits, F &&finish)
 {
     const unsigned long long all = r.old + r.addend;
     const long long value = (long long)(all & (kPosInfFlag - 1)) - (long long)k_splits * (1ll << 46);
@@ -140,26 +136,27 @@ __device__ __forceinline__ void finish_last(const Arrival &r, unsigned long long
     const unsigned long long flags = all & (kPosInfFlag | kNegInfFlag);
     if (flags)
         result = flags == kPosInfFlag ? __builtin_inff() : flags == kNegInfFlag ? -__builtin_inff() : __builtin_nanf("");
-    *yout = __float2half_rn(add_bias(result, bias));
+    *yout = __float2half_rn(finish(result));
     __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ void complete_output(const Arrival &r, bool valid, unsigned long long *word, __half *yout,
-                                                int k_splits, uint32_t bias)
+__device__ __forceinline__ void finish_last(const Arrival &r, unsigned long long *word, __half *yout, int k_splits)
 {
-    if (arrived_last(r, valid, k_splits)) finish_last(r, word, yout, k_splits, bias);
+    finish_last(r, word, yout, k_splits, [](float sum) { return sum; });
 }
 
-// (`valid`: this lane delivers `out`)
-__device__ __forceinline__ void finish_output(float total, uint32_t bias, bool valid, int out, __half *y,
+template <bool BIAS>
+__device__ __forceinline__ void finish_output(float total, bool active, int out, int lane, __half *y,
                                               unsigned long long *accum, const MatvecArgs &a)
 {
+    const bool valid = active && (lane & 1) == 0 && out < a.n;
     if (a.k_splits == 1) {
-        if (valid) y[(size_t)out * a.y_stride] = __float2half_rn(add_bias(total, bias));
+        if (valid) y[(size_t)out * a.y_stride] = __float2half_rn(add_bias<BIAS>(a, total, out));
         return;
     }
     const Arrival r = arrive_output(total, valid, accum + out);
-    complete_output(r, valid, accum + out, y + (size_t)out * a.y_stride, a.k_splits, bias);
+    if (arrived_last(r, valid, a.k_splits))
+        finish_last(r, accum + out, y + (size_t)out * a.y_stride, a.k_splits, [&](float sum) { return add_bias<BIAS>(a, sum, out); });
 }
 
 // Split-k sums of a wavefront's N registers of four values through memory, for kernels that finish many values per

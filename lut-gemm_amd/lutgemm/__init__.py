@@ -284,7 +284,7 @@ class BCQWeight:
         _check(load().lutgemm_matvec(self._h, x_ptr, y_ptr, m, stream or None))
 
     def matvec_bias(self, x_ptr, y_ptr, bias_ptr, m=1, stream=0):
-        """matvec with an fp16 bias [n] (0 for none) added to the fp32 sums before they are rounded."""
+        """matvec with an fp16 bias [n] (0 for none) added."""
         _check(load().lutgemm_matvec_bias(self._h, x_ptr, y_ptr, bias_ptr or None, m, stream or None))
 
     def matvec_static(self, x_ptr, y_ptr, m=1, stream=0):

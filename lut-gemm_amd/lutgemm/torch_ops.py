@@ -214,8 +214,7 @@ class LutLinear(torch.nn.Module):
         return Wt
 
     def forward(self, x):
-        """The bias joins the fp32 sums before their rounding where it is what the constructor made of it (float16 [n] on
-        x's device); one that the program has put in its place since (another dtype, a parameter) is added to the result."""
+        """The bias goes with the call where it is what the constructor made of it (float16 [n] on x's device); one that the program has put in its place since (another dtype, a parameter) is added to the result."""
         rows = x.numel() // x.shape[-1]
         if x.dtype != torch.float16:
             x = x.to(torch.float16)
