@@ -827,7 +827,6 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
     a.n = s.n;
     a.ts = s.ts;
     a.nb = s.nb;
-    if (m == 1 || (m > kRowsPerPass && s.k <= kMaxRowsK)) a.bias = bias;   // the others get it behind their launches
     const uint16_t *xh = static_cast<const uint16_t *>(x);
     uint16_t *yh = static_cast<uint16_t *>(y);
     if (((uintptr_t)x & 15u) != 0)  // rows of x are k fp16 apart and k is a multiple of 32
@@ -885,9 +884,9 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
     }
     a.x_row_stride = s.k;
     a.accum_row_stride = (long long)s.nb * kBatch;
-    // The kernels of 2 to 16 rows take no bias (add_bias in tile_device.h): a small kernel follows them.
+    // The kernels of 2 to 16 rows take no bias (add_bias in tile_device.h): a small kernel follows their launches.
     auto add_bias_behind = [&]() -> int {
-        if (!bias || a.bias) return LUTGEMM_OK;
+        if (!bias || m == 1) return LUTGEMM_OK;
         const hipError_t e = lutgemm_kernels::launch_add_bias(y, bias, m, s.n, st);
         return e == hipSuccess ? LUTGEMM_OK : hip_fail(e, "launch add_bias_kernel");
     };
@@ -907,6 +906,7 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
         a.y_stride = cols ? m : 1;   // y [n][m] or [m][n]
         a.y_row_stride = cols ? 1 : s.n;
         g.row_chunks = plan.row_chunks;
+        g.bias = bias;
         g.q = s.q;
         g.gsub = s.gsub;
         g.wide_y = !cols && s.n % 4 == 0 && ((uintptr_t)y & 7u) == 0;
@@ -962,7 +962,7 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
             a.y_row_stride = s.n;
         }
         hipError_t e = lutgemm_kernels::launch_matvec(s.q, s.has_offset, s.gsub, a, plan.ntiles * plan.k_splits,
-                                                      plan.waves, st);
+                                                      plan.waves, st, m == 1 ? bias : nullptr);
         if (e != hipSuccess) {
             if (static_ws && r > 0) g_static_dirty[w->device] = true;
             return hip_fail(e, "launch lut_matvec_kernel");

@@ -15,8 +15,6 @@ struct MatvecArgs {
     void *y;                // fp16 outputs, element j at y[j * y_stride]
     unsigned long long *accum;  // [rows][nb*32] split-k accumulators (count | flags | fixed-point sum), zero
                                 // between launches; used when k_splits > 1 (launch_rows: only counts)
-    const void *bias;       // one row (launch_matvec) and launch_rows: fp16 [n] added to the fp32 sum of an output before
-                            // its one rounding, null for none
     int k, n;
     int ts, nb;             // k-blocks, output batches
     int ntiles;             // column tiles = ceil(nb / waves)
@@ -61,9 +59,10 @@ struct DequantArgs {
     int transposed;
 };
 
-// workgroups = ntiles * k_splits, `waves` wavefronts of 64 lanes per workgroup.
+// workgroups = ntiles * k_splits, `waves` wavefronts of 64 lanes per workgroup.  `bias` (one row only): fp16 [n] added to
+// the fp32 sum of an output before its one rounding.
 hipError_t launch_matvec(int q, int has_offset, int gsub, const MatvecArgs &a, int workgroups,
-                         int waves, hipStream_t stream);
+                         int waves, hipStream_t stream, const void *bias = nullptr);
 
 // entries that all have one row or all have two, sharing q, has_offset, gsub and the wavefronts per workgroup
 hipError_t launch_matvec_multi(int q, int has_offset, int gsub, const MultiMatvecArgs &m, int workgroups, int waves,
@@ -109,6 +108,7 @@ constexpr int kRowsTilesMin = 2, kRowsTilesMax = 4;
 struct RowsGrid {
     int row_chunks;
     int q, gsub;
+    const void *bias;  // fp16 [n] added to the fp32 sum of an output before its one rounding; null for none
     float *partials;   // k_splits > 1: partial sums (no initial value)
     int wide_y;   // four neighbouring outputs of a row are 8-byte aligned in y
 };

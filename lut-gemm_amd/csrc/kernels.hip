@@ -449,7 +449,7 @@ __device__ __forceinline__ float reduce_across_lanes(float (&acc)[kBatch], int l
 
 // Workgroup `block` of one matvec (the body of lut_matvec_kernel and of lut_matvec_multi_kernel).
 template <int Q, bool OFF, int GSUB, bool BIAS>
-__device__ __forceinline__ void matvec_workgroup(const MatvecArgs &a, int block)
+__device__ __forceinline__ void matvec_workgroup(const MatvecArgs &a, int block, const __half *bias)
 {
     constexpr int QO = Q + (OFF ? 1 : 0);
     // Two table sets: while the lookups of k-block t read one, the other is rebuilt for t+1.
@@ -526,13 +526,20 @@ __device__ __forceinline__ void matvec_workgroup(const MatvecArgs &a, int block)
     }
 
     const float total = reduce_across_lanes(acc, lane);
-    finish_output<BIAS>(total, active, nb * kBatch + (lane >> 1), lane, reinterpret_cast<__half *>(a.y), a.accum, a);
+    finish_output<BIAS>(total, active, nb * kBatch + (lane >> 1), lane, reinterpret_cast<__half *>(a.y), a.accum, a, bias);
 }
 
-template <int Q, bool OFF, int GSUB, bool BIAS>
+template <int Q, bool OFF, int GSUB>
 __global__ __launch_bounds__(768) void lut_matvec_kernel(MatvecArgs a)
 {
-    matvec_workgroup<Q, OFF, GSUB, BIAS>(a, blockIdx.x);
+    matvec_workgroup<Q, OFF, GSUB, false>(a, blockIdx.x, nullptr);
+}
+
+// the same with a bias
+template <int Q, bool OFF, int GSUB>
+__global__ __launch_bounds__(768) void lut_matvec_bias_kernel(MatvecArgs a, const __half *bias)
+{
+    matvec_workgroup<Q, OFF, GSUB, true>(a, blockIdx.x, bias);
 }
 
 // Several independent one-row matvecs in one launch: the workgroups of entry i follow those of
@@ -544,7 +551,7 @@ __global__ __launch_bounds__(768) void lut_matvec_multi_kernel(MultiMatvecArgs m
 {
     int i = 0;
     while (i + 1 < m.count && (int)blockIdx.x >= m.first_block[i + 1]) i++;   // scalar: at most 31 steps
-    matvec_workgroup<Q, OFF, GSUB, false>(m.entry[i], (int)blockIdx.x - m.first_block[i]);
+    matvec_workgroup<Q, OFF, GSUB, false>(m.entry[i], (int)blockIdx.x - m.first_block[i], nullptr);
 }
 
 // process_tile for two activation rows (tables of lookup8x2).
@@ -784,27 +791,26 @@ hipError_t allow_two_table_sets(Kernel kernel, std::atomic<unsigned long long> &
     return hipSuccess;
 }
 
-template <int Q, bool OFF, int GSUB, bool BIAS>
-hipError_t launch_one_row(const MatvecArgs &a, int workgroups, int threads, hipStream_t stream)
-{
-    static std::atomic<unsigned long long> allowed{0};
-    const hipError_t e = allow_two_table_sets(&lut_matvec_kernel<Q, OFF, GSUB, BIAS>, allowed);
-    if (e != hipSuccess) return e;
-    const size_t lds = (size_t)(a.blocks_per_split == 1 ? 1 : 2) * kTableFloats * sizeof(float);
-    hipLaunchKernelGGL((lut_matvec_kernel<Q, OFF, GSUB, BIAS>), dim3(workgroups), dim3(threads), lds, stream, a);
-    return hipGetLastError();
-}
-
 template <int Q, bool OFF, int GSUB>
-hipError_t launch_one(const MatvecArgs &a, int workgroups, int threads, hipStream_t stream)
+hipError_t launch_one(const MatvecArgs &a, int workgroups, int threads, hipStream_t stream, const void *bias)
 {
     if (a.rows == 0)  // read probe
         hipLaunchKernelGGL((read_probe_kernel<Q, OFF, GSUB>), dim3(workgroups), dim3(threads), 0, stream, a);
     else if (a.rows > 1)
         hipLaunchKernelGGL((lut_matvec2_kernel<Q, OFF, GSUB>), dim3(workgroups), dim3(threads), 0, stream, a);
     else
-        return a.bias ? launch_one_row<Q, OFF, GSUB, true>(a, workgroups, threads, stream)
-                      : launch_one_row<Q, OFF, GSUB, false>(a, workgroups, threads, stream);
+    {
+        const size_t lds = (size_t)(a.blocks_per_split == 1 ? 1 : 2) * kTableFloats * sizeof(float);
+        static std::atomic<unsigned long long> allowed{0}, allowed_bias{0};
+        const hipError_t e = bias ? allow_two_table_sets(&lut_matvec_bias_kernel<Q, OFF, GSUB>, allowed_bias)
+                                  : allow_two_table_sets(&lut_matvec_kernel<Q, OFF, GSUB>, allowed);
+        if (e != hipSuccess) return e;
+        if (bias)
+            hipLaunchKernelGGL((lut_matvec_bias_kernel<Q, OFF, GSUB>), dim3(workgroups), dim3(threads), lds, stream, a,
+                               static_cast<const __half *>(bias));
+        else
+            hipLaunchKernelGGL((lut_matvec_kernel<Q, OFF, GSUB>), dim3(workgroups), dim3(threads), lds, stream, a);
+    }
     return hipGetLastError();
 }
 
@@ -826,36 +832,36 @@ hipError_t launch_multi_one(const MultiMatvecArgs &m, int workgroups, int thread
 }
 
 template <int Q, bool OFF>
-hipError_t launch_gsub(int gsub, const MatvecArgs &a, int wg, int th, hipStream_t s)
+hipError_t launch_gsub(int gsub, const MatvecArgs &a, int wg, int th, hipStream_t s, const void *bias)
 {
     switch (gsub) {
-        case 1: return launch_one<Q, OFF, 1>(a, wg, th, s);
-        case 2: return launch_one<Q, OFF, 2>(a, wg, th, s);
-        default: return launch_one<Q, OFF, 4>(a, wg, th, s);
+        case 1: return launch_one<Q, OFF, 1>(a, wg, th, s, bias);
+        case 2: return launch_one<Q, OFF, 2>(a, wg, th, s, bias);
+        default: return launch_one<Q, OFF, 4>(a, wg, th, s, bias);
     }
 }
 
 template <int Q>
-hipError_t launch_off(int has_offset, int gsub, const MatvecArgs &a, int wg, int th, hipStream_t s)
+hipError_t launch_off(int has_offset, int gsub, const MatvecArgs &a, int wg, int th, hipStream_t s, const void *bias)
 {
-    return has_offset ? launch_gsub<Q, true>(gsub, a, wg, th, s) : launch_gsub<Q, false>(gsub, a, wg, th, s);
+    return has_offset ? launch_gsub<Q, true>(gsub, a, wg, th, s, bias) : launch_gsub<Q, false>(gsub, a, wg, th, s, bias);
 }
 
 }  // namespace
 
 hipError_t launch_matvec(int q, int has_offset, int gsub, const MatvecArgs &a, int workgroups,
-                         int waves, hipStream_t stream)
+                         int waves, hipStream_t stream, const void *bias)
 {
     const int th = waves * kLanes;
     switch (q) {
-        case 1: return launch_off<1>(has_offset, gsub, a, workgroups, th, stream);
-        case 2: return launch_off<2>(has_offset, gsub, a, workgroups, th, stream);
-        case 3: return launch_off<3>(has_offset, gsub, a, workgroups, th, stream);
-        case 4: return launch_off<4>(has_offset, gsub, a, workgroups, th, stream);
-        case 5: return launch_off<5>(has_offset, gsub, a, workgroups, th, stream);
-        case 6: return launch_off<6>(has_offset, gsub, a, workgroups, th, stream);
-        case 7: return launch_off<7>(has_offset, gsub, a, workgroups, th, stream);
-        case 8: return launch_off<8>(has_offset, gsub, a, workgroups, th, stream);
+        case 1: return launch_off<1>(has_offset, gsub, a, workgroups, th, stream, bias);
+        case 2: return launch_off<2>(has_offset, gsub, a, workgroups, th, stream, bias);
+        case 3: return launch_off<3>(has_offset, gsub, a, workgroups, th, stream, bias);
+        case 4: return launch_off<4>(has_offset, gsub, a, workgroups, th, stream, bias);
+        case 5: return launch_off<5>(has_offset, gsub, a, workgroups, th, stream, bias);
+        case 6: return launch_off<6>(has_offset, gsub, a, workgroups, th, stream, bias);
+        case 7: return launch_off<7>(has_offset, gsub, a, workgroups, th, stream, bias);
+        case 8: return launch_off<8>(has_offset, gsub, a, workgroups, th, stream, bias);
         default: return hipErrorInvalidValue;
     }
 }

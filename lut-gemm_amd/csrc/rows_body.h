@@ -294,7 +294,7 @@ __global__ __launch_bounds__(kRowsWaves * 64) void lut_rows_kernel(MatvecArgs a,
     float bias[2][4];
     static_for<8>([&](auto I) {
         const int out = nb * kBatch + 16 * (I / 4) + 4 * kappa + I % 4;
-        bias[I / 4][I % 4] = a.bias && out < a.n ? __half2float(static_cast<const __half *>(a.bias)[out]) : -0.f;   // -0 changes no value
+        bias[I / 4][I % 4] = g.bias && out < a.n ? __half2float(static_cast<const __half *>(g.bias)[out]) : -0.f;   // -0 changes no value
     });
     static_for<2 * RT>([&](auto I) {
         constexpr int h = I % 2, t = I / 2;

@@ -68,12 +68,12 @@ __device__ __forceinline__ void load_tile(TileRegs<Q, QO, GSUB> &r, const NextTi
     for (int u = 0; u < 2 * Q; u++) r.sign[u] = __builtin_nontemporal_load(n.sign + u * n.sign_stride);
 }
 
-// value + the bias of output `out` (in the kernels that take one; the bias is a template argument because even a test for
+// value + the bias of output `out` (in the kernels that take one; BIAS is a template argument because even a test for
 // its absence at the end of a workgroup cost the batch kernel 2 to 7 %)
 template <bool BIAS>
-__device__ __forceinline__ float add_bias(const MatvecArgs &a, float value, int out)
+__device__ __forceinline__ float add_bias(const __half *bias, float value, int out)
 {
-    if constexpr (BIAS) return value + __half2float(static_cast<const __half *>(a.bias)[out]);
+    if constexpr (BIAS) return value + __half2float(bias[out]);
     else return value;
 }
 
@@ -147,16 +147,16 @@ __device__ __forceinline__ void finish_last(const Arrival &r, unsigned long long
 
 template <bool BIAS>
 __device__ __forceinline__ void finish_output(float total, bool active, int out, int lane, __half *y,
-                                              unsigned long long *accum, const MatvecArgs &a)
+                                              unsigned long long *accum, const MatvecArgs &a, const __half *bias)
 {
     const bool valid = active && (lane & 1) == 0 && out < a.n;
     if (a.k_splits == 1) {
-        if (valid) y[(size_t)out * a.y_stride] = __float2half_rn(add_bias<BIAS>(a, total, out));
+        if (valid) y[(size_t)out * a.y_stride] = __float2half_rn(add_bias<BIAS>(bias, total, out));
         return;
     }
     const Arrival r = arrive_output(total, valid, accum + out);
     if (arrived_last(r, valid, a.k_splits))
-        finish_last(r, accum + out, y + (size_t)out * a.y_stride, a.k_splits, [&](float sum) { return add_bias<BIAS>(a, sum, out); });
+        finish_last(r, accum + out, y + (size_t)out * a.y_stride, a.k_splits, [&](float sum) { return add_bias<BIAS>(bias, sum, out); });
 }
 
 // Split-k sums of a wavefront's N registers of four values through memory, for kernels that finish many values per
