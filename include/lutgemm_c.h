@@ -120,8 +120,9 @@ int lutgemm_weight_info(const lutgemm_weight *w, lutgemm_weight_info_t *info);
 #define LUTGEMM_MAX_BATCH 4096
 int lutgemm_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *stream);
 
-/* lutgemm_matvec with a bias: y[r][j] = fp16(sum + bias[j]), rounded once for one row and for more than 16, else
- * fp16(fp16(sum) + bias[j]); bias fp16 [n] on the device, NULL for none.  No counterpart in the reference, whose callers add a bias with a kernel of their own. */
+/* lutgemm_matvec with a bias: y[r][j] = fp16(fp16(sum) + bias[j]) for every m, the bits that adding the bias to the
+ * result of lutgemm_matvec in fp16 gives; bias fp16 [n] on the device, NULL for none.  No counterpart in the reference,
+ * whose callers add a bias with a kernel of their own. */
 int lutgemm_matvec_bias(const lutgemm_weight *w, const void *x, void *y, const void *bias, int m, void *stream);
 
 /* lutgemm_matvec without any allocation, for callers that cannot allocate: code under HIP graph

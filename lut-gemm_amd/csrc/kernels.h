@@ -60,7 +60,7 @@ struct DequantArgs {
 };
 
 // workgroups = ntiles * k_splits, `waves` wavefronts of 64 lanes per workgroup.  `bias` (one row only): fp16 [n] added to
-// the fp32 sum of an output before its one rounding.
+// the rounded sum of an output, which is rounded again.
 hipError_t launch_matvec(int q, int has_offset, int gsub, const MatvecArgs &a, int workgroups,
                          int waves, hipStream_t stream, const void *bias = nullptr);
 
@@ -108,7 +108,7 @@ constexpr int kRowsTilesMin = 2, kRowsTilesMax = 4;
 struct RowsGrid {
     int row_chunks;
     int q, gsub;
-    const void *bias;  // fp16 [n] added to the fp32 sum of an output before its one rounding; null for none
+    const void *bias;  // fp16 [n] added to the rounded sum of an output, which is rounded again; null for none
     float *partials;   // k_splits > 1: partial sums (no initial value)
     int wide_y;   // four neighbouring outputs of a row are 8-byte aligned in y
 };

@@ -291,15 +291,16 @@ __global__ __launch_bounds__(kRowsWaves * 64) void lut_rows_kernel(MatvecArgs a,
             return;
     }
     __half *y = reinterpret_cast<__half *>(a.y);
-    float bias[2][4];
-    static_for<8>([&](auto I) {
-        const int out = nb * kBatch + 16 * (I / 4) + 4 * kappa + I % 4;
-        bias[I / 4][I % 4] = g.bias && out < a.n ? __half2float(static_cast<const __half *>(g.bias)[out]) : -0.f;   // -0 changes no value
-    });
+    if (g.bias)
+        static_for<8>([&](auto I) {
+            constexpr int h = I / 4, v = I % 4;
+            const int out = nb * kBatch + 16 * h + 4 * kappa + v;
+            const float bias = out < a.n ? __half2float(static_cast<const __half *>(g.bias)[out]) : 0.f;
+#pragma unroll
+            for (int t = 0; t < RT; t++) acc[h][t][v] = plus_bias(acc[h][t][v], bias);
+        });
     static_for<2 * RT>([&](auto I) {
         constexpr int h = I % 2, t = I / 2;
-#pragma unroll
-        for (int v = 0; v < 4; v++) acc[h][t][v] += bias[h][v];
         const int row = row0 + 16 * t + j, out = nb * kBatch + 16 * h + 4 * kappa;
         if (row >= a.rows) return;
         __half *at = y + (size_t)row * a.y_row_stride + (size_t)out * a.y_stride;

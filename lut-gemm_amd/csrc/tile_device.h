@@ -68,12 +68,15 @@ __device__ __forceinline__ void load_tile(TileRegs<Q, QO, GSUB> &r, const NextTi
     for (int u = 0; u < 2 * Q; u++) r.sign[u] = __builtin_nontemporal_load(n.sign + u * n.sign_stride);
 }
 
-// value + the bias of output `out` (in the kernels that take one; BIAS is a template argument because even a test for
+// The output that `value` rounds to plus a bias, still to be rounded: what adding the bias to a finished output gives
+__device__ __forceinline__ float plus_bias(float value, float bias) { return __half2float(__float2half_rn(value)) + bias; }
+
+// plus_bias of output `out` (in the kernels that take a bias; BIAS is a template argument because even a test for
 // its absence at the end of a workgroup cost the batch kernel 2 to 7 %)
 template <bool BIAS>
 __device__ __forceinline__ float add_bias(const __half *bias, float value, int out)
 {
-    if constexpr (BIAS) return value + __half2float(bias[out]);
+    if constexpr (BIAS) return plus_bias(value, __half2float(bias[out]));
     else return value;
 }
 

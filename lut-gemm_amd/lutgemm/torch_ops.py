@@ -214,7 +214,8 @@ class LutLinear(torch.nn.Module):
         return Wt
 
     def forward(self, x):
-        """The bias goes with the call where it is what the constructor made of it (float16 [n] on x's device); one that the program has put in its place since (another dtype, a parameter) is added to the result."""
+        """The bias is added to the float16 result.  On the packed route it goes with the call, which gives the same bits,
+        where it is what the constructor made of it (float16 [n] on x's device)."""
         rows = x.numel() // x.shape[-1]
         if x.dtype != torch.float16:
             x = x.to(torch.float16)
@@ -223,12 +224,12 @@ class LutLinear(torch.nn.Module):
                  and bias.device == x.device and bias.is_contiguous())
         threshold = self.dense_threshold
         if rows > threshold and not (threshold == self._extends and rows <= self._packed_rows):
-            y = torch.nn.functional.linear(x, self.dense_weight(), bias if joins else None)
+            y = torch.nn.functional.linear(x, self.dense_weight())
         elif joins:
             return torch.ops.lutgemm.matvec_bias(x, self.handle, bias)
         else:
             y = torch.ops.lutgemm.matvec(x, self.handle)
-        return y if bias is None or joins else y + bias
+        return y if bias is None else y + bias
 
 
 def container_from_numpy(bW, alpha, k, n, q, num_groups, q_bias=None):

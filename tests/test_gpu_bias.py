@@ -2,23 +2,21 @@
 import numpy as np
 import pytest
 
-from test_gpu_parity import assert_within_tolerance, make, say, truth_of
+from test_gpu_parity import make, say, truth_of
 
 pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("k,n,q,g,offset", [(512, 40, 3, 128, False), (4096, 70, 2, 64, True), (1024, 1001, 5, 32, False)])
 def test_bias_on_every_kernel(lutgemm, oracle, device, k, n, q, g, offset):
-    """One row, two rows, the batch kernel and the kernel for many rows, with and without splits along k.  With weights
-    of zero the result is the bias bit for bit.  Otherwise one row and more than 16 are within the tolerance of the
-    path around sum + bias, which are rounded once; 2 to 16 rows are the result without bias plus the bias in fp16."""
+    """One row, two rows, the batch kernel and the kernel for many rows, with and without splits along k: the result
+    without bias plus the bias in fp16, bit for bit; with weights of zero, the bias."""
     import torch
     from lutgemm import synth
     w, W = make(lutgemm, synth, k, n, q, g, offset=offset, seed=k + n)
     zero = lutgemm.BCQWeight(w["bW"], w["alpha"] * 0, k, n, q, k // g, None)
     x = synth.make_x(40, k, seed=n)
     b = (np.random.default_rng(n).standard_normal(n) * 3).astype(np.float16)
-    truth = truth_of(oracle, w, x) + b.astype(np.float64)
     xd, bd = torch.from_numpy(x).to(device), torch.from_numpy(b).to(device)
     st = torch.cuda.current_stream().cuda_stream
     for m in (1, 2, 3, 16, 17, 40):
@@ -31,10 +29,7 @@ def test_bias_on_every_kernel(lutgemm, oracle, device, k, n, q, g, offset):
             torch.cuda.synchronize()
             want = torch.full_like(y, float("nan"))
             W.matvec(xd.data_ptr(), want.data_ptr(), m, st)
-            if 2 <= m <= 16:
-                assert torch.equal(y, want + bd), m
-            else:
-                assert_within_tolerance(y.cpu().numpy(), truth[:m], "m=%d splits=%d" % (m, splits))
+            assert torch.equal(y.view(torch.int16), (want + bd).view(torch.int16)), m
             zero.set_plan(4, splits)
             zero.set_batch_plan(8, splits)
             zero.matvec_bias(xd.data_ptr(), y.data_ptr(), bd.data_ptr(), m, st)
@@ -75,3 +70,20 @@ def test_layer_bias(lutgemm, oracle, device, rows):
     with pytest.raises(Exception):
         torch.ops.lutgemm.matvec_bias(x, layer.handle, b.to(device)[:-1])
     layer.weight.close()
+
+
+@pytest.mark.parametrize("rows", [1, 2, 16, 17, 40, 600])
+def test_layer_bias_has_the_bits_of_an_addition(lutgemm, device, rows):
+    """Whether the bias goes with the call or not, on the packed route and on the dense one."""
+    import torch
+    from lutgemm import synth, torch_ops
+    k, n, q, g = 1024, 200, 3, 128
+    w = synth.make_weight(k, n, q, g, seed=10)
+    c = dict(bW=w["bW"], alpha=w["alpha"], q_bias=None, k=k, n=n, q=q, num_groups=k // g)
+    b = torch.randn(n, generator=torch.Generator().manual_seed(2)).half().to(device)
+    layer, plain = torch_ops.LutLinear(c, bias=b), torch_ops.LutLinear(c)
+    x = torch.from_numpy(synth.make_x(rows, k, seed=10)).to(device)
+    say("case layer bias bits", rows)
+    assert torch.equal(layer(x).view(torch.int16), (plain(x) + b).view(torch.int16))
+    layer.weight.close()
+    plain.weight.close()
