@@ -5,7 +5,7 @@
 
 The operator launches on torch's current stream and allocates nothing but its output, so it can
 be captured into a HIP graph like any other torch op.  Batches larger than `dense_threshold`
-rows (by default more than `packed_rows` of the weight) go through the dequantised fp16 weight and the library GEMM, the route the reference takes
+rows go through the dequantised fp16 weight and the library GEMM, the route the reference takes
 for every m > 1 (lutGEMM/src/kernels.cu:73-79).  Like the reference, which dequantises into one
 grow-only scratch buffer of the process on every such call (lutGEMM/src/cuda/tmpWeight.hpp:28-35,
 lutGEMM/src/nQWeight_fp16.cu:93-99), the dense weight is rebuilt per call in a scratch buffer shared
@@ -13,38 +13,31 @@ by all layers (one per device and stream), so a layer never holds more than its 
 `keep_dense=True` keeps a private dense copy instead (2 k n bytes) and skips the rebuild.  Up to
 the threshold the library streams the packed weight
 (one or two rows through the table-lookup kernels, 3 to 16 through the batch kernel, more through the kernel
-for many rows).  The default depends on the weight and on keep_dense (default_dense_threshold, packed_rows):
+for many rows).  The default threshold depends on the weight and on keep_dense (default_dense_threshold):
 it is where the two routes met when measured on MI355X.
 """
 
 
 def default_dense_threshold(weight, keep_dense=False):
-    """Rows up to which the packed route is taken whatever the weight's size (LutLinear(dense_threshold=...)
-    overrides): 80 for one or two planes, 64 for three, 48 beyond.  The dense route costs the dequantisation (75 us up to
-    four planes, 97-130 us for five to eight at k = n = 12288) plus the GEMM; the packed route at 48 rows 40 us (one plane)
-    to 120 us (four and an offset).  packed_rows() extends the line by the size of the weight.  A layer that keeps its dense
-    copy (keep_dense) pays the GEMM alone: 32 rows for one or two planes, 16 for three to seven, 2 for eight."""
+    """Rows up to which the packed route beats dequantised weight + library GEMM (measured on MI355X
+    at k = n = 12288 and at k = 7168, n = 28672; LutLinear(dense_threshold=...) overrides).
+
+    A pass of the batch kernel over up to 16 rows costs 22 / 24 / 30 / 36 us for one to four planes
+    and 41 / 43 / 50 / 57 us for five to eight (k = n = 12288).  The dense route costs the
+    dequantisation (75 us up to four planes, 97-130 us for five to eight) plus the GEMM (50-56 us up
+    to 32 rows), so by default it only pays from the number of passes on that costs as much:
+    80 rows for one or two planes, 64 for three, 48 beyond.  A layer that keeps its dense copy
+    (keep_dense) pays the GEMM alone: 32 rows for one or two planes, 16 for three to seven, and
+    eight planes leave the packed route from three rows on (57 against 50 us).
+
+    More than 16 rows no longer take passes of 16, so the packed route would stay ahead for longer (12288 x 12288,
+    three planes, 160 rows: 130 against 192 us).  The line is kept all the same, because the routes are not
+    interchangeable: the dense one passes gradients to x, follows autocast, can be captured on a stream that has not
+    launched on the handle, and rounds the weight to fp16, so its results differ by some 4e-4 of their norm."""
     q = weight.nb
     if keep_dense:
         return 32 if q <= 2 else 16 if q <= 7 else 2
     return 80 if q <= 2 else 64 if q == 3 else 48
-
-
-def packed_rows(weight):
-    """Rows up to which the packed route beats dequantised weight + library GEMM for a weight of this size, for a layer
-    with the default threshold that keeps no dense copy.
-
-    In microseconds, with P planes (an offset counts as one): packed 8 + 1.6e-9 to 2.5e-9 k n P per row, dense
-    12 + 0.9e-6 k n + 1.1e-9 k n per row, and never less than the 30 that its launches take on the host (measured at 49 to 512
-    rows of fourteen weights from 512 x 64 to 7168 x 28672, one to eight planes).  The line is drawn with 2.3e-9, on
-    whole row tiles, and not beyond the 512 rows measured.  Packed / dense on either side of it:
-    12288 x 12288, P = 3 (160): 130 / 192 us at 160 rows, 207 / 205 at 256; P = 5 (80): 161 / 168 at 81, 195 / 167 at 97;
-    7168 x 28672, P = 2 (256): 195 / 231 at 256, 293 / 227 at 320; 4096 x 4096, P = 5 (112): 28 / 40 at 128, 45 / 38 at 256;
-    2048 x 2048, P = 2 (512): 14 / 30 at 65, 16 / 35 at 512."""
-    kn, planes = float(weight.kSize) * weight.mSize, weight.nb + int(weight.has_offset)
-    dense_us = max(30.0, 12.0 + 0.9e-6 * kn)
-    rows = (dense_us - 8.0) / (kn * (2.3e-9 * planes - 1.1e-9))
-    return min(512, int(rows) // 16 * 16)
 
 
 import weakref
@@ -155,18 +148,12 @@ class LutLinear(torch.nn.Module):
             self.weight.autotune(torch.cuda.current_stream().cuda_stream)
         self.handle = register(self.weight)
         self.in_features, self.out_features = c["k"], c["n"]
-        self._set_threshold(dense_threshold)
+        self.dense_threshold = default_dense_threshold(self.weight, keep_dense) if dense_threshold is None else dense_threshold
         self._dense = None
         if bias is not None:
             self.register_buffer("bias", torch.as_tensor(bias).to(torch.float16).to(self.device))
         else:
             self.bias = None
-
-    def _set_threshold(self, threshold):
-        self.dense_threshold = default_dense_threshold(self.weight, self.keep_dense) if threshold is None else threshold
-        # rows up to which a default threshold (one that nobody has set, here or later) is extended
-        self._extends = self.dense_threshold if threshold is None and not self.keep_dense else None
-        self._packed_rows = packed_rows(self.weight) if self._extends is not None else 0
 
     @classmethod
     def from_file(cls, path, bias=None, **kw):
@@ -179,7 +166,8 @@ class LutLinear(torch.nn.Module):
             self.weight.autotune(torch.cuda.current_stream().cuda_stream)
         self.handle = register(self.weight)
         self.in_features, self.out_features = self.weight.kSize, self.weight.mSize
-        self._set_threshold(kw.get("dense_threshold"))
+        dt = kw.get("dense_threshold")
+        self.dense_threshold = default_dense_threshold(self.weight, self.keep_dense) if dt is None else dt
         self._dense = None
         if bias is not None:
             self.register_buffer("bias", torch.as_tensor(bias).to(torch.float16).to(self.device))
@@ -222,8 +210,7 @@ class LutLinear(torch.nn.Module):
         bias = self.bias
         joins = (bias is not None and bias.dtype == torch.float16 and bias.shape == (self.out_features,) and not bias.requires_grad
                  and bias.device == x.device and bias.is_contiguous())
-        threshold = self.dense_threshold
-        if rows > threshold and not (threshold == self._extends and rows <= self._packed_rows):
+        if rows > self.dense_threshold:
             y = torch.nn.functional.linear(x, self.dense_weight())
         elif joins:
             return torch.ops.lutgemm.matvec_bias(x, self.handle, bias)

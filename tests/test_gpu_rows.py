@@ -92,31 +92,3 @@ def test_many_rows_under_capture_and_on_two_streams(lutgemm, oracle, device):
                     eager = run_matvec(lutgemm, W, x.cpu().numpy(), device)
                     assert np.array_equal(out.cpu().numpy().view(np.uint16), eager.view(np.uint16))
     W.close()
-
-
-def test_layer_takes_the_packed_route_by_its_size(lutgemm, oracle, device):
-    """A default threshold is extended by the weight's size; one that was set, at construction or later, is kept to."""
-    import torch
-    from lutgemm import synth, torch_ops
-    k, n, q, g = 4096, 512, 5, 128
-    w = synth.make_weight(k, n, q, g, offset=True, seed=8)
-    c = dict(bW=w["bW"], alpha=w["alpha"], q_bias=w["q_bias"], k=k, n=n, q=q, num_groups=k // g)
-    layer = torch_ops.LutLinear(c)
-    limit = torch_ops.packed_rows(layer.weight)
-    assert layer.dense_threshold == 48 and limit % 16 == 0 and 48 < limit <= 512
-    dense = [0]
-    weight_of = layer.dense_weight
-    layer.dense_weight = lambda: dense.__setitem__(0, dense[0] + 1) or weight_of()
-    x = synth.make_x(limit + 1, k, seed=8)
-    truth = truth_of(oracle, w, x)
-    xd = torch.from_numpy(x).to(device)
-    for rows, routes in ((49, 0), (limit, 0), (limit + 1, 1)):
-        say("case layer route", rows)
-        y = layer(xd[:rows]).cpu().double().numpy()
-        assert dense[0] == routes, rows
-        assert np.linalg.norm(y - truth[:rows]) / np.linalg.norm(truth[:rows]) <= 1e-3
-    layer.dense_threshold = 40
-    layer(xd[:41])
-    assert dense[0] == 2
-    assert torch_ops.LutLinear(c, dense_threshold=48)._packed_rows == 0
-    layer.weight.close()

@@ -127,3 +127,41 @@ def test_default_dense_threshold_follows_the_weight(lutgemm, device):
         kept.weight.close()
         assert torch_ops.LutLinear(c, dense_threshold=7).dense_threshold == 7
         layer.weight.close()
+
+
+@pytest.mark.parametrize("qbits,rows", [(2, 81), (3, 65), (5, 49), (5, 512)])
+def test_rows_above_the_default_threshold_keep_what_the_dense_route_gives(lutgemm, device, qbits, rows):
+    """The bits of the library product with the dequantised weight, a gradient for the activations, the result type of
+    autocast, and capture on a stream that has not launched on the handle, which is in use on another."""
+    from lutgemm import quantize, torch_ops
+    print("case dense route above the threshold", qbits, rows, flush=True)
+    lin, gen = _layer(6, out_f=192, in_f=512)
+    c, _ = quantize.quantize_linear(lin.weight.detach(), qbits, 128, "rtn")
+    layer = torch_ops.LutLinear(c, bias=lin.bias.detach())
+    layer(torch.zeros(1, 512, dtype=torch.float16, device=device))
+    x = torch.randn(rows, 512, generator=gen).to(torch.float16).to(device)
+    Wt = layer.dense_weight().clone()
+    want = torch.nn.functional.linear(x, Wt) + layer.bias
+    assert torch.equal(layer(x), want)
+    leaf = x.clone().requires_grad_()
+    layer(leaf).backward(torch.ones_like(want))
+    truth = Wt.double().sum(0).expand(rows, -1)          # the gradient of a sum over the outputs
+    assert (leaf.grad.double() - truth).norm() <= 1e-3 * truth.norm()   # fp16 result of an fp32 sum: 2^-11 and the sum's order
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert layer(x).dtype == (torch.nn.functional.linear(x, Wt) + layer.bias).dtype
+    side, static_x = torch.cuda.Stream(), x.clone()
+    with torch.cuda.stream(side):
+        torch.nn.functional.linear(static_x, Wt)         # the library's own first call on the stream
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            static_y = layer(static_x)
+    torch.cuda.synchronize()
+    for rep in range(3):
+        static_x.copy_(x * (rep + 1))
+        eager = layer(static_x)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(static_y, eager), rep
+    layer.weight.close()
