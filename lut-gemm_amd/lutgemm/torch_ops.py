@@ -44,6 +44,7 @@ import weakref
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from . import BCQWeight, LutGemmError, ERR_BAD_SHAPE, MAX_BATCH
 
@@ -132,6 +133,17 @@ def _(x, handle, bias):
     return x.new_empty(x.shape[:-1] + (w.mSize,))
 
 
+_transformed = getattr(torch._C._functorch, "is_functorch_wrapped_tensor", lambda bias: True)
+
+
+def _joins_call(bias, x, n):
+    """Whether the bias may go with the call, which treats it as a constant: float16 [n] on x's device, and neither
+    differentiated (in reverse or forward mode), mapped over nor traced (a compiler fuses an addition by itself)."""
+    return (bias.dtype == torch.float16 and bias.shape == (n,) and bias.device == x.device and not bias.requires_grad
+            and not torch.compiler.is_compiling() and type(bias) in (torch.Tensor, torch.nn.Parameter) and not _transformed(bias)
+            and forward_ad.unpack_dual(bias).tangent is None and bias.is_contiguous())
+
+
 class LutLinear(torch.nn.Module):
     """y = x @ W (+ bias) with W held as a packed BCQ weight on the current device.
 
@@ -203,16 +215,14 @@ class LutLinear(torch.nn.Module):
 
     def forward(self, x):
         """The bias is added to the float16 result.  On the packed route it goes with the call, which gives the same bits,
-        where it is what the constructor made of it (float16 [n] on x's device)."""
+        where it is what the constructor made of it (_joins_call)."""
         rows = x.numel() // x.shape[-1]
         if x.dtype != torch.float16:
             x = x.to(torch.float16)
         bias = self.bias
-        joins = (bias is not None and bias.dtype == torch.float16 and bias.shape == (self.out_features,) and not bias.requires_grad
-                 and bias.device == x.device and bias.is_contiguous())
         if rows > self.dense_threshold:
             y = torch.nn.functional.linear(x, self.dense_weight())
-        elif joins:
+        elif bias is not None and _joins_call(bias, x, self.out_features):
             return torch.ops.lutgemm.matvec_bias(x, self.handle, bias)
         else:
             y = torch.ops.lutgemm.matvec(x, self.handle)

@@ -87,3 +87,43 @@ def test_layer_bias_has_the_bits_of_an_addition(lutgemm, device, rows):
     assert torch.equal(layer(x).view(torch.int16), (plain(x) + b).view(torch.int16))
     layer.weight.close()
     plain.weight.close()
+
+
+@pytest.mark.parametrize("transform", ["vmap", "vmap last", "jvp", "forward mode", "grad", "vmap of grad", "backward"])
+def test_layer_bias_is_transformed_like_an_addition(lutgemm, device, transform):
+    """A bias that is mapped over or differentiated is added to the result, whose derivative in it is one."""
+    import torch
+    import torch.autograd.forward_ad as forward_ad
+    from lutgemm import synth, torch_ops
+    k, n, q, g, m = 512, 40, 3, 128, 3
+    w = synth.make_weight(k, n, q, g, seed=11)
+    layer = torch_ops.LutLinear(dict(bW=w["bW"], alpha=w["alpha"], q_bias=None, k=k, n=n, q=q, num_groups=k // g), bias=torch.zeros(n))
+    x = torch.from_numpy(synth.make_x(m, k, seed=11)).to(device)
+    y = torch.ops.lutgemm.matvec(x, layer.handle)
+    some = torch.randn(4, n, generator=torch.Generator().manual_seed(3)).half().to(device)
+    ones = torch.ones(n, dtype=torch.float16, device=device)
+
+    def call(bias):
+        return torch.func.functional_call(layer, {"bias": bias}, (x,))
+
+    say("case layer bias transform", transform)
+    if transform == "vmap":
+        assert torch.equal(torch.vmap(call)(some), y + some[:, None])
+    elif transform == "vmap last":
+        assert torch.equal(torch.vmap(call, in_dims=1)(some.t().contiguous()), y + some[:, None])
+    elif transform == "jvp":
+        value, tangent = torch.func.jvp(call, (some[0],), (ones,))
+        assert torch.equal(value, y + some[0]) and torch.equal(tangent, ones.expand(m, n))
+    elif transform == "forward mode":
+        with forward_ad.dual_level():
+            value, tangent = forward_ad.unpack_dual(call(forward_ad.make_dual(some[0], ones)))
+            assert torch.equal(value, y + some[0]) and torch.equal(tangent, ones.expand(m, n))
+    elif transform == "grad":
+        assert torch.equal(torch.func.grad(lambda b: call(b).sum())(some[0]), ones * m)
+    elif transform == "vmap of grad":
+        assert torch.equal(torch.vmap(torch.func.grad(lambda b: call(b).sum()))(some), (ones * m).expand(4, n))
+    else:
+        leaf = some[0].clone().requires_grad_()
+        call(leaf).sum().backward()
+        assert torch.equal(leaf.grad, ones * m)
+    layer.weight.close()
