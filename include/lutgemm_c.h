@@ -116,7 +116,11 @@ int lutgemm_weight_info(const lutgemm_weight *w, lutgemm_weight_info_t *info);
  * Non-finite values follow IEEE arithmetic whatever the launch plan: a NaN activation gives NaN
  * outputs, infinite partial sums give an infinity of their sign, or NaN if both signs occur.  With
  * more than one k-split the partial sums are added as fixed-point integers (2^-24 resolution);
- * a finite partial sum beyond +-4.1e6 (64 times binary16's range) counts as an infinity. */
+ * a finite partial sum beyond +-4.1e6 (64 times binary16's range) counts as an infinity (up to 16 rows; launches of more
+ * add the fp32 partial sums themselves).  From three rows on an infinite scale multiplies sums of 128 or 64 activations
+ * where the group size is a multiple of that, and single activations where it is not: infinities of both signs give NaN.
+ * More than 16 rows against a weight with non-finite scales or offsets are taken 16 per pass, with the results of such
+ * passes. */
 #define LUTGEMM_MAX_BATCH 4096
 int lutgemm_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *stream);
 

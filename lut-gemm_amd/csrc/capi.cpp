@@ -86,6 +86,7 @@ struct lutgemm_weight {
     int compute_units;
     uint8_t *d_signs;
     uint16_t *d_scales;
+    bool finite_scales;           // no infinity or NaN among the scales and offsets
     std::mutex slot_mutex;
     StreamSet set[kStreamSlots];
     int slots_used;               // sets that serve a stream
@@ -593,6 +594,27 @@ int copy_tiles(lutgemm_weight *w, const void *signs, const void *scales, hipMemc
     return LUTGEMM_OK;
 }
 
+// Whether the kernel for many rows takes a call.  It contracts with the scales as matrix operand, where an infinite one
+// gives NaN as soon as the signs of its group mix; the batch kernel multiplies it with the group's sum.  And it addresses
+// 64 rows with 32 bits.  Otherwise the batch kernel takes the rows, 16 per pass.
+bool takes_rows_kernel(const lutgemm_weight *w, int m)
+{
+    return m > kRowsPerPass && w->shape.k <= kMaxRowsK && w->finite_scales;
+}
+
+// Sets w->finite_scales from the tiles on the device.  The answer comes in a word of set 0, which is back at zero afterwards.
+int check_scales(lutgemm_weight *w)
+{
+    unsigned long long *word = w->set[0].accum, found = 0;
+    hipError_t e = lutgemm_kernels::launch_find_non_finite(w->d_scales, scale_bytes(w->shape) / 16, word, nullptr);
+    if (e != hipSuccess) return hip_fail(e, "launch find_non_finite_kernel");
+    e = hipMemcpy(&found, word, sizeof found, hipMemcpyDeviceToHost);   // behind the kernel
+    if (e == hipSuccess && found) e = hipMemset(word, 0, sizeof found);
+    if (e != hipSuccess) return hip_fail(e, "reading whether scales are finite");
+    w->finite_scales = found == 0;
+    return LUTGEMM_OK;
+}
+
 // New handle for shape s on the current device from tiles already in the device layout
 // (host or device memory, `kind` says which).
 int create_from_tiles(const Shape &s, const void *signs, const void *scales, hipMemcpyKind kind,
@@ -602,6 +624,7 @@ int create_from_tiles(const Shape &s, const void *signs, const void *scales, hip
     int st = new_handle(s, &w);
     if (st != LUTGEMM_OK) return st;
     st = copy_tiles(w, signs, scales, kind);
+    if (st == LUTGEMM_OK) st = check_scales(w);
     if (st != LUTGEMM_OK) {
         lutgemm_weight_destroy(w);
         return st;
@@ -734,6 +757,7 @@ int create_common(const uint32_t *bW, const void *alpha, const void *q_bias, boo
         }
         if (st == LUTGEMM_OK) st = copy_tiles(w, signs.data(), scales.data(), hipMemcpyHostToDevice);
     }
+    if (st == LUTGEMM_OK) st = check_scales(w);
     if (st != LUTGEMM_OK) {
         lutgemm_weight_destroy(w);
         return st;
@@ -891,8 +915,8 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
         return e == hipSuccess ? LUTGEMM_OK : hip_fail(e, "launch add_bias_kernel");
     };
     // More rows than a pass of the batch kernel takes: one launch over all of them, except for the allocation-free entry
-    // point (its words hold no partial sums) and for a k beyond the kernel's 32-bit offsets.
-    if (m > kRowsPerPass && !static_ws && s.k <= kMaxRowsK) {
+    // point (its words hold no partial sums).
+    if (takes_rows_kernel(w, m) && !static_ws) {
         lutgemm_kernels::RowsGrid g{};
         RowsPlan plan = choose_rows_plan(s, w->compute_units, m, true);
         if (plan.k_splits > 1 && !(g.partials = partials_of(mw, slot, stream)))
@@ -1529,7 +1553,7 @@ int lutgemm_weight_plan_for(const lutgemm_weight *w, int m, int *workgroups, int
     if (m < 1 || m > LUTGEMM_MAX_BATCH)
         return fail(LUTGEMM_ERR_BAD_SHAPE, "m=%d outside 1..%d", m, LUTGEMM_MAX_BATCH);
     Plan p = m == 1 ? w->plan : w->plan2;
-    if (m > kRowsPerPass && w->shape.k <= kMaxRowsK) {
+    if (takes_rows_kernel(w, m)) {
         const RowsPlan r = choose_rows_plan(w->shape, w->compute_units, m, true);
         p = Plan{lutgemm_kernels::kRowsWaves, r.ntiles * r.row_chunks, r.blocks_per_split, r.k_splits};
     } else if (m >= 3) {

@@ -150,6 +150,9 @@ hipError_t launch_gather_columns(const void *cols, void *rows, int k, int m, hip
 // hipErrorInvalidValue for a weight beyond the kernels' grids (2^31 threads)
 hipError_t launch_pack(const PackArgs &a, hipStream_t stream);
 
+// *found = 1 if one of the halves in 16 * `pieces` bytes is an infinity or a NaN, else as it was
+hipError_t launch_find_non_finite(const uint16_t *halves, size_t pieces, unsigned long long *found, hipStream_t stream);
+
 hipError_t launch_dequantize(const DequantArgs &a, hipStream_t stream);
 
 // The matvec's loads without its arithmetic (same grid and arguments; x, y and accum unused):

@@ -87,7 +87,27 @@ __global__ __launch_bounds__(256) void pack_scales_kernel(PackArgs a)
     a.scales[idx] = v;
 }
 
+// Bound by reading the scales (4096 x 16384, four planes with offset: 5 MB, a few microseconds behind the kernels above).
+__global__ __launch_bounds__(256) void find_non_finite_kernel(const u32x4 *halves, size_t pieces, unsigned long long *found)
+{
+    bool any = false;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < pieces; i += (size_t)gridDim.x * blockDim.x) {
+        const u32x4 v = halves[i];
+#pragma unroll
+        for (int c = 0; c < 4; c++) any |= (v[c] & 0x7c00u) == 0x7c00u || (v[c] & 0x7c000000u) == 0x7c000000u;
+    }
+    if (any) *found = 1;   // every thread that stores stores the same
+}
+
 }  // namespace
+
+hipError_t launch_find_non_finite(const uint16_t *halves, size_t pieces, unsigned long long *found, hipStream_t stream)
+{
+    const size_t blocks = (pieces + 255) / 256;
+    hipLaunchKernelGGL(find_non_finite_kernel, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, stream,
+                       reinterpret_cast<const u32x4 *>(halves), pieces, found);
+    return hipGetLastError();
+}
 
 hipError_t launch_pack(const PackArgs &a, hipStream_t stream)
 {

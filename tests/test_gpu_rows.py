@@ -92,3 +92,32 @@ def test_many_rows_under_capture_and_on_two_streams(lutgemm, oracle, device):
                     eager = run_matvec(lutgemm, W, x.cpu().numpy(), device)
                     assert np.array_equal(out.cpu().numpy().view(np.uint16), eager.view(np.uint16))
     W.close()
+
+
+@pytest.mark.parametrize("q,g,offset,value", [(1, 128, False, np.inf), (3, 512, False, -np.inf), (2, 64, True, np.inf),
+                                              (2, 32, False, np.inf), (3, 128, True, np.nan), (2, 128, False, 65520.0)])
+def test_many_rows_non_finite_scales(lutgemm, device, tmp_path, q, g, offset, value):
+    """Non-finite scales (or offsets: the last group's) give the bits of 16 rows at a time, whichever way the weight was
+    made; an infinite scale of a group that is one sum (64 or 128 activations) gives infinities, not NaN."""
+    from lutgemm import synth
+    k, n, m = 2048, 70, 40
+    w = synth.make_weight(k, n, q, g, offset=offset, seed=q + g)
+    alpha, z = w["alpha"].copy(), None if w["q_bias"] is None else w["q_bias"].copy()
+    alpha[1, 0, 5] = value
+    if z is not None:
+        z[-1, 64] = value
+    x = synth.make_x(m, k, seed=12)
+    W = lutgemm.BCQWeight(w["bW"], alpha, k, n, q, k // g, z)
+    W.save(str(tmp_path / "w.lutw"))
+    made = [W, lutgemm.BCQWeight.load(str(tmp_path / "w.lutw")), W.clone()]
+    say("case rows non-finite scales", q, g, offset, value)
+    want = np.concatenate([run_matvec(lutgemm, W, x[:16], device), run_matvec(lutgemm, W, x[16:32], device),
+                           run_matvec(lutgemm, W, x[24:], device)[8:]])
+    for V in made:
+        for cols in (False, True):
+            y = run_matvec(lutgemm, V, x, device, cols=cols)
+            assert np.array_equal(y.view(np.uint16), want.view(np.uint16))
+    assert not np.isfinite(want[:, 5]).any() and (g not in (64, 128) or np.isnan(value) or np.isinf(want[:, 5]).all())
+    assert np.isfinite(np.delete(want, [5, 64], axis=1)).all()
+    for V in made:
+        V.close()
