@@ -40,7 +40,7 @@ typedef enum lutgemm_status {
 
 /* Opaque packed weight: device-resident sign tiles, scales and offsets plus the launch plan
  * and the workspace of the launching streams (split-k accumulators: 64-bit words, one per output and
- * activation row of a pass; staging rows of the column-batched form).  Stands in for class lutGEMM::nQWeight_fp16
+ * activation row of a pass; staging rows of the column-batched form; partial sums of calls of more than 16 rows).  Stands in for class lutGEMM::nQWeight_fp16
  * (lutGEMM/include/nQWeight_fp16.h:27-52). */
 typedef struct lutgemm_weight lutgemm_weight;
 
@@ -84,7 +84,8 @@ int lutgemm_weight_info(const lutgemm_weight *w, lutgemm_weight_info_t *info);
  * on `stream` (a hipStream_t passed as void*, NULL = the default stream).  x and y are
  * device pointers, row-major [m][k] and [m][n], x 16-byte aligned.  The offset term is applied
  * iff the weight was created with q_bias.  No memset of y is needed and none is issued; a
- * call of up to 16 rows allocates nothing.  The result is deterministic (bit-identical from launch to launch).
+ * call of up to 16 rows allocates nothing.  The result is deterministic (bit-identical from launch to launch,
+ * captured or not).
  * Replaces lutGEMM::matmul(void* output, void* input, nQWeight_fp16&, int m, int algo)
  * (lutGEMM/include/kernels.h:27, lutGEMM/src/kernels.cu:64-71), which for m == 1 runs
  * kernel::nqmv (mv_fp16.hpp:121) or kernel::nqmv_bias (mv_fp16_bias.hpp:143) and for m > 1
@@ -95,7 +96,9 @@ int lutgemm_weight_info(const lutgemm_weight *w, lutgemm_weight_info_t *info);
  * matrix cores while a tile is in registers (any number of planes and any group size; weights of
  * more than four planes with workgroups of exactly eight wavefronts), and more rows through a kernel that contracts
  * a tile with up to 64 of them.  A launch of more than 16 rows that splits k keeps partial sums in memory of the stream's set,
- * allocated (up to 16 MiB) at the first such launch; under graph capture, where it cannot be, k is not split.  Batch results are deterministic and within
+ * allocated when a launch first needs as much (a power of two of bytes, 2 KiB to 16 MiB; mostly 1 to 4 MiB; also under graph
+ * capture, so that a captured launch gives the bits of an eager one) and held until the handle is destroyed; where the
+ * device has no such memory left, k is not split and a result may differ in the last bit.  Batch results are deterministic and within
  * the same tolerance, but a row may differ in the last bit from its own one-row call (another order
  * of the fp32 additions).
  * Launches on one stream run one after the other and share one set of split-k accumulators of the

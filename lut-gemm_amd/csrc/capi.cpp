@@ -49,6 +49,7 @@ constexpr int kMaxSplits = 128;  // the split-k arrival count has 8 bits, the su
 constexpr int kStreamSlots = 4;  // sets of split-k words per handle: one per stream that launches on it
 constexpr int kRowsPerPass = lutgemm_kernels::kBatchRows;  // activation rows a launch can take (rows of split-k words per set)
 constexpr int kMaxRowsK = 1 << 24;  // the kernel for more rows addresses 64 of them with 32 bits
+constexpr int kRoomSizes = 14;   // sizes of the room for partial sums: 2^0 .. 2^13 units (kPartialUnits)
 constexpr int kTableRows = 2;    // rows per pass of the table-lookup kernels
 constexpr int kStagedColumns = 16;  // column-batched calls up to this m never allocate
 
@@ -73,7 +74,8 @@ struct StreamSet {
     unsigned long long *accum;   // kRowsPerPass x (padded outputs) split-k words, zero between launches
     void *xrows;                 // staging of column-batched activations: xrows_cols rows of k halves,
     int xrows_cols;              //   grown on demand
-    float *partials;             // sums of launches of more than 16 rows that split k: from the first such launch on
+    float *partials[kRoomSizes]; // room for the sums of launches of more than 16 rows that split k: [c] holds 2^c units,
+    bool no_room;                //   from the first launch that needs it on; an allocation failed: none is tried again
     hipEvent_t done;             // recorded behind the set's latest launch (only while done_valid)
     bool done_valid;
     unsigned long long last_use;
@@ -297,11 +299,15 @@ FusedPlan choose_fused_batch_plan(const Shape *const *shapes, const int *rows, i
 
 // Launch plan of the kernel for more than 16 rows (rows_body.h): output batches per workgroup (8, or 4 with the
 // wavefronts in two groups along k), row tiles of 16 per workgroup, workgroups along the rows and along k.
-struct RowsPlan { int nw, row_tiles, row_chunks, ntiles, blocks_per_split, k_splits; };
+struct RowsPlan {
+    int nw, row_tiles, row_chunks, ntiles, blocks_per_split, k_splits;
+    size_t units(const Shape &s) const { return (size_t)s.nb * row_chunks * row_tiles * k_splits; }   // of partial sums
+};
 
 // Sums that split k through memory come in units of 16 rows x 32 outputs (2 KiB).  A launch splits k to fill the
 // device, so some 256 workgroups of 8 batches x 4 row tiles bound what it needs: 16 MiB, less for narrow weights.
 constexpr size_t kPartialUnits = 8192, kPartialUnitBytes = 2048;
+static_assert(kPartialUnits == (size_t)1 << (kRoomSizes - 1), "the largest plan's room is the largest there is");
 constexpr int kMaxRowsSplits = 32, kMaxSplitChunks = 16;
 size_t partial_units(const Shape &s)
 {
@@ -399,18 +405,35 @@ int alloc_workspace(lutgemm_weight *w)
     return alloc_set(w, 0);
 }
 
-// The set's room for partial sums, allocated once (it never moves, so another call on the stream may hold it); null
-// where it is not there and cannot be had: under graph capture, or out of memory.  The caller then does not split k.
-float *partials_of(lutgemm_weight *w, int slot, void *stream)
+// Room for `units` units of partial sums in the set; null where the device has none, and the caller then does not split k.
+// A power of two of units is allocated for the first plan that needs that much.  It stays where it is until the handle is
+// destroyed, since launches in flight and captured graphs hold its address; all sizes together are less than four times
+// what the largest plan needs.  The room belongs to the set like its split-k words: handles that shared one per stream would
+// race where a graph captured on the stream is replayed on another.
+// The allocation is part of no graph and waits for nothing, so it is also made while this stream or another is being
+// captured, which plain hipMalloc is not allowed to: a captured launch has the plan, and the bits, of an eager one.
+float *partials_of(lutgemm_weight *w, int slot, size_t units)
 {
+    int size = 0;
+    while (((size_t)1 << size) < units) size++;
     std::lock_guard<std::mutex> lock(w->slot_mutex);
     StreamSet &t = w->set[slot];
-    if (!t.partials && !stream_capturing(stream) &&
-        hipMalloc((void **)&t.partials, partial_units(w->shape) * kPartialUnitBytes) != hipSuccess) {
-        (void)hipGetLastError();
-        t.partials = nullptr;
+    for (int c = size; c < kRoomSizes; c++)
+        if (t.partials[c]) return t.partials[c];
+    if (t.no_room || size >= kRoomSizes) return nullptr;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // of this host thread, until it is exchanged back
+    hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+    if (e == hipSuccess) {
+        e = hipMalloc((void **)&t.partials[size], kPartialUnitBytes << size);
+        const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+        if (e == hipSuccess) e = back;
     }
-    return t.partials;
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        t.no_room = true;   // the same call keeps giving the same bits
+        if (!t.partials[size]) return nullptr;
+    }
+    return t.partials[size];
 }
 
 size_t workspace_bytes(const lutgemm_weight *w)
@@ -418,7 +441,8 @@ size_t workspace_bytes(const lutgemm_weight *w)
     size_t bytes = 0;
     for (int i = 0; i < kStreamSlots; i++) {
         if (w->set[i].accum) bytes += set_words(w) * sizeof(unsigned long long);
-        if (w->set[i].partials) bytes += partial_units(w->shape) * kPartialUnitBytes;
+        for (int c = 0; c < kRoomSizes; c++)
+            if (w->set[i].partials[c]) bytes += kPartialUnitBytes << c;
         if (w->set[i].xrows) bytes += (size_t)w->set[i].xrows_cols * w->shape.k * sizeof(uint16_t);
     }
     return bytes;
@@ -919,7 +943,7 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
     if (takes_rows_kernel(w, m) && !static_ws) {
         lutgemm_kernels::RowsGrid g{};
         RowsPlan plan = choose_rows_plan(s, w->compute_units, m, true);
-        if (plan.k_splits > 1 && !(g.partials = partials_of(mw, slot, stream)))
+        if (plan.k_splits > 1 && !(g.partials = partials_of(mw, slot, plan.units(s))))
             plan = choose_rows_plan(s, w->compute_units, m, false);
         a.ntiles = plan.ntiles;
         a.k_splits = plan.k_splits;
@@ -1255,7 +1279,7 @@ int lutgemm_weight_destroy(lutgemm_weight *w)
     for (StreamSet &t : w->set) {
         ptrs.push_back(t.accum);
         ptrs.push_back(t.xrows);
-        ptrs.push_back(t.partials);
+        ptrs.insert(ptrs.end(), t.partials, t.partials + kRoomSizes);
         if (t.done) (void)hipEventDestroy(t.done);
     }
     for (void *p : ptrs)
@@ -1301,6 +1325,7 @@ int lutgemm_weight_reset_workspace(lutgemm_weight *w, void *stream)
     for (StreamSet &t : w->set) {
         t.stream = nullptr;
         t.done_valid = false;
+        t.no_room = false;
         if (!t.accum) continue;
         e = lutgemm_kernels::launch_fill_zero(t.accum, set_words(w), static_cast<hipStream_t>(stream));
         if (e != hipSuccess) return hip_fail(e, "launch fill_zero_kernel");

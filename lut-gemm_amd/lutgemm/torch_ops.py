@@ -3,8 +3,9 @@
   torch.ops.lutgemm.matvec(x, handle)   y[..., n] = x[..., k] @ W  for a packed BCQ weight
   LutLinear                             nn.Module around one packed weight (+ optional bias)
 
-The operator launches on torch's current stream and allocates nothing but its output, so it can
-be captured into a HIP graph like any other torch op.  Batches larger than `dense_threshold`
+The operator launches on torch's current stream and allocates nothing but its output (and, when more than 16
+rows first need it, the handle's room for partial sums, which capture allows), so it can
+be captured into a HIP graph like any other torch op once it has run on the capturing stream.  Batches larger than `dense_threshold`
 rows go through the dequantised fp16 weight and the library GEMM, the route the reference takes
 for every m > 1 (lutGEMM/src/kernels.cu:73-79).  Like the reference, which dequantises into one
 grow-only scratch buffer of the process on every such call (lutGEMM/src/cuda/tmpWeight.hpp:28-35,

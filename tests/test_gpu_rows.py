@@ -59,8 +59,8 @@ def test_many_rows_non_finite_activations(lutgemm, device, q, g):
 
 
 def test_many_rows_under_capture_and_on_two_streams(lutgemm, oracle, device):
-    """A capture on a stream whose set has no room for partial sums yet does not split k; once it has, eager launches,
-    replays and a second stream give the same bits."""
+    """Whether the stream's set has room for partial sums already or gets it under capture: eager launches, replays and a
+    second stream give the same bits."""
     import torch
     from lutgemm import synth
     k, n, q, g, m = 8192, 512, 3, 128, 40
@@ -88,9 +88,8 @@ def test_many_rows_under_capture_and_on_two_streams(lutgemm, oracle, device):
                 graph.replay()
                 torch.cuda.synchronize()
                 assert_within_tolerance(out.cpu().numpy(), t, "replay %d" % rep)
-                if room:
-                    eager = run_matvec(lutgemm, W, x.cpu().numpy(), device)
-                    assert np.array_equal(out.cpu().numpy().view(np.uint16), eager.view(np.uint16))
+                eager = run_matvec(lutgemm, W, x.cpu().numpy(), device)
+                assert np.array_equal(out.cpu().numpy().view(np.uint16), eager.view(np.uint16)), (room, rep)
     W.close()
 
 
@@ -121,3 +120,72 @@ def test_many_rows_non_finite_scales(lutgemm, device, tmp_path, q, g, offset, va
     assert np.isfinite(np.delete(want, [5, 64], axis=1)).all()
     for V in made:
         V.close()
+
+
+def test_many_rows_beside_a_capture(lutgemm, device):
+    """A launch that needs room for partial sums, made by another host thread while a stream is being captured in global
+    mode, neither spoils the capture nor takes another plan."""
+    import threading
+
+    import torch
+    from lutgemm import synth
+    k, n, q, g, m = 8192, 512, 3, 128, 40
+    w, W = make(lutgemm, synth, k, n, q, g, seed=13)
+    assert W.plan(m)["k_splits"] > 1
+    x = torch.from_numpy(synth.make_x(m, k, seed=13)).to(device)
+    want = run_matvec(lutgemm, W, x.cpu().numpy(), device)
+    y, z = (torch.zeros((m, n), dtype=torch.float16, device=device) for _ in range(2))
+    mine, other = torch.cuda.Stream(), torch.cuda.Stream()
+    W.matvec(x.data_ptr(), y.data_ptr(), 1, other.cuda_stream)          # the stream's set, without room for partial sums
+    torch.cuda.synchronize()
+    errors = []
+
+    def work():
+        try:
+            W.matvec(x.data_ptr(), y.data_ptr(), m, other.cuda_stream)
+        except Exception as e:   # reported by the main thread
+            errors.append(repr(e))
+
+    say("case rows beside a capture")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(mine):
+        z.add_(0.0)
+        mine.synchronize()
+        with torch.cuda.graph(graph, stream=mine):
+            z.add_(1.0)
+            thread = threading.Thread(target=work)
+            thread.start()
+            thread.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    assert np.array_equal(y.cpu().numpy().view(np.uint16), want.view(np.uint16))
+    for rep in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(z, torch.full_like(z, rep + 1.0)), rep
+    W.close()
+
+
+def test_room_for_partial_sums_is_what_the_plan_needs(lutgemm, device):
+    """A handle's device memory grows by less than twice what the plan of a call exchanges, once for calls that need as
+    much, and not at all by calls that do not split k."""
+    from lutgemm import synth
+    k, n, q, g = 4096, 1024, 4, 128
+    w, W = make(lutgemm, synth, k, n, q, g, seed=14)
+    x = synth.make_x(512, k, seed=14)
+    before, largest = W.info().device_bytes, 0
+    for m in (512, 20, 32, 100, 64):
+        plan = W.plan(m)
+        say("case room", m, plan)
+        run_matvec(lutgemm, W, x[:m], device)
+        grown = W.info().device_bytes - before
+        if plan["k_splits"] == 1:
+            assert grown == 0, m
+            continue
+        # fp32 sums of whole tiles of 16 rows (up to 4 of them in a workgroup) and 32 outputs
+        largest = max(largest, plan["k_splits"] * 4 * (n + 31) // 32 * 32 * -(-m // 64) * 64)
+        assert 0 < grown < 4 * largest, (m, grown, largest)
+        run_matvec(lutgemm, W, x[:m], device)
+        assert W.info().device_bytes - before == grown
+    assert largest
+    W.close()
