@@ -135,13 +135,13 @@ int lutgemm_matvec_bias(const lutgemm_weight *w, const void *x, void *y, const v
 /* lutgemm_matvec without any allocation, for callers that cannot allocate: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the
  * reference.  Same arguments, same kernels and bit-identical results; the only difference is where
- * the split-k accumulators live: not in the handle's allocation but in a static device array of
- * the library (8 MiB on every device the library runs on, held until the process ends), whose
- * address is looked up once per device.  Limit: n <= 65,536 outputs (LUTGEMM_ERR_UNSUPPORTED
+ * the split-k accumulators and partial sums live: not in the handle's allocation but in static device arrays of
+ * the library (24 MiB on every device the library runs on, held until the process ends), whose
+ * addresses are looked up once per device.  Limit: n <= 65,536 outputs (LUTGEMM_ERR_UNSUPPORTED
  * beyond).  The call performs no hipMalloc / hipFree and calls no allocating library routine.  All
- * calls on one device share that device's array, whatever the handle or stream: calls that overlap
+ * calls on one device share that device's arrays, whatever the handle or stream: calls that overlap
  * in time on one device race on it (issue them on one stream, or use lutgemm_matvec, which keeps
- * accumulators per handle and stream).  Completed launches leave the array at zero; after a launch
+ * accumulators per handle and stream).  Completed launches leave the accumulators at zero; after a launch
  * that failed in the middle of a batched call the next call clears it with a fill kernel first. */
 int lutgemm_matvec_static(const lutgemm_weight *w, const void *x, void *y, int m, void *stream);
 
@@ -255,8 +255,7 @@ int lutgemm_weight_plan_for(const lutgemm_weight *w, int m, int *workgroups, int
  * (1..12 wavefronts per workgroup, 1..min(k/512 rounded up, 128) k-splits). */
 int lutgemm_weight_set_plan(lutgemm_weight *w, int waves_per_group, int k_splits);
 
-/* Override the batch kernel's launch plan (calls with 3 to 16 rows, and the passes of 16 rows that
- * lutgemm_matvec_static makes of more): 8..16 wavefronts per
+/* Override the batch kernel's launch plan (calls with 3 to 16 rows): 8..16 wavefronts per
  * workgroup (exactly 8 for weights of more than four planes; fewer than 16 where four scale
  * groups per 128 k leave less LDS) and the k-splits; both 0: back to the automatic choice.
  * LUTGEMM_ERR_BAD_SHAPE if the request cannot be launched.  No launch on the handle may be in

@@ -307,6 +307,7 @@ struct RowsPlan {
 // Sums that split k through memory come in units of 16 rows x 32 outputs (2 KiB).  A launch splits k to fill the
 // device, so some 256 workgroups of 8 batches x 4 row tiles bound what it needs: 16 MiB, less for narrow weights.
 constexpr size_t kPartialUnits = 8192, kPartialUnitBytes = 2048;
+static_assert(kPartialUnits * kPartialUnitBytes == lutgemm_kernels::kStaticPartials * sizeof(float), "both entry points take the same plans");
 static_assert(kPartialUnits == (size_t)1 << (kRoomSizes - 1), "the largest plan's room is the largest there is");
 constexpr int kMaxRowsSplits = 32, kMaxSplitChunks = 16;
 size_t partial_units(const Shape &s)
@@ -857,7 +858,7 @@ int read_file(const char *path, Shape *s, std::vector<uint8_t> *signs, std::vect
     return st;
 }
 
-// `static_ws`: take the split-k words from the static device array instead of the handle's
+// `static_ws`: take the split-k words and partial sums from the static device arrays instead of the handle's
 // per-stream sets (rows form only; nothing on this route allocates).
 int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *stream, bool cols, bool static_ws,
                const void *bias = nullptr)
@@ -881,6 +882,7 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
         return fail(LUTGEMM_ERR_BAD_SHAPE, "x must be 16-byte aligned");
     hipStream_t st = static_cast<hipStream_t>(stream);
     int slot = 0;
+    float *static_partials = nullptr;
     SetLease lease;   // ends when this call returns
     if (static_ws) {
         const size_t words = lutgemm_kernels::kStaticSplitKWords;
@@ -888,8 +890,11 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
             return fail(LUTGEMM_ERR_UNSUPPORTED,
                         "n=%d is beyond what the static workspace holds (%zu outputs per activation row)", s.n,
                         words / kRowsPerPass);
-        hipError_t es = lutgemm_kernels::static_split_k_words(w->device, &a.accum);
-        if (es != hipSuccess) return hip_fail(es, "hipGetSymbolAddress(static split-k words)");
+        lutgemm_kernels::StaticWorkspace at;
+        hipError_t es = lutgemm_kernels::static_workspace(w->device, &at);
+        if (es != hipSuccess) return hip_fail(es, "hipGetSymbolAddress(static workspace)");
+        a.accum = at.words;
+        static_partials = at.partials;
         if (g_static_dirty[w->device].exchange(false)) {  // a launch failed half way through a call: start from zero again
             hipError_t e = lutgemm_kernels::launch_fill_zero(a.accum, words, st);
             if (e != hipSuccess) {
@@ -938,12 +943,11 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
         const hipError_t e = lutgemm_kernels::launch_add_bias(y, bias, m, s.n, st);
         return e == hipSuccess ? LUTGEMM_OK : hip_fail(e, "launch add_bias_kernel");
     };
-    // More rows than a pass of the batch kernel takes: one launch over all of them, except for the allocation-free entry
-    // point (its words hold no partial sums).
-    if (takes_rows_kernel(w, m) && !static_ws) {
+    // more rows than a pass of the batch kernel takes: one launch over all of them
+    if (takes_rows_kernel(w, m)) {
         lutgemm_kernels::RowsGrid g{};
         RowsPlan plan = choose_rows_plan(s, w->compute_units, m, true);
-        if (plan.k_splits > 1 && !(g.partials = partials_of(mw, slot, plan.units(s))))
+        if (plan.k_splits > 1 && !(g.partials = static_ws ? static_partials : partials_of(mw, slot, plan.units(s))))
             plan = choose_rows_plan(s, w->compute_units, m, false);
         a.ntiles = plan.ntiles;
         a.k_splits = plan.k_splits;

@@ -134,12 +134,16 @@ hipError_t launch_fill_zero(unsigned long long *words, size_t count, hipStream_t
 // Split-k words of the allocation-free entry point: a static device array of kStaticSplitKWords
 // 64-bit words (8 MiB on every device the library runs on, enough for 65,536 outputs per
 // activation row of a pass of kBatchRows rows), zero at load and zero again after every completed
-// launch.
-// Returns its device address on `device`, which must be the current device (0 <= device <
+// launch; and the room for the partial sums of launch_rows (16 MiB, as much as any plan needs).
+// static_workspace gives their device addresses on `device`, which must be the current device (0 <= device <
 // kMaxDevices); looked up once per device.
-constexpr size_t kStaticSplitKWords = (size_t)1 << 20;
+constexpr size_t kStaticSplitKWords = (size_t)1 << 20, kStaticPartials = (size_t)1 << 22;
+struct StaticWorkspace {
+    unsigned long long *words;
+    float *partials;
+};
 constexpr int kMaxDevices = 64;
-hipError_t static_split_k_words(int device, unsigned long long **words);
+hipError_t static_workspace(int device, StaticWorkspace *out);
 
 // y [m][n] += bias [n], fp16
 hipError_t launch_add_bias(void *y, const void *bias, int m, int n, hipStream_t stream);

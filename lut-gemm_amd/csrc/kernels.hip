@@ -38,9 +38,10 @@ using namespace lutgemm_layout;
 
 namespace {
 
-// Split-k words of the allocation-free entry point.  In host code this name is not a device
-// address, only the handle hipGetSymbolAddress takes; kernels get the address it returns.
+// Split-k words and partial sums of the allocation-free entry point.  In host code these names are not device
+// addresses, only the handles hipGetSymbolAddress takes; kernels get the addresses it returns.
 static __device__ __align__(256) unsigned long long scratch[kStaticSplitKWords];
+static __device__ __align__(256) float scratch_partials[kStaticPartials];
 
 constexpr int kTableFloats = 256 * kLanes;  // one table set: 64 KiB
 
@@ -866,20 +867,20 @@ hipError_t launch_matvec(int q, int has_offset, int gsub, const MatvecArgs &a, i
     }
 }
 
-hipError_t static_split_k_words(int device, unsigned long long **words)
+hipError_t static_workspace(int device, StaticWorkspace *out)
 {
     static std::mutex mutex;
-    static unsigned long long *address[kMaxDevices];  // each device holds its own copy of the array
+    static StaticWorkspace address[kMaxDevices];  // each device holds its own copy of the arrays
     if (device < 0 || device >= kMaxDevices) return hipErrorInvalidDevice;
     std::lock_guard<std::mutex> lock(mutex);
-    if (!address[device]) {
-        unsigned long long *p = nullptr;
-        const hipError_t e = hipGetSymbolAddress((void **)&p, HIP_SYMBOL(scratch));
+    StaticWorkspace &at = address[device];
+    if (!at.words || !at.partials) {
+        hipError_t e = hipGetSymbolAddress((void **)&at.words, HIP_SYMBOL(scratch));
+        if (e == hipSuccess) e = hipGetSymbolAddress((void **)&at.partials, HIP_SYMBOL(scratch_partials));
         if (e != hipSuccess) return e;
-        if (!p) return hipErrorInvalidSymbol;
-        address[device] = p;
+        if (!at.words || !at.partials) return hipErrorInvalidSymbol;
     }
-    *words = address[device];
+    *out = at;
     return hipSuccess;
 }
 

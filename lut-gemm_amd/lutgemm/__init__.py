@@ -288,7 +288,7 @@ class BCQWeight:
         _check(load().lutgemm_matvec_bias(self._h, x_ptr, y_ptr, bias_ptr or None, m, stream or None))
 
     def matvec_static(self, x_ptr, y_ptr, m=1, stream=0):
-        """matvec with the split-k words in the library's static device array: allocates nothing."""
+        """matvec with its workspace in the library's static device arrays: allocates nothing."""
         _check(load().lutgemm_matvec_static(self._h, x_ptr, y_ptr, m, stream or None))
 
     def matvec_cols(self, x_ptr, y_ptr, m=1, stream=0):

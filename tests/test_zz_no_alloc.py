@@ -59,3 +59,21 @@ def test_static_workspace_rejects_what_it_cannot_hold(lutgemm, device):
     assert st == lutgemm.ERR_UNSUPPORTED
     assert b"static workspace" in L.lutgemm_last_error()
     W.close()
+
+
+@pytest.mark.parametrize("k,n,q,g,off,m,splits", [(8192, 500, 3, 128, True, 40, True), (49152, 40, 2, 64, False, 63, True),
+                                                  (512, 8200, 1, 256, False, 200, False)])
+def test_static_workspace_entry_point_matches_matvec_for_many_rows(lutgemm, device, k, n, q, g, off, m, splits):
+    """More than 16 rows, with and without splits along k, bit for bit, and a call of up to 16 rows in between, whose
+    words have to be at zero."""
+    from lutgemm import synth
+    print("case static rows", k, n, q, g, off, m, flush=True)
+    w = synth.make_weight(k, n, q, g, offset=off, seed=k + n)
+    W = lutgemm.BCQWeight(w["bW"], w["alpha"], k, n, q, k // g, w["q_bias"])
+    assert (W.plan(m)["k_splits"] > 1) == splits
+    x = synth.make_x(m, k, seed=n)
+    for rows in (m, 9, m, 17):
+        want = run(lutgemm, W, x[:rows], device, static=False)
+        got = run(lutgemm, W, x[:rows], device, static=True)
+        assert np.array_equal(got.view(np.uint16), want.view(np.uint16)), rows
+    W.close()
