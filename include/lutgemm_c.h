@@ -244,7 +244,8 @@ int lutgemm_weight_plan(const lutgemm_weight *w, int *workgroups, int *waves_per
                         int *k_splits, int *k_blocks_per_group);
 
 /* The same for the launches a call with m activation rows makes (m = 1: the plan above; m = 2:
- * the two-row plan; 3 <= m <= 16: the batch kernel's plan; beyond: that of the kernel for many rows).  LUTGEMM_ERR_BAD_SHAPE for m outside
+ * the two-row plan; 3 <= m <= 16: the batch kernel's plan; beyond: that of the kernel for many rows, or the batch
+ * kernel's if it takes them, with non-finite scales or a plan of the caller's).  LUTGEMM_ERR_BAD_SHAPE for m outside
  * 1..LUTGEMM_MAX_BATCH.  No counterpart in the reference. */
 int lutgemm_weight_plan_for(const lutgemm_weight *w, int m, int *workgroups, int *waves_per_group,
                             int *k_splits, int *k_blocks_per_group);
@@ -255,7 +256,8 @@ int lutgemm_weight_plan_for(const lutgemm_weight *w, int m, int *workgroups, int
  * (1..12 wavefronts per workgroup, 1..min(k/512 rounded up, 128) k-splits). */
 int lutgemm_weight_set_plan(lutgemm_weight *w, int waves_per_group, int k_splits);
 
-/* Override the batch kernel's launch plan (calls with 3 to 16 rows): 8..16 wavefronts per
+/* Override the batch kernel's launch plan (calls with 3 to 16 rows; calls with more then go through the
+ * batch kernel as well, 16 rows per pass): 8..16 wavefronts per
  * workgroup (exactly 8 for weights of more than four planes; fewer than 16 where four scale
  * groups per 128 k leave less LDS) and the k-splits; both 0: back to the automatic choice.
  * LUTGEMM_ERR_BAD_SHAPE if the request cannot be launched.  No launch on the handle may be in

@@ -99,6 +99,7 @@ struct lutgemm_weight {
     // [1], valid when batch_measured[i]; otherwise the model's choice is taken.
     Plan plan_batch[2];
     bool batch_measured[2];
+    bool batch_set;               // they are the caller's (lutgemm_weight_set_batch_plan)
 };
 
 namespace {
@@ -621,10 +622,10 @@ int copy_tiles(lutgemm_weight *w, const void *signs, const void *scales, hipMemc
 
 // Whether the kernel for many rows takes a call.  It contracts with the scales as matrix operand, where an infinite one
 // gives NaN as soon as the signs of its group mix; the batch kernel multiplies it with the group's sum.  And it addresses
-// 64 rows with 32 bits.  Otherwise the batch kernel takes the rows, 16 per pass.
+// 64 rows with 32 bits.  Otherwise, and where the caller has set the batch kernel's plan, that takes the rows, 16 per pass.
 bool takes_rows_kernel(const lutgemm_weight *w, int m)
 {
-    return m > kRowsPerPass && w->shape.k <= kMaxRowsK && w->finite_scales;
+    return m > kRowsPerPass && w->shape.k <= kMaxRowsK && w->finite_scales && !w->batch_set;
 }
 
 // Sets w->finite_scales from the tiles on the device.  The answer comes in a word of set 0, which is back at zero afterwards.
@@ -1211,6 +1212,7 @@ int lutgemm_weight_clone(const lutgemm_weight *w, lutgemm_weight **out)
             (*out)->plan_batch[i] = w->plan_batch[i];
             (*out)->batch_measured[i] = w->batch_measured[i];
         }
+        (*out)->batch_set = w->batch_set;
     }
     return st;
 }
@@ -1602,7 +1604,7 @@ int lutgemm_weight_set_batch_plan(lutgemm_weight *w, int waves_per_group, int k_
     if (!w) return fail(LUTGEMM_ERR_NULL_POINTER, "null argument to weight_set_batch_plan");
     const Shape &s = w->shape;
     if (waves_per_group == 0 && k_splits == 0) {   // back to the model's choice
-        w->batch_measured[0] = w->batch_measured[1] = false;
+        w->batch_measured[0] = w->batch_measured[1] = w->batch_set = false;
         return LUTGEMM_OK;
     }
     const int wmax = lutgemm_kernels::batch_waves_max(s.gsub, s.q, s.qo);
@@ -1615,7 +1617,7 @@ int lutgemm_weight_set_batch_plan(lutgemm_weight *w, int waves_per_group, int k_
     if (batch_plan_cost(s, w->compute_units, waves_per_group, k_splits, 8, &p) < 0.0)
         return fail(LUTGEMM_ERR_BAD_SHAPE, "k_splits=%d leaves a k-split without k-blocks (%d k-blocks)", k_splits, s.ts);
     w->plan_batch[0] = w->plan_batch[1] = p;
-    w->batch_measured[0] = w->batch_measured[1] = true;
+    w->batch_measured[0] = w->batch_measured[1] = w->batch_set = true;
     return LUTGEMM_OK;
 }
 
@@ -1814,6 +1816,7 @@ int lutgemm_weight_autotune(lutgemm_weight *w, void *stream)
         w->plan_batch[bi] = ok ? chosen_batch[bi] : before_batch[bi];
         w->batch_measured[bi] = ok ? true : before_measured[bi];
     }
+    if (status == LUTGEMM_OK && have_batch[1]) w->batch_set = false;   // the caller's plan is replaced
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     if (x) (void)hipFree(x);

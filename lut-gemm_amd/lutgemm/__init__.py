@@ -262,7 +262,7 @@ class BCQWeight:
         _check(load().lutgemm_weight_set_plan(self._h, waves, k_splits))
 
     def set_batch_plan(self, waves=0, k_splits=0):
-        """Launch plan of the batch kernel (3 or more rows); defaults: back to the automatic choice."""
+        """Launch plan of the batch kernel, which then takes all calls of 3 or more rows; defaults: back to the automatic choice."""
         _check(load().lutgemm_weight_set_batch_plan(self._h, waves, k_splits))
 
     def autotune(self, stream=0):

@@ -9,8 +9,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("k,n,q,g,offset", [(512, 40, 3, 128, False), (4096, 70, 2, 64, True), (1024, 1001, 5, 32, False)])
 def test_bias_on_every_kernel(lutgemm, oracle, device, k, n, q, g, offset):
-    """One row, two rows, the batch kernel and the kernel for many rows, with and without splits along k: the result
-    without bias plus the bias in fp16, bit for bit; with weights of zero, the bias."""
+    """One row, two rows, the batch kernel (17 and 40 rows too where its plan is set) and the kernel for many rows, with
+    and without splits along k: the result without bias plus the bias in fp16, bit for bit; with weights of zero, the bias."""
     import torch
     from lutgemm import synth
     w, W = make(lutgemm, synth, k, n, q, g, offset=offset, seed=k + n)
@@ -20,18 +20,20 @@ def test_bias_on_every_kernel(lutgemm, oracle, device, k, n, q, g, offset):
     xd, bd = torch.from_numpy(x).to(device), torch.from_numpy(b).to(device)
     st = torch.cuda.current_stream().cuda_stream
     for m in (1, 2, 3, 16, 17, 40):
-        for splits in (1, min(4, (k + 511) // 512)):
-            say("case bias", k, n, q, "m", m, "splits", splits)
-            W.set_plan(4, splits)
-            W.set_batch_plan(8, splits)
+        for splits in (0, 1, min(4, (k + 511) // 512)):   # 0: the automatic plans
+            say("case bias", k, n, q, "m", m, "splits", splits, W.plan(m))
+            W.set_plan(4 if splits else 0, splits)
+            W.set_batch_plan(8 if splits else 0, splits)
+            if m > 16 and not splits:
+                assert (W.plan(m)["k_splits"] > 1) == (k > 1024)
             y = torch.full((m, n), float("nan"), dtype=torch.float16, device=device)
             W.matvec_bias(xd.data_ptr(), y.data_ptr(), bd.data_ptr(), m, st)
             torch.cuda.synchronize()
             want = torch.full_like(y, float("nan"))
             W.matvec(xd.data_ptr(), want.data_ptr(), m, st)
             assert torch.equal(y.view(torch.int16), (want + bd).view(torch.int16)), m
-            zero.set_plan(4, splits)
-            zero.set_batch_plan(8, splits)
+            zero.set_plan(4 if splits else 0, splits)
+            zero.set_batch_plan(8 if splits else 0, splits)
             zero.matvec_bias(xd.data_ptr(), y.data_ptr(), bd.data_ptr(), m, st)
             assert torch.equal(y, bd.expand(m, n)), m
             # no bias: lutgemm_matvec

@@ -189,3 +189,28 @@ def test_room_for_partial_sums_is_what_the_plan_needs(lutgemm, device):
         assert W.info().device_bytes - before == grown
     assert largest
     W.close()
+
+
+def test_a_batch_plan_that_is_set_holds_for_many_rows(lutgemm, oracle, device):
+    """lutgemm_weight_set_batch_plan acts on calls of more than 16 rows, which take passes of 16 with it, until it is reset
+    or replaced by a measurement; clones have it too."""
+    from lutgemm import synth
+    k, n, q, g, m = 4096, 600, 3, 128, 40
+    w, W = make(lutgemm, synth, k, n, q, g, seed=15)
+    x = synth.make_x(m, k, seed=15)
+    auto, y_auto = W.plan(m), run_matvec(lutgemm, W, x, device)
+    W.set_batch_plan(9, 4)
+    V = W.clone()
+    for handle in (W, V):
+        say("case rows set batch plan", handle.plan(m))
+        assert handle.plan(m) == handle.plan(16) and handle.plan(m)["waves"] == 9 and handle.plan(m)["k_splits"] == 4
+        y = run_matvec(lutgemm, handle, x, device)
+        passes = [run_matvec(lutgemm, handle, x[r:r + 16], device) for r in (0, 16, 32)]
+        assert np.array_equal(y.view(np.uint16), np.concatenate(passes).view(np.uint16))
+        assert_within_tolerance(y, truth_of(oracle, w, x), "passes")
+    W.set_batch_plan()
+    V.autotune()
+    for handle in (W, V):
+        assert handle.plan(m) == auto
+        assert np.array_equal(run_matvec(lutgemm, handle, x, device).view(np.uint16), y_auto.view(np.uint16))
+        handle.close()
