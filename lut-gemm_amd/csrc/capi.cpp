@@ -72,6 +72,7 @@ struct Plan {
 struct StreamSet {
     void *stream;                // the stream the set serves
     unsigned long long *accum;   // kRowsPerPass x (padded outputs) split-k words, zero between launches
+    bool zeroed;                 // they are, for work behind the fill on the stream that first claimed the set
     void *xrows;                 // staging of column-batched activations: xrows_cols rows of k halves,
     int xrows_cols;              //   grown on demand
     float *partials[kRoomSizes]; // room for the sums of launches of more than 16 rows that split k: [c] holds 2^c units,
@@ -383,28 +384,27 @@ int refuse_capture(void *stream, const char *what)
     return fail(LUTGEMM_ERR_UNSUPPORTED, "%s synchronises with the device and cannot run on a stream under graph capture", what);
 }
 
-// Device memory of set i (idempotent).  Allocates: not for a stream that is being captured.
-int alloc_set(lutgemm_weight *w, int i)
+// Device memory of set i (idempotent), its words zeroed on `stream`, which has to be the first to launch on the set: a
+// hipMemset would run on the null stream, with which a stream need not be synchronised, and might come behind the first
+// launches, whose counts it would clear.  Allocates: not for a stream that is being captured.
+int alloc_set(lutgemm_weight *w, int i, void *stream)
 {
     StreamSet &t = w->set[i];
     if (!t.accum) {
-        const size_t bytes = set_words(w) * sizeof(unsigned long long);
-        hipError_t e = hipMalloc((void **)&t.accum, bytes);
+        hipError_t e = hipMalloc((void **)&t.accum, set_words(w) * sizeof(unsigned long long));
         if (e != hipSuccess) return hip_fail(e, "hipMalloc(split-k accumulators)");
-        e = hipMemset(t.accum, 0, bytes);
-        if (e != hipSuccess) return hip_fail(e, "hipMemset(split-k accumulators)");
     }
     if (!t.xrows) {
         hipError_t e = hipMalloc(&t.xrows, (size_t)kStagedColumns * w->shape.k * sizeof(uint16_t));
         if (e != hipSuccess) return hip_fail(e, "hipMalloc(column staging)");
         t.xrows_cols = kStagedColumns;
     }
+    if (!t.zeroed) {
+        hipError_t e = lutgemm_kernels::launch_fill_zero(t.accum, set_words(w), static_cast<hipStream_t>(stream));
+        if (e != hipSuccess) return hip_fail(e, "launch fill_zero_kernel");
+        t.zeroed = true;
+    }
     return LUTGEMM_OK;
-}
-
-int alloc_workspace(lutgemm_weight *w)
-{
-    return alloc_set(w, 0);
 }
 
 // Room for `units` units of partial sums in the set; null where the device has none, and the caller then does not split k.
@@ -469,16 +469,16 @@ int stream_set_once(lutgemm_weight *w, void *stream, int *slot, bool last_attemp
     int take = -1;
     if (w->slots_used < kStreamSlots) {
         take = w->slots_used;
-        if ((!w->set[take].accum || !w->set[take].xrows) && stream_capturing(stream))
+        if (!w->set[take].zeroed && stream_capturing(stream))
             return fail(LUTGEMM_ERR_UNSUPPORTED,
                         "the first launch of a stream on this handle allocates the stream's split-k words, which "
                         "graph capture forbids: launch once on the stream before capturing, or capture "
                         "lutgemm_matvec_static");
-        if (int st = alloc_set(w, take)) return st;
         if (!w->set[take].done) {
             hipError_t e = hipEventCreateWithFlags(&w->set[take].done, hipEventDisableTiming);
             if (e != hipSuccess) return hip_fail(e, "hipEventCreate");
         }
+        if (int st = alloc_set(w, take, stream)) return st;
         w->slots_used++;
     } else {
         // all sets serve a stream: take over the least recently used one whose latest launch is known to
@@ -571,7 +571,7 @@ struct SetLease {
 // have left non-zero; the next call on that device clears them first.
 std::atomic<bool> g_static_dirty[lutgemm_kernels::kMaxDevices];
 
-// New handle for shape s on the current device, its tiles not yet filled in.
+// New handle for shape s on the current device, its tiles not yet filled in (check_scales has to follow when they are).
 int new_handle(const Shape &s, lutgemm_weight **out)
 {
     int count = 0;
@@ -601,7 +601,7 @@ int new_handle(const Shape &s, lutgemm_weight **out)
     if (st == LUTGEMM_OK) {
         w->plan = w->plan2 = choose_plan(s, w->compute_units);
         w->batch_measured[0] = w->batch_measured[1] = false;
-        st = alloc_workspace(w);
+        st = alloc_set(w, 0, nullptr);   // check_scales waits for the null stream before any stream can launch on the handle
     }
     if (st != LUTGEMM_OK) {
         lutgemm_weight_destroy(w);
@@ -628,14 +628,18 @@ bool takes_rows_kernel(const lutgemm_weight *w, int m)
     return m > kRowsPerPass && w->shape.k <= kMaxRowsK && w->finite_scales && !w->batch_set;
 }
 
-// Sets w->finite_scales from the tiles on the device.  The answer comes in a word of set 0, which is back at zero afterwards.
+// Sets w->finite_scales from the tiles on the device.  The answer comes in a word of set 0, which is back at zero
+// afterwards, and everything that the creation of the handle left on the null stream is done.
 int check_scales(lutgemm_weight *w)
 {
     unsigned long long *word = w->set[0].accum, found = 0;
     hipError_t e = lutgemm_kernels::launch_find_non_finite(w->d_scales, scale_bytes(w->shape) / 16, word, nullptr);
     if (e != hipSuccess) return hip_fail(e, "launch find_non_finite_kernel");
     e = hipMemcpy(&found, word, sizeof found, hipMemcpyDeviceToHost);   // behind the kernel
-    if (e == hipSuccess && found) e = hipMemset(word, 0, sizeof found);
+    if (e == hipSuccess && found) {
+        e = lutgemm_kernels::launch_fill_zero(word, 1, nullptr);
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);   // before any stream can launch on the handle
+    }
     if (e != hipSuccess) return hip_fail(e, "reading whether scales are finite");
     w->finite_scales = found == 0;
     return LUTGEMM_OK;
@@ -1642,7 +1646,7 @@ int lutgemm_weight_set_plan(lutgemm_weight *w, int waves_per_group, int k_splits
     hipError_t e = hipDeviceSynchronize();  // no launch may still be using the old workspace
     if (e != hipSuccess) return hip_fail(e, "hipDeviceSynchronize");
     w->plan = w->plan2 = p;
-    return alloc_workspace(w);
+    return LUTGEMM_OK;
 }
 
 int lutgemm_weight_autotune(lutgemm_weight *w, void *stream)

@@ -759,6 +759,36 @@ def test_one_handle_on_two_streams(lutgemm, oracle, device):
     W.close()
 
 
+def test_first_launches_of_a_stream_beside_a_busy_default_stream(lutgemm, oracle, device):
+    """The split-k words of a stream are zeroed on that stream: work that keeps the default stream busy while the first
+    launches run, and ends amid them, changes nothing."""
+    import torch
+    from lutgemm import synth
+    k, n, q, g = 8192, 4096, 3, 128
+    w, W = make(lutgemm, synth, k, n, q, g, seed=21)
+    W.set_plan(8, 8)
+    xd = torch.from_numpy(synth.make_x(1, k, seed=21)).to(device)
+    want = torch.zeros((1, n), dtype=torch.float16, device=device)
+    W.matvec(xd.data_ptr(), want.data_ptr(), 1, torch.cuda.current_stream().cuda_stream)
+    assert_within_tolerance(want.cpu().numpy(), truth_of(oracle, w, xd.cpu().numpy()), "default stream")
+    a = torch.randn(4096, 4096, dtype=torch.float16, device=device)
+    torch.matmul(a, a)
+    out = torch.zeros((200, n), dtype=torch.float16, device=device)
+    torch.cuda.synchronize()
+    for rounds in (1, 4, 12):   # each with a stream of its own
+        say("case first launches beside a busy default stream", rounds)
+        side = torch.cuda.Stream()
+        out.zero_()
+        torch.cuda.synchronize()
+        for _ in range(rounds):
+            torch.matmul(a, a)
+        for y in out:
+            W.matvec(xd.data_ptr(), y.data_ptr(), 1, side.cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want.expand_as(out)), rounds
+    W.close()
+
+
 def test_one_handle_on_many_streams(lutgemm, oracle, device):
     """A handle keeps four stream sets; further streams take over the set used least recently, waiting
     for its launches if they have not completed: seven streams in sequence, then seven streams whose
