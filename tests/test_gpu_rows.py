@@ -1,5 +1,10 @@
 """GPU parity of the kernel for more than 16 activation rows: the edges of its tiles (rows, outputs, k-blocks),
-every plane count with and without an offset, every scale layout, splits along k, both forms of the call."""
+every plane count with and without an offset, every scale layout, splits along k, both forms of the call (plans of two
+row tiles, by their sizes; test_every_instance has them all)."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -214,3 +219,13 @@ def test_a_batch_plan_that_is_set_holds_for_many_rows(lutgemm, oracle, device):
         assert handle.plan(m) == auto
         assert np.array_equal(run_matvec(lutgemm, handle, x, device).view(np.uint16), y_auto.view(np.uint16))
         handle.close()
+
+
+def test_every_instance(lutgemm):
+    """Planes, row tiles, k groups and splits along k that the plans of the sizes above do not reach (rows_test.cpp)."""
+    program = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "rows_test")
+    assert os.path.exists(program), "build the C++ tests first (make -C tests/cpp, or __graft_entry__.build())"
+    r = subprocess.run([program], capture_output=True, text=True, timeout=110)
+    sys.stdout.write(r.stdout)
+    sys.stderr.write(r.stderr)
+    assert r.returncode == 0 and "ROWS OK 288" in r.stdout

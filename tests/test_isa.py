@@ -1,5 +1,5 @@
-"""What the compiler made of the batch kernel, checked on the generated gfx950 assembly of the
-library's own translation unit (no GPU needed: hipcc cross-compiles; about a minute).  The hot
+"""What the compiler made of the batch kernel and of the kernel for many rows, checked on the generated gfx950 assembly of the
+library's own translation units (no GPU needed: hipcc cross-compiles; about a minute).  The hot
 loop and the end of a workgroup depend on properties the source can only ask for: the
 transposition done by the LDS, the matrix instructions present, the index and the scale
 multiply-add in one instruction each, no packed fp32 forms, no register used while an LDS read
@@ -17,15 +17,16 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "lut-gemm_amd", "csrc")
 
 
+ROWS_SOURCES = [("rows.hip", 1), ("rows_two_groups.hip", 2)]   # k groups
 SOURCES = [("batch.hip", "lut_batch_kernel", "10MatvecArgs"), ("batch_multi.hip", "lut_batch_multi_kernel", "15MultiMatvecArgs")]
 
 
 @pytest.fixture(scope="module")
 def assembly(tmp_path_factory):
-    """gfx950 assembly of the two translation units of the batch kernel, compiled side by side."""
+    """gfx950 assembly of the translation units of the two kernels, compiled side by side."""
     out_dir = tmp_path_factory.mktemp("isa")
     jobs = {}
-    for source, _, _ in SOURCES:
+    for source in [s[0] for s in SOURCES + ROWS_SOURCES]:
         out = os.path.join(str(out_dir), source + ".s")
         cmd = ["/opt/rocm/bin/hipcc", "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-Xclang", "-target-feature",
                "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument", "-I", CSRC, "-S", "--cuda-device-only",
@@ -151,3 +152,28 @@ def test_batch_kernel_assembly(assembly, source, kernel, args):
     # the headline instantiation of the decoder-layer chain (two planes, no offset, one group per 128 k): no scratch memory
     body, meta = kernels["ILi2ELb0ELi1ELi16ELb0E"]
     assert re.search(r"\.amdhsa_private_segment_fixed_size 0\b", meta)
+
+
+# register spills of the kernel for many rows (scratch memory per lane, bytes): only with four row tiles (96 registers
+# of sums and activations) and six planes or more
+MAX_ROWS_SCRATCH_BYTES = {(8, 4, 1): 40, (6, 4, 2): 12, (7, 4, 2): 88, (8, 4, 2): 144, (9, 4, 2): 80}
+
+
+@pytest.mark.parametrize("source,groups", ROWS_SOURCES)
+def test_rows_kernel_assembly(assembly, source, groups):
+    text = assembly[source]
+    names = re.findall(r"^(_ZN\S*lut_rows_kernelILi(\d)ELi(\d)ELi(\d)E\S*):", text, re.M)
+    assert sorted((int(p), int(t), int(k)) for _, p, t, k in names) == [(p, t, groups) for p in range(1, 10) for t in (2, 3, 4)]
+    for name, *args in names:
+        planes, row_tiles, _ = instance = tuple(int(v) for v in args)
+        body = text[text.index("\n%s:" % name):]
+        ops = [ln.split()[0] for ln in body[:body.index(".Lfunc_end")].splitlines() if re.match(r"\t[a-z]", ln)]
+        meta = text[text.index(".amdhsa_kernel " + name):]
+        meta = meta[:meta.index(".end_amdhsa_kernel")]
+        # two of its eight wavefronts share a SIMD
+        assert int(re.search(r"\.amdhsa_next_free_vgpr (\d+)", meta).group(1)) <= 256, instance
+        assert ops.count("ds_read_b64_tr_b8") == 4 * planes, instance
+        assert ops.count("v_smfmac_f32_16x16x64_f16") == 32 * planes * row_tiles, instance
+        assert not any(op.startswith(("v_pk_add_f32", "v_pk_mul_f32", "v_pk_fma_f32")) for op in ops), instance
+        scratch = int(re.search(r"\.amdhsa_private_segment_fixed_size (\d+)", meta).group(1))
+        assert scratch <= MAX_ROWS_SCRATCH_BYTES.get(instance, 0), (instance, scratch)
