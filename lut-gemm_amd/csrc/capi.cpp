@@ -323,7 +323,8 @@ size_t partial_units(const Shape &s)
 // throttled to 0.95 us (both from the plans of four shapes, 7168 x 7168 to 12288 x 12288, two to five planes with the
 // offset counted as one, 17 to 256 rows).  A launch has a fixed part, more for every further round of workgroups, and
 // a k-split adds the exchange of the sums: a round trip, a load per partial sum and the traffic of both.  Over those shapes
-// the choice is within 6 % of the fastest measured plan.
+// the choice is within 6 % of the fastest measured plan.  Row tiles that leave no padding cost the same by it; of plans that
+// tie, the first one is taken, with the fewest row tiles.
 RowsPlan choose_rows_plan(const Shape &s, int cus, int m, bool may_split)
 {
     const double kFixed = 8.0, kRound = 4.0, kAlone = 0.65, kThrottled = 0.95, kSplit = 3.0, kSplitEach = 0.3, kPartialBytesPerUs = 4.0e6;

@@ -12,10 +12,12 @@
 //    consecutive k 128 kappa + 32 w, which belong to one scale group whatever its size, so an operand of a lane is one scale
 //    repeated, and one kernel serves every group size.  An offset is one more plane, whose signs are all plus.
 //  * LDS reads of a step run a step ahead (the compiler keeps counted waits), global loads a stage ahead.
-// What bounds it: the matrix unit.  7168 x 7168, 3 planes, 256 rows: 4.8 million matrix instructions in 79 us, 16
-// cycles each busy, 43 % of the cycles, and the rate at which a loop of nothing but this instruction runs with such operands is
-// 24 cycles (65 %); LDS 25 % busy, no bank conflicts.  The launch replaces 16 of the batch kernel: 257 us -> 79 us.
-// 12288 x 12288, 3 planes, 48 rows: 75 -> 53 us; 2048 x 2048, 1 plane, 64 rows: 27 -> 9 us.
+// What bounds it: the matrix unit.  7168 x 7168, 3 planes, 256 rows (RT = 2, KW = 1): 4.8 million matrix instructions in 77
+// us, 16 cycles each busy, 41 % of the cycles, and the rate at which a loop of nothing but this instruction runs with such operands
+// is 24 cycles (62 %); LDS 21 % busy, no bank conflicts.  The launch replaces 16 of the batch kernel: 257 us -> 77 us.
+// 12288 x 12288, 3 planes, 48 rows (RT = 3, KW = 2, two splits): 75 -> 53 us; 2048 x 2048, 1 plane, 64 rows: 27 -> 9 us.
+// Registers: up to 256 (two wavefronts share a SIMD).  With RT = 4 five instances spill: P = 8 with KW = 1 (40 bytes per lane)
+// and P = 6, 7, 8, 9 with KW = 2 (12, 88, 144, 80).
 //
 // A workgroup is eight wavefronts, each with one batch of 32 outputs; KW = 2 makes them two groups of four that share out
 // the k-blocks and add their sums through LDS at the end (more workgroups for a narrow weight, no exchange between them).

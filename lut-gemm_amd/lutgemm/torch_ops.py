@@ -32,7 +32,8 @@ def default_dense_threshold(weight, keep_dense=False):
     eight planes leave the packed route from three rows on (57 against 50 us).
 
     More than 16 rows no longer take passes of 16, so the packed route would stay ahead for longer (12288 x 12288,
-    three planes, 160 rows: 130 against 192 us).  The line is kept all the same, because the routes are not
+    three planes, 160 rows: 130 against 192 us).  The lines are kept all the same (those of layers
+    with a dense copy rest on passes of 16 rows as well), because the routes are not
     interchangeable: the dense one passes gradients to x, follows autocast, can be captured on a stream that has not
     launched on the handle, and rounds the weight to fp16, so its results differ by some 4e-4 of their norm."""
     q = weight.nb
