@@ -98,7 +98,8 @@ int lutgemm_weight_info(const lutgemm_weight *w, lutgemm_weight_info_t *info);
  * a tile with up to 64 of them.  A launch of more than 16 rows that splits k keeps partial sums in memory of the stream's set,
  * allocated when a launch first needs as much (a power of two of bytes, 2 KiB to 16 MiB; mostly 1 to 4 MiB; also under graph
  * capture, so that a captured launch gives the bits of an eager one) and held until the handle is destroyed; where the
- * device has no such memory left, k is not split and a result may differ in the last bit.  Batch results are deterministic and within
+ * device has no such memory left, k is not split on that set from then on (until lutgemm_weight_reset_workspace) and a
+ * result may differ in the last bit.  Batch results are deterministic and within
  * the same tolerance, but a row may differ in the last bit from its own one-row call (another order
  * of the fp32 additions).
  * Launches on one stream run one after the other and share one set of split-k accumulators of the
