@@ -168,23 +168,20 @@ __device__ __forceinline__ void finish_output(float total, bool active, int out,
 // its registers (1 KiB runs), counts itself in once, and the one that comes last adds up all partial sums in the
 // order of their k ranges, so that the result does not depend on who that is; it returns true with the totals in the
 // registers and the count back at zero.
-// The XCDs' L2 caches are not coherent among each other: the stores and loads of the partial sums are device-scope
-// atomics (which go past the L2), and the count is raised only when the stores are acknowledged.
+// The XCDs' L2 caches are not coherent among each other: the stores and loads of the partial sums are device-scope (they
+// go past the L2), and the count is raised only when the stores are acknowledged.  A lane moves 16 bytes at a time: as 8-byte
+// halves of them, which the memory side gets as partial lines, the exchange of 8 MB took 5 us longer (4096 x 16384, three
+// planes, 16 rows, 4 splits: 21.9 us).
 // `partials`: k_splits blocks of N * 256 floats; `of(I)`: register I.
 template <int N, typename F>
 __device__ __forceinline__ bool sum_partials(float *partials, unsigned *count, int ks, int k_splits, int lane, F &&of)
 {
-    typedef unsigned long long u64;
-    u64 *at = reinterpret_cast<u64 *>(partials) + lane * 2;
-    auto pack = [](float a, float b) { return (u64)__builtin_bit_cast(uint32_t, a) | ((u64)__builtin_bit_cast(uint32_t, b) << 32); };
-    {
-        u64 *mine = at + (size_t)ks * (N * 128);
-        static_for<N>([&](auto I) {
-            const auto &v = of(I);
-            __hip_atomic_store(mine + I * 128, pack(v[0], v[1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(mine + I * 128 + 1, pack(v[2], v[3]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        });
-    }
+    typedef float float4v __attribute__((ext_vector_type(4)));
+    constexpr int kDeviceScope = 16;   // sc1: write through, and read past the L2
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)partials, (short)0, -1, 0x00020000);
+    static_for<N>([&](auto I) {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, (float4v)of(I)), rsrc, lane * 16, (ks * N + I) * 1024, kDeviceScope);
+    });
     asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
     unsigned before = 0;
     if (lane == 0) before = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -192,25 +189,19 @@ __device__ __forceinline__ bool sum_partials(float *partials, unsigned *count, i
     if (before != (unsigned)(k_splits - 1)) return false;
     asm volatile("" : : : "memory");
     static_for<N>([&](auto I) { auto &v = of(I); v[0] = v[1] = v[2] = v[3] = 0.f; });
-    constexpr int AHEAD = N <= 4 ? 4 : 2;   // partial sums in flight: a load past the L2 takes a microsecond
+    // Loads past the L2 take a microsecond, so as many partial sums as fit are on their way together; no more than there are,
+    // since they also cost their bytes.
+    constexpr int AHEAD = N <= 2 ? 8 : N <= 4 ? 4 : 2;
     for (int s = 0; s < k_splits; s += AHEAD) {
-        u64 lo[AHEAD][N], hi[AHEAD][N];
-        static_for<AHEAD>([&](auto J) {
-            const u64 *from = at + (size_t)min(s + J, k_splits - 1) * (N * 128);
-            static_for<N>([&](auto I) {
-                lo[J][I] = __hip_atomic_load(from + I * 128, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                hi[J][I] = __hip_atomic_load(from + I * 128 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            });
-        });
+        u32x4 part[AHEAD][N];
         static_for<AHEAD>([&](auto J) {
             if (s + J < k_splits)   // uniform
                 static_for<N>([&](auto I) {
-                    auto &v = of(I);
-                    v[0] += __builtin_bit_cast(float, (uint32_t)lo[J][I]);
-                    v[1] += __builtin_bit_cast(float, (uint32_t)(lo[J][I] >> 32));
-                    v[2] += __builtin_bit_cast(float, (uint32_t)hi[J][I]);
-                    v[3] += __builtin_bit_cast(float, (uint32_t)(hi[J][I] >> 32));
+                    part[J][I] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane * 16, ((s + J) * N + I) * 1024, kDeviceScope));
                 });
+        });
+        static_for<AHEAD>([&](auto J) {
+            if (s + J < k_splits) static_for<N>([&](auto I) { of(I) += __builtin_bit_cast(float4v, part[J][I]); });
         });
     }
     if (lane == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
