@@ -101,6 +101,8 @@ struct lutgemm_weight {
     Plan plan_batch[2];
     bool batch_measured[2];
     bool batch_set;               // they are the caller's (lutgemm_weight_set_batch_plan)
+    // The kernel for few rows (3 to 16, where takes_few_kernel): plans for up to 8 rows and for 9 to 16
+    Plan plan_few[2];
 };
 
 namespace {
@@ -248,6 +250,60 @@ Plan choose_batch_plan(const Shape &s, int cus, int rows)
     return best;
 }
 
+// Sums that split k through memory come in units of 16 rows x 32 outputs (2 KiB).  A launch of more than 16 rows splits k to
+// fill the device, so some 256 workgroups of 8 batches x 4 row tiles bound what it needs: 16 MiB, less for narrow weights.
+constexpr size_t kPartialUnits = 8192, kPartialUnitBytes = 2048;
+static_assert(kPartialUnits * kPartialUnitBytes == lutgemm_kernels::kStaticPartials * sizeof(float), "both entry points take the same plans");
+static_assert(kPartialUnits == (size_t)1 << (kRoomSizes - 1), "the largest plan's room is the largest there is");
+
+// What a k-split of the kernel for few rows (few_body.h) adds, in microseconds: an atomic per value, or partial sums through
+// memory, a round trip each for stores, count and loads and the traffic of all rows of the batch.  The atomics win where there
+// are few values (512 outputs, 8 rows, 16 splits: 8.7 against 9.4 us for the launch), memory where there are many (12288
+// outputs, 8 rows, 5 splits: 15.6 against 18.6).
+double few_atomics_cost(const Shape &s, int rows, int ks) { return 2.34 + 5.07e-6 * (double)s.n * rows * ks; }
+double few_partials_cost(const Shape &s, int rows, int ks)
+{
+    return (size_t)s.nb * ks > kPartialUnits ? 1e30 : 0.79 + 0.143 * ks + (double)s.nb * ks * rows * (2 * kBatch * sizeof(float)) / 2.7e6;
+}
+bool few_takes_atomics(const Shape &s, int rows, int ks) { return few_atomics_cost(s, rows, ks) < few_partials_cost(s, rows, ks); }
+
+// Launch plan of the kernel for few rows: wavefronts per workgroup and k-splits.  Cost model in microseconds (-1 when `ks` names
+// the same plan as a smaller number of k-splits): a round of one workgroup per compute unit works through its tiles (at most
+// one round trip to memory per k-block faster) while the weight streams, and the two get in each other's way as the root
+// of their squares.  Fitted to 9,500 measured launches over 18 shapes (k 768 to 49152, n 32 to 49152, one to eight planes, 3 to
+// 16 rows; rms error 4 %); the plan it names is 0.8 % slower than the fastest on average, 19 % at worst.
+double few_plan_cost(const Shape &s, int cus, int waves, int ks, int rows, Plan *out)
+{
+    const double base = 3.493, round_us = 1.5, tile_us = 0.0745, two_rows = 1.1212, block_us = 0.169, block_floor = 0.6, bytes_per_us = 7.135e6;
+    const int ntiles = div_up(s.nb, waves), bps = div_up(s.ts, ks);
+    if (div_up(s.ts, bps) != ks) return -1.0;
+    *out = Plan{waves, ntiles, bps, ks};
+    const double rounds = (double)(((long)ntiles * ks + cus - 1) / cus);
+    double block = waves * s.qo * tile_us * (rows > 8 ? two_rows : 1.0) + block_us;
+    if (block < block_floor) block = block_floor;
+    const double work = rounds * bps * block, stream = (double)(sign_bytes(s) + scale_bytes(s)) / bytes_per_us;
+    double cost = base + rounds * round_us + std::sqrt(work * work + stream * stream);
+    if (ks > 1) cost += few_takes_atomics(s, rows, ks) ? few_atomics_cost(s, rows, ks) : few_partials_cost(s, rows, ks);
+    return cost;
+}
+
+// `rows`: 8 for calls of up to 8 rows, 16 for larger ones (the two plans a handle keeps)
+Plan choose_few_plan(const Shape &s, int cus, int rows)
+{
+    Plan best{lutgemm_kernels::kFewWavesMin, div_up(s.nb, lutgemm_kernels::kFewWavesMin), s.ts, 1};
+    double best_cost = 1e30;
+    for (int waves = lutgemm_kernels::kFewWavesMin; waves <= lutgemm_kernels::few_waves_max(s.qo); waves++)
+        for (int ks = 1; ks <= s.ts && ks <= kMaxSplits; ks++) {
+            Plan p;
+            const double cost = few_plan_cost(s, cus, waves, ks, rows, &p);
+            if (cost >= 0.0 && cost < best_cost) {
+                best_cost = cost;
+                best = p;
+            }
+        }
+    return best;
+}
+
 static_assert(lutgemm_kernels::kBatchMaxPlanes == 8, "the batch kernel takes every plane count a weight can have");
 
 // Launch shape of several independent batches in one grid (lutgemm_matvec_many): one number of
@@ -306,11 +362,6 @@ struct RowsPlan {
     size_t units(const Shape &s) const { return (size_t)s.nb * row_chunks * row_tiles * k_splits; }   // of partial sums
 };
 
-// Sums that split k through memory come in units of 16 rows x 32 outputs (2 KiB).  A launch splits k to fill the
-// device, so some 256 workgroups of 8 batches x 4 row tiles bound what it needs: 16 MiB, less for narrow weights.
-constexpr size_t kPartialUnits = 8192, kPartialUnitBytes = 2048;
-static_assert(kPartialUnits * kPartialUnitBytes == lutgemm_kernels::kStaticPartials * sizeof(float), "both entry points take the same plans");
-static_assert(kPartialUnits == (size_t)1 << (kRoomSizes - 1), "the largest plan's room is the largest there is");
 constexpr int kMaxRowsSplits = 32, kMaxSplitChunks = 16;
 size_t partial_units(const Shape &s)
 {
@@ -354,6 +405,9 @@ RowsPlan choose_rows_plan(const Shape &s, int cus, int m, bool may_split)
     }
     return best;
 }
+
+// Shapes that the kernel for few rows takes: one scale group per row of a tile, and rows that 32 bits address.
+bool few_shape(const Shape &s) { return s.gsub == 1 && s.k <= kMaxRowsK; }
 
 // A handle's device memory belongs to the device that was current when it was created.
 int check_device(const lutgemm_weight *w)
@@ -602,6 +656,8 @@ int new_handle(const Shape &s, lutgemm_weight **out)
     if (st == LUTGEMM_OK) {
         w->plan = w->plan2 = choose_plan(s, w->compute_units);
         w->batch_measured[0] = w->batch_measured[1] = false;
+        if (few_shape(s))
+            for (int i = 0; i < 2; i++) w->plan_few[i] = choose_few_plan(s, w->compute_units, i ? kRowsPerPass : 8);
         st = alloc_set(w, 0, nullptr);   // check_scales waits for the null stream before any stream can launch on the handle
     }
     if (st != LUTGEMM_OK) {
@@ -627,6 +683,14 @@ int copy_tiles(lutgemm_weight *w, const void *signs, const void *scales, hipMemc
 bool takes_rows_kernel(const lutgemm_weight *w, int m)
 {
     return m > kRowsPerPass && w->shape.k <= kMaxRowsK && w->finite_scales && !w->batch_set;
+}
+
+// The same for the kernel for few rows, which also contracts with the scales as matrix operand.  It is the faster one of the two
+// on every shape measured (0.72 to 1.0 of the batch kernel's time, 0.79 on average); that keeps weights with finer scale groups,
+// with non-finite scales, and calls for which the caller has set its plan.
+bool takes_few_kernel(const lutgemm_weight *w, int m)
+{
+    return m >= 3 && m <= kRowsPerPass && few_shape(w->shape) && w->finite_scales && !w->batch_measured[m > 8];
 }
 
 // Sets w->finite_scales from the tiles on the device.  The answer comes in a word of set 0, which is back at zero
@@ -915,7 +979,11 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
         lease.stream = stream;
         a.accum = mw->set[slot].accum;
     }
-    if (cols && m > 1) {
+    // few rows (few_body.h); workgroups of kFewWavesMin wavefronts read columns as they are
+    const bool few = takes_few_kernel(w, m);
+    const Plan few_plan = few ? w->plan_few[m > 8] : Plan{};
+    const bool few_columns = few && cols && few_plan.waves == lutgemm_kernels::kFewWavesMin;
+    if (cols && m > 1 && !few_columns) {
         // gather the m columns into contiguous rows first (the kernel reads 16 bytes per lane); the
         // staging rows belong to the stream's set, or, for the allocation-free entry point, to set 0
         StreamSet &t = mw->set[slot];
@@ -943,12 +1011,32 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
     }
     a.x_row_stride = s.k;
     a.accum_row_stride = (long long)s.nb * kBatch;
-    // The kernels of 2 to 16 rows take no bias (add_bias in tile_device.h): a small kernel follows their launches.
+    // The two-row and batch kernels take no bias (add_bias in tile_device.h): a small kernel follows their launches.
     auto add_bias_behind = [&]() -> int {
         if (!bias || m == 1) return LUTGEMM_OK;
         const hipError_t e = lutgemm_kernels::launch_add_bias(y, bias, m, s.n, st);
         return e == hipSuccess ? LUTGEMM_OK : hip_fail(e, "launch add_bias_kernel");
     };
+    if (few) {
+        lutgemm_kernels::FewGrid g{};
+        a.ntiles = few_plan.ntiles;
+        a.k_splits = few_plan.k_splits;
+        a.blocks_per_split = few_plan.blocks_per_split;
+        a.rows = m;
+        a.x = xh;
+        a.y = yh;
+        a.y_stride = cols ? m : 1;   // y [n][m] or [m][n]
+        a.y_row_stride = cols ? 1 : s.n;
+        if (a.k_splits > 1 && !few_takes_atomics(s, m, a.k_splits))   // without room for partial sums atomics it is
+            g.partials = static_ws ? static_partials : partials_of(mw, slot, (size_t)s.nb * a.k_splits);
+        g.bias = bias;
+        g.columns = few_columns;
+        g.wide_y = !cols && s.n % 4 == 0 && ((uintptr_t)y & 7u) == 0;
+        hipError_t e = lutgemm_kernels::launch_few(s.q, s.has_offset, a, g, few_plan.waves, st);
+        if (e != hipSuccess) return hip_fail(e, "launch lut_few_kernel");
+        lease.launched = true;
+        return LUTGEMM_OK;
+    }
     // more rows than a pass of the batch kernel takes: one launch over all of them
     if (takes_rows_kernel(w, m)) {
         lutgemm_kernels::RowsGrid g{};
@@ -1218,6 +1306,7 @@ int lutgemm_weight_clone(const lutgemm_weight *w, lutgemm_weight **out)
             (*out)->batch_measured[i] = w->batch_measured[i];
         }
         (*out)->batch_set = w->batch_set;
+        for (int i = 0; i < 2; i++) (*out)->plan_few[i] = w->plan_few[i];
     }
     return st;
 }
@@ -1589,7 +1678,9 @@ int lutgemm_weight_plan_for(const lutgemm_weight *w, int m, int *workgroups, int
     if (m < 1 || m > LUTGEMM_MAX_BATCH)
         return fail(LUTGEMM_ERR_BAD_SHAPE, "m=%d outside 1..%d", m, LUTGEMM_MAX_BATCH);
     Plan p = m == 1 ? w->plan : w->plan2;
-    if (takes_rows_kernel(w, m)) {
+    if (takes_few_kernel(w, m)) {
+        p = w->plan_few[m > 8];
+    } else if (takes_rows_kernel(w, m)) {
         const RowsPlan r = choose_rows_plan(w->shape, w->compute_units, m, true);
         p = Plan{lutgemm_kernels::kRowsWaves, r.ntiles * r.row_chunks, r.blocks_per_split, r.k_splits};
     } else if (m >= 3) {
@@ -1705,15 +1796,17 @@ int lutgemm_weight_autotune(lutgemm_weight *w, void *stream)
     if (e == hipSuccess) e = hipEventCreate(&e1);
     if (e != hipSuccess) status = hip_fail(e, "autotune setup");
     const Plan before = w->plan, before2 = w->plan2;
-    const Plan before_batch[2] = {w->plan_batch[0], w->plan_batch[1]};
+    // weights that the kernel for few rows takes have its plans measured, the others the batch kernel's
+    const bool few = few_shape(s) && w->finite_scales;
+    const Plan before_batch[2] = {(few ? w->plan_few : w->plan_batch)[0], (few ? w->plan_few : w->plan_batch)[1]};
     const bool before_measured[2] = {w->batch_measured[0], w->batch_measured[1]};
     size_t turn = 0;
     // time `reps` launches over `rows` activation rows with plan p, rotating over the copies
     auto measure = [&](const Plan &p, int rows, int reps, float *ms_out) -> int {
         for (lutgemm_weight *c : copies) {
             if (rows > kTableRows) {
-                c->plan_batch[rows > 8] = p;
-                c->batch_measured[rows > 8] = true;
+                (few ? c->plan_few : c->plan_batch)[rows > 8] = p;
+                c->batch_measured[rows > 8] = !few;
             } else {
                 (rows == 2 ? c->plan2 : c->plan) = p;
             }
@@ -1779,18 +1872,20 @@ int lutgemm_weight_autotune(lutgemm_weight *w, void *stream)
                 }
             }
     }
-    // The batch kernel, for passes of up to 8 rows and of 9..16 rows: the model's ten best plans,
-    // measured the same way.
+    // Batches of up to 8 rows and of 9..16 rows: the model's ten best plans of their kernel, measured the same way.
     Plan chosen_batch[2] = {before_batch[0], before_batch[1]};
     bool have_batch[2] = {false, false};
     for (int bi = 0; bi < 2; bi++) {
         const int rows = bi ? kRowsPerPass : 8;
         struct Timed { float ms; double cost; Plan p; };
         std::vector<Timed> timed;
-        for (int waves = lutgemm_kernels::kBatchWavesMin; waves <= lutgemm_kernels::batch_waves_max(s.gsub, s.q, s.qo); waves++)
+        const int wmin = few ? lutgemm_kernels::kFewWavesMin : lutgemm_kernels::kBatchWavesMin;
+        const int wmax = few ? lutgemm_kernels::few_waves_max(s.qo) : lutgemm_kernels::batch_waves_max(s.gsub, s.q, s.qo);
+        for (int waves = wmin; waves <= wmax; waves++)
             for (int ks = 1; ks <= s.ts && ks <= kMaxSplits; ks++) {
                 Plan p;
-                const double cost = batch_plan_cost(s, w->compute_units, waves, ks, rows, &p);
+                const double cost = few ? few_plan_cost(s, w->compute_units, waves, ks, rows, &p)
+                                        : batch_plan_cost(s, w->compute_units, waves, ks, rows, &p);
                 if (cost >= 0.0) timed.push_back(Timed{1e30f, cost, p});
             }
         std::sort(timed.begin(), timed.end(), [](const Timed &a, const Timed &b) { return a.cost < b.cost; });
@@ -1818,8 +1913,8 @@ int lutgemm_weight_autotune(lutgemm_weight *w, void *stream)
     w->plan2 = status == LUTGEMM_OK ? chosen[1] : before2;
     for (int bi = 0; bi < 2; bi++) {
         const bool ok = status == LUTGEMM_OK && have_batch[bi];
-        w->plan_batch[bi] = ok ? chosen_batch[bi] : before_batch[bi];
-        w->batch_measured[bi] = ok ? true : before_measured[bi];
+        (few ? w->plan_few : w->plan_batch)[bi] = ok ? chosen_batch[bi] : before_batch[bi];
+        w->batch_measured[bi] = ok ? !few : before_measured[bi];
     }
     if (status == LUTGEMM_OK && have_batch[1]) w->batch_set = false;   // the caller's plan is replaced
     if (e0) (void)hipEventDestroy(e0);

@@ -1,0 +1,13 @@
+// The kernel for 3 to 16 activation rows (few_body.h): activations as rows, at most one per wavefront, and the dispatch.
+#include "few_body.h"
+
+namespace lutgemm_kernels {
+
+hipError_t launch_few(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t s)
+{
+    if (a.rows < 1 || a.rows > kBatchRows || waves < kFewWavesMin || waves > few_waves_max(q + (has_offset ? 1 : 0))) return hipErrorInvalidValue;
+    if (g.columns) return waves == kFewWavesMin ? launch_few_columns(q, has_offset, a, g, s) : hipErrorInvalidValue;
+    return a.rows <= waves ? launch_few_input<FewInput::kOneRow>(q, has_offset, a, g, waves, s) : launch_few_two_rows(q, has_offset, a, g, waves, s);
+}
+
+}  // namespace lutgemm_kernels

@@ -1,0 +1,11 @@
+// The kernel for 3 to 16 activation rows (few_body.h): instances that read activations stored as columns.
+#include "few_body.h"
+
+namespace lutgemm_kernels {
+
+hipError_t launch_few_columns(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, hipStream_t s)
+{
+    return launch_few_input<FewInput::kColumns>(q, has_offset, a, g, kFewWavesMin, s);
+}
+
+}  // namespace lutgemm_kernels
