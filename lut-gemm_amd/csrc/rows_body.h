@@ -12,12 +12,16 @@
 //    consecutive k 128 kappa + 32 w, which belong to one scale group whatever its size, so an operand of a lane is one scale
 //    repeated, and one kernel serves every group size.  An offset is one more plane, whose signs are all plus.
 //  * LDS reads of a step run a step ahead (the compiler keeps counted waits), global loads a stage ahead.
-// What bounds it: the matrix unit.  7168 x 7168, 3 planes, 256 rows (RT = 2, KW = 1): 4.8 million matrix instructions in 77
-// us, 16 cycles each busy, 41 % of the cycles, and the rate at which a loop of nothing but this instruction runs with such operands
-// is 24 cycles (62 %); LDS 21 % busy, no bank conflicts.  The launch replaces 16 of the batch kernel: 257 us -> 77 us.
-// 12288 x 12288, 3 planes, 48 rows (RT = 3, KW = 2, two splits): 75 -> 53 us; 2048 x 2048, 1 plane, 64 rows: 27 -> 9 us.
-// Registers: up to 256 (two wavefronts share a SIMD).  With RT = 4 five instances spill: P = 8 with KW = 1 (40 bytes per lane)
-// and P = 6, 7, 8, 9 with KW = 2 (12, 88, 144, 80).
+//  * A matrix instruction holds the vector unit of its SIMD for 16 cycles and takes one other vector instruction for nothing,
+//    every further one in 4 cycles (few_body.h), so indices and activations are made one instruction behind each matrix
+//    instruction, and addresses are scalar (buffer loads).
+// What bounds it: power.  7168 x 7168, 3 planes, 256 rows (RT = 2, KW = 1): 4.8 million matrix instructions in 77 us; a loop of
+// nothing but them with such operands takes 50 us on the whole device (10.7 ns each and SIMD, 6.9 on a few compute units), and
+// the compute units that the plan leaves idle, start and end the rest.  Before the instructions were spread: 82 to 89 us; 12288 x
+// 12288, 3 planes, 48 rows (RT = 3, five splits): 58 -> 49 us.  The launch replaced 16 of the batch kernel: 257 us.
+// Tried: a staging area for each sign vector, written a pass ahead and read when the words before are done with, so that no
+// transposition is waited for: no faster.
+// Registers: up to 256 (two wavefronts share a SIMD).  One instance spills: P = 8, RT = 4, KW = 2 (36 bytes per lane).
 //
 // A workgroup is eight wavefronts, each with one batch of 32 outputs; KW = 2 makes them two groups of four that share out
 // the k-blocks and add their sums through LDS at the end (more workgroups for a narrow weight, no exchange between them).
@@ -52,12 +56,6 @@ typedef __attribute__((address_space(3))) v2i lds_v2i;
 
 constexpr int kStageBytes = 1024;   // per wavefront: one sign vector of a tile
 
-// word (x[2i], x[2i+1]) -> (-x[2i], +x[2i]) (selector 0x01000100) or (-x[2i+1], +x[2i+1]) (0x03020302)
-__device__ __forceinline__ uint32_t minus_plus(uint32_t pair, uint32_t selector)
-{
-    return __builtin_amdgcn_perm(pair, pair, selector) ^ 0x00008000u;
-}
-
 // P planes (an offset counts as one whose signs are all plus), RT row tiles of 16 activation rows per workgroup,
 // KW groups of wavefronts that take every KW-th k-block.
 template <int P, int RT, int KW>
@@ -73,6 +71,7 @@ __global__ __launch_bounds__(kRowsWaves * 64) void lut_rows_kernel(MatvecArgs a,
     constexpr int PIECES = (16 * RT + ROWS - 1) / ROWS;     // 16-byte pieces of a stage per thread
     constexpr int GROUP = rows_staged(RT, KW) * PITCH;      // bytes of a lane group's share of a stage
     constexpr int XBUF = 4 * GROUP;
+    constexpr bool SPREAD = PIECES < 4;   // activations are converted between the matrix instructions (four pieces: registers)
     static_assert(GROUP % 256 == 0, "no shift of the banks from group to group");
     static_assert(PIECES * ROWS == rows_staged(RT, KW), "kernels.h states the LDS of this kernel");
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_generic[];
@@ -94,9 +93,8 @@ __global__ __launch_bounds__(kRowsWaves * 64) void lut_rows_kernel(MatvecArgs a,
     const int ts0 = ks * a.blocks_per_split, ts1 = min(ts0 + a.blocks_per_split, a.ts);
     const int iterations = (ts1 - ts0 + KW - 1) / KW;
 
-    const u32x4 *signs = reinterpret_cast<const u32x4 *>(a.signs);
-    const __half *x = reinterpret_cast<const __half *>(a.x);
     const size_t tile0 = (size_t)(active ? nb : 0) * a.ts;
+    constexpr int kBufferFlags = 0x00020000;   // 32-bit elements, offsets in bytes
 
     lds_byte *xbuf = lds + (size_t)kw * 2 * XBUF;
     lds_byte *stage = lds + (size_t)KW * 2 * XBUF + wave * kStageBytes;
@@ -108,12 +106,14 @@ __global__ __launch_bounds__(kRowsWaves * 64) void lut_rows_kernel(MatvecArgs a,
     lds_v2i *stage_r0 = reinterpret_cast<lds_v2i *>(stage + (r_off ^ ((kappa & 1) * 128)));
     lds_v2i *stage_r1 = reinterpret_cast<lds_v2i *>(stage + ((r_off + 128) ^ ((kappa & 1) * 128)));
 
-    // scales of output j (both halves) for the group of word w
+    // scales of output j (both halves) for the group of word w, in bytes
     const int subl = 16 / g.gsub, lh = 2 * g.gsub * P;
-    const int sc_lane = (kappa * 16 + j % subl) * lh + (j / subl) * P, sc_sub = subl * lh, sc_h = g.gsub * P;
+    const int sc_lane = 2 * ((kappa * 16 + j % subl) * lh + (j / subl) * P), sc_sub = 2 * subl * lh, sc_h = 2 * g.gsub * P;
+    const bool one_group = g.gsub == 1;   // of a lane in a tile: the four words have the same scales
 
     // Activation pieces (16 bytes: one chunk of one row) of this thread.  Rows beyond the batch read its last row: a row
-    // is a column of the matrix product, and theirs are never stored.  A wavefront moves, per piece, the 16 chunks of one
+    // is a column of the matrix product, and theirs are never stored; k beyond the weight reads zero (an offset beyond the
+    // buffer).  A wavefront moves, per piece, the 16 chunks of one
     // word w in four rows: lane bits 0-1 the byte of the word, 2-3 the row, 4-5 the lane group kappa of the chunk.
     // In LDS a stage is [B lane group kb][row][w][step][half of the B operand], 16 bytes each: chunk (kappa, byte) is
     // in half kappa / 2 of lane group 2 (kappa % 2) + byte % 2, for the steps of byte / 2.  The rows' pitch shifts their
@@ -124,10 +124,12 @@ __global__ __launch_bounds__(kRowsWaves * 64) void lut_rows_kernel(MatvecArgs a,
     const int piece_w = nw % WS, piece_row = 16 * (nw / (4 * WS)) + 2 * ((nw / WS) & 3) + ((lane >> 2) & 1) + (lane & 8);
     const int piece_k = (16 * c_kappa + 4 * piece_w + c_byte) * kChunk;
     auto piece_row_step = [](int i) constexpr { return 16 * (i * NW / (4 * WS)) + 2 * ((i * NW / WS) & 3); };
-    const __half *x_chunk = x + (size_t)row0 * (size_t)a.x_row_stride;
-    uint32_t piece_off[PIECES];
+    const auto x_rsrc = __builtin_amdgcn_make_buffer_rsrc(   // of this workgroup's rows: at most 64 of 2^24 halves, 2^31 bytes
+        (void *)(reinterpret_cast<const __half *>(a.x) + (size_t)row0 * (size_t)a.x_row_stride), (short)0,
+        (int)((uint32_t)min(a.rows - row0, 16 * RT) * (uint32_t)a.x_row_stride * 2u), kBufferFlags);
+    uint32_t piece_off[PIECES];   // of the row, in bytes
     static_for<PIECES>([&](auto I) {
-        piece_off[I] = (uint32_t)min(piece_row + piece_row_step(I), a.rows - 1 - row0) * (uint32_t)a.x_row_stride;
+        piece_off[I] = (uint32_t)min(piece_row + piece_row_step(I), a.rows - 1 - row0) * (uint32_t)a.x_row_stride * 2u;
     });
     const int first = c_byte & 1;
     const uint32_t sel_a = first ? 0x03020302u : 0x01000100u, sel_b = first ? 0x01000100u : 0x03020302u;
@@ -135,25 +137,28 @@ __global__ __launch_bounds__(kRowsWaves * 64) void lut_rows_kernel(MatvecArgs a,
                          (c_kappa >> 1) * 16 + 32 * first;
     const int to_other = 32 - 64 * first;
     u32x4 piece[PIECES];
-    uint32_t piece_mask;
-    // words w0 .. w0 + WS - 1 of k-block kb; k beyond the weight becomes zero when stored
+    // words w0 .. w0 + WS - 1 of k-block kb
     auto load_pieces = [&](int kb, int w0) {
         const int kpos = kb * kBlockK + 32 * w0 + piece_k, limit = kb < ts1 ? a.k : 0;
-        piece_mask = kpos < limit ? 0xffffffffu : 0u;
+        const uint32_t at = (uint32_t)kpos * 2u, beyond = kpos < limit ? 0u : 0xffffff00u;
         static_for<PIECES>([&](auto I) {
-            piece[I] = *reinterpret_cast<const u32x4 *>(x_chunk + (piece_off[I] + ((uint32_t)kpos & piece_mask)));
+            piece[I] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, (int)((piece_off[I] + at) | beyond), 0, 0));
         });
     };
+    // A piece becomes a 16-byte block of each parity of k, [-x, +x] x 4: instruction N of 16 for piece I (with a write behind the
+    // eighth and the last)
+    constexpr int PIECE_OPS = 16;
+    uint32_t block[PIECES][4];
+    auto piece_op = [&](auto I, auto N, int buf) {
+        constexpr int second = N / 8, d = (N % 8) / 2;
+        if constexpr (N % 2 == 0) block[I][d] = __builtin_amdgcn_perm(piece[I][d], piece[I][d], second ? sel_b : sel_a);
+        else block[I][d] ^= 0x00008000u;
+        if constexpr (N % 8 == 7)
+            *reinterpret_cast<lds_u32x4 *>(piece_at + buf * XBUF + piece_row_step(I) * PITCH + (second ? to_other : 0)) =
+                u32x4{block[I][0], block[I][1], block[I][2], block[I][3]};
+    };
     auto store_pieces = [&](int buf) {
-        static_for<PIECES>([&](auto I) {
-            lds_byte *at = piece_at + buf * XBUF + piece_row_step(I) * PITCH;
-            const uint32_t m = piece_mask;
-            const u32x4 v = u32x4{piece[I].x & m, piece[I].y & m, piece[I].z & m, piece[I].w & m};
-            *reinterpret_cast<lds_u32x4 *>(at) =
-                u32x4{minus_plus(v.x, sel_a), minus_plus(v.y, sel_a), minus_plus(v.z, sel_a), minus_plus(v.w, sel_a)};
-            *reinterpret_cast<lds_u32x4 *>(at + to_other) =
-                u32x4{minus_plus(v.x, sel_b), minus_plus(v.y, sel_b), minus_plus(v.z, sel_b), minus_plus(v.w, sel_b)};
-        });
+        static_for<PIECES * PIECE_OPS>([&](auto N) { piece_op(std::integral_constant<int, N / PIECE_OPS>{}, std::integral_constant<int, N % PIECE_OPS>{}, buf); });
     };
 
     float4v acc[2][RT];
@@ -167,48 +172,61 @@ __global__ __launch_bounds__(kRowsWaves * 64) void lut_rows_kernel(MatvecArgs a,
     asm("" : "+s"(mask55));
     asm("" : "+v"(high88));
 
-    auto tile_of = [&](int it) {   // tile of this wavefront's iteration `it`, a valid one past the end
+    auto block_of = [&](int it) {   // k-block of this wavefront's iteration `it`, a valid one past the end
         const int kb = ts0 + it * KW + kw;
-        return tile0 + (size_t)(kb < ts1 ? kb : ts0);
+        return kb < ts1 ? kb : ts0;
     };
+    const auto sign_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(a.signs + tile0 * (size_t)(2 * g.q * kUnitBytes)), (short)0, -1, kBufferFlags);
+    const auto scale_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(a.scales + tile0 * (size_t)(kLanes * lh)), (short)0, -1, kBufferFlags);
     u32x4 sign[NU];
-    auto load_signs = [&](size_t tile, auto Pc) {
-        const u32x4 *base = signs + tile * (size_t)(2 * g.q * kLanes) + lane;
+    auto load_signs = [&](int kb, auto Pc) {
         static_for<NU>([&](auto U) {
             constexpr int unit = Pc * NU + U;
-            if constexpr (unit < 2 * P) sign[U] = __builtin_nontemporal_load(base + (unit < 2 * g.q ? unit : 0) * kLanes);
+            if constexpr (unit < 2 * P)
+                sign[U] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(sign_rsrc, lane * 16, (kb * 2 * g.q + (unit < 2 * g.q ? unit : 0)) * kUnitBytes, 2));
         });
     };
-    uint32_t scale[NU];   // raw scales of the next word's units
-    auto load_scales = [&](size_t tile, int w, auto Pc) {
-        const uint16_t *sp = a.scales + tile * (size_t)(kLanes * lh) + sc_lane + (w * g.gsub / 4) * sc_sub;
+    uint32_t scale[NU];   // raw scales of the units whose operands are made next
+    auto load_scales = [&](int kb, int w, auto Pc) {
+        const int at = kb * (2 * kLanes * lh) + (w * g.gsub / 4) * sc_sub;
         static_for<NU>([&](auto U) {
             constexpr int b = Pc * QP + U / 2, h = U % 2;
-            if constexpr (b < P) scale[U] = sp[h * sc_h + b];
+            if constexpr (b < P) scale[U] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(scale_rsrc, sc_lane, at + h * sc_h + 2 * b, 0);
+        });
+    };
+    half8 A[NU];
+    auto make_operands = [&](uint32_t vmask, auto Pc) {
+        static_for<NU>([&](auto U) {
+            if constexpr (Pc * QP + U / 2 < P) {
+                const uint32_t s = scale[U] * vmask;
+                A[U] = __builtin_bit_cast(half8, u32x4{s, s, s, s});
+            }
         });
     };
     // signs of the last plane when that is the offset
     const uint32_t all_plus = g.q < P ? 0xffffffffu : 0u;
 
     load_pieces(ts0 + kw, 0);
-    load_signs(tile_of(0), std::integral_constant<int, 0>{});
-    load_scales(tile_of(0), 0, std::integral_constant<int, 0>{});
+    load_signs(block_of(0), std::integral_constant<int, 0>{});
+    load_scales(block_of(0), 0, std::integral_constant<int, 0>{});
     store_pieces(0);
     __syncthreads();
 
     int buf = 0;
     for (int it = 0; it < iterations; it++) {
         const int kb = ts0 + it * KW + kw;
-        const bool valid = kb < ts1;
-        const size_t tile = tile_of(it), next_tile = tile_of(it + 1);
-        const uint32_t vmask = valid ? 0x10001u : 0u;
+        const int cur = block_of(it), next = block_of(it + 1);
+        const uint32_t vmask = kb < ts1 ? 0x10001u : 0u;
         static_for<PG>([&](auto Pc) {
-            constexpr int pg = Pc;
+            constexpr int pg = Pc, b0 = pg * QP;
+            constexpr int ACTIVE = 2 * (P - b0 < QP ? P - b0 : QP);   // units of this pass
             constexpr bool last_pass = pg + 1 == PG;
+            constexpr int pg_next = (pg + 1) % PG;
+            make_operands(vmask, Pc);
             // this pass's sign bits of output j, refill of the registers behind it
             u32x4 R[NU];
             static_for<NU>([&](auto U) {
-                constexpr int b = pg * QP + U / 2;
+                constexpr int b = b0 + U / 2;
                 if constexpr (b < P) {
                     *stage_w = sign[U];
                     const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32(stage_r0);
@@ -222,7 +240,12 @@ __global__ __launch_bounds__(kRowsWaves * 64) void lut_rows_kernel(MatvecArgs a,
                     }
                 }
             });
-            load_signs(last_pass ? next_tile : tile, std::integral_constant<int, (pg + 1) % PG>{});
+            // Index registers.  With two row tiles those of the next pair of steps are made while one is contracted; with more,
+            // those of the next unit, again for each step of a pair (two of them at a time, so that the registers do).
+            constexpr bool BY_UNIT = RT > 2;
+            uint32_t index[2][BY_UNIT ? 1 : NU], shifted;
+            auto even_index = [&](auto U, auto W) { return (R[U][(int)W] & mask55) | high88; };
+            static_for<BY_UNIT ? 1 : ACTIVE>([&](auto U) { index[0][U] = even_index(U, std::integral_constant<int, 0>{}); });
             static_for<4 / WS>([&](auto Sc) {
                 constexpr int w0 = Sc * WS;
                 constexpr bool last_stage = w0 + WS == 4;
@@ -230,10 +253,12 @@ __global__ __launch_bounds__(kRowsWaves * 64) void lut_rows_kernel(MatvecArgs a,
                 if constexpr (!last_stage) load_pieces(kb, w0 + WS);
                 else if constexpr (!last_pass) load_pieces(kb, 0);
                 else load_pieces(kb + KW, 0);
+                if constexpr (Sc == 0) load_signs(last_pass ? next : cur, std::integral_constant<int, pg_next>{});
                 const lds_byte *xr = xbuf + buf * XBUF + xlane;
                 half16 B[2][RT];
+                // step: word, parity p of k, half hh of the index register; one index serves the two steps of (w, p)
                 auto read_step = [&](auto Gc) {
-                    constexpr int wl = Gc / 4, hh = (Gc / 2) % 2, p = Gc % 2;
+                    constexpr int wl = Gc / 4, p = (Gc / 2) % 2, hh = Gc % 2;
                     static_for<RT>([&](auto T) {
                         const lds_byte *at = xr + T * (16 * PITCH) + wl * 128 + (2 * hh + p) * 32;
                         const half8 b0 = *reinterpret_cast<const lds_half8 *>(at);
@@ -242,33 +267,59 @@ __global__ __launch_bounds__(kRowsWaves * 64) void lut_rows_kernel(MatvecArgs a,
                     });
                 };
                 read_step(std::integral_constant<int, 0>{});
-                half8 A[NU];
+                __builtin_amdgcn_sched_barrier(0);
                 static_for<4 * WS>([&](auto Gc) {
-                    constexpr int w = w0 + Gc / 4, hh = (Gc / 2) % 2, p = Gc % 2;
-                    if constexpr (Gc % 4 == 0) {   // the scales of this word become operands, those of the next are fetched
-                        static_for<NU>([&](auto U) {
-                            if constexpr (pg * QP + U / 2 < P) {
-                                const uint32_t s = scale[U] * vmask;
-                                A[U] = __builtin_bit_cast(half8, u32x4{s, s, s, s});
-                            }
-                        });
-                        if constexpr (w < 3) load_scales(tile, w + 1, Pc);
-                        else load_scales(last_pass ? next_tile : tile, 0, std::integral_constant<int, (pg + 1) % PG>{});
+                    constexpr int w = w0 + Gc / 4, p = (Gc / 2) % 2, hh = Gc % 2, pair = 2 * w + p;
+                    constexpr bool last_word = w == 3, stage_end = Gc / 4 == WS - 1;
+                    if constexpr (Gc % 4 == 0) {   // scales of the next word
+                        if constexpr (!last_word) {
+                            if (!one_group) load_scales(cur, w + 1, Pc);
+                        } else {
+                            load_scales(last_pass ? next : cur, 0, std::integral_constant<int, pg_next>{});
+                        }
                     }
                     if constexpr (Gc + 1 < 4 * WS) read_step(std::integral_constant<int, (Gc + 1 < 4 * WS ? Gc + 1 : 0)>{});
                     __builtin_amdgcn_sched_barrier(0);   // the reads of the next step go out ahead of this one's products
-                    static_for<NU>([&](auto U) {
-                        if constexpr (pg * QP + U / 2 < P) {
-                            const uint32_t word = w == 0 ? R[U].x : w == 1 ? R[U].y : w == 2 ? R[U].z : R[U].w;
-                            const int index = (int)(((p ? word >> 1 : word) & mask55) | high88);
-                            static_for<RT>([&](auto T) {
-                                acc[U % 2][T] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(A[U], B[Gc % 2][T], acc[U % 2][T], index, 0, hh);
+                    static_for<ACTIVE * RT>([&](auto Sl) {
+                        constexpr int U = Sl / RT, T = Sl % RT;
+                        const int picks = (int)(BY_UNIT ? index[U % 2][0] : index[pair % 2][BY_UNIT ? 0 : U]);
+                        acc[U % 2][T] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(A[U], B[Gc % 2][T], acc[U % 2][T], picks, 0, hh);
+                        __builtin_amdgcn_sched_barrier(0);
+                        // Behind each matrix instruction one other, for nothing: the indices (for even k one instruction, for odd k
+                        // two), and in the last steps of a stage the next stage's activations.
+                        constexpr int step_slots = BY_UNIT ? ACTIVE * (RT - 2) : ACTIVE * RT;
+                        constexpr int made = BY_UNIT || last_word || p == 0 ? 0 : ACTIVE;   // slots of the pair taken by indices
+                        constexpr int slot = hh * step_slots + (BY_UNIT ? U * (RT - 2) + T - 2 : Sl);
+                        if constexpr (BY_UNIT) {
+                            constexpr bool wraps = U + 1 == ACTIVE;   // the next unit is the first one of the next step
+                            constexpr int nu = wraps ? 0 : U + 1, np = wraps && hh ? 1 - p : p, nw_ = wraps && hh && p ? w + 1 : w;
+                            if constexpr (nw_ < 4) {
+                                if constexpr (np == 0 && T == 0) index[nu % 2][0] = even_index(std::integral_constant<int, nu>{}, std::integral_constant<int, nw_ % 4>{});
+                                if constexpr (np == 1 && T == 0) shifted = R[nu][nw_ % 4] >> 1;
+                                if constexpr (np == 1 && T == 1) index[nu % 2][0] = (shifted & mask55) | high88;
+                            }
+                        } else if constexpr (p == 0) {
+                            if constexpr (slot < 2 * ACTIVE) {
+                                if constexpr (slot % 2 == 0) shifted = R[slot / 2 % NU][w] >> 1;
+                                else index[(pair + 1) % 2][slot / 2 % NU] = (shifted & mask55) | high88;
+                            }
+                        } else if constexpr (slot < made) {
+                            index[(pair + 1) % 2][slot % NU] = even_index(std::integral_constant<int, slot % NU>{}, std::integral_constant<int, (w + 1) % 4>{});
+                        }
+                        if constexpr (SPREAD && p == 1 && stage_end && (BY_UNIT ? T >= 2 : slot >= made)) {
+                            constexpr int total = PIECES * PIECE_OPS, slots = 2 * step_slots - made, per = (total + slots - 1) / slots;
+                            static_for<per>([&](auto N) {
+                                constexpr int n = (slot - made) * per + N;
+                                if constexpr (n < total) piece_op(std::integral_constant<int, n / PIECE_OPS>{}, std::integral_constant<int, n % PIECE_OPS>{}, buf ^ 1);
                             });
                         }
+                        __builtin_amdgcn_sched_barrier(0);
                     });
-                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (Gc % 4 == 3 && !last_word) {
+                        if (!one_group) make_operands(vmask, Pc);
+                    }
                 });
-                store_pieces(buf ^ 1);
+                if constexpr (!SPREAD) store_pieces(buf ^ 1);
                 __syncthreads();
                 buf ^= 1;
             });
