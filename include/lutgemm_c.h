@@ -91,11 +91,11 @@ int lutgemm_weight_info(const lutgemm_weight *w, lutgemm_weight_info_t *info);
  * kernel::nqmv (mv_fp16.hpp:121) or kernel::nqmv_bias (mv_fp16_bias.hpp:143) and for m > 1
  * dequantises the whole weight and calls a library GEMM (kernels.cu:73-79); here every
  * 1 <= m <= LUTGEMM_MAX_BATCH streams the packed weight: m == 1 and m == 2 through the table-lookup
- * kernels (a two-row pass gives each row bit-identical to its own one-row call), 3 to 16 rows through
- * the batch kernel, which takes them in one pass over the weight and contracts them on the
- * matrix cores while a tile is in registers (any number of planes and any group size; weights of
- * more than four planes with workgroups of exactly eight wavefronts), and more rows through a kernel that contracts
- * a tile with up to 64 of them.  A launch of more than 16 rows that splits k keeps partial sums in memory of the stream's set,
+ * kernels (a two-row pass gives each row bit-identical to its own one-row call), 3 to 16 rows in one
+ * pass over the weight, contracted on the matrix cores while a tile is in registers (scale groups of a multiple of 128 k
+ * through the kernel for few rows, finer ones and weights with an infinite or NaN scale through the batch kernel), and more
+ * rows through a kernel that contracts a tile with up to 64 of them.  Partial sums of launches of 3 to 16 rows lie in memory that
+ * a stream's set is made with (none where the device had none left: sums then go through the accumulators).  A launch of more than 16 rows that splits k keeps partial sums in memory of the stream's set,
  * allocated when a launch first needs as much (a power of two of bytes, 2 KiB to 16 MiB; mostly 1 to 4 MiB; also under graph
  * capture, so that a captured launch gives the bits of an eager one) and held until the handle is destroyed; where the
  * device has no such memory left, k is not split on that set from then on (until lutgemm_weight_reset_workspace) and a
@@ -245,7 +245,7 @@ int lutgemm_weight_plan(const lutgemm_weight *w, int *workgroups, int *waves_per
                         int *k_splits, int *k_blocks_per_group);
 
 /* The same for the launches a call with m activation rows makes (m = 1: the plan above; m = 2:
- * the two-row plan; 3 <= m <= 16: the batch kernel's plan; beyond: that of the kernel for many rows, or the batch
+ * the two-row plan; 3 <= m <= 16: that of the kernel for few rows or of the batch kernel, whichever takes the call; beyond: that of the kernel for many rows, or the batch
  * kernel's if it takes them, with non-finite scales or a plan of the caller's).  LUTGEMM_ERR_BAD_SHAPE for m outside
  * 1..LUTGEMM_MAX_BATCH.  No counterpart in the reference. */
 int lutgemm_weight_plan_for(const lutgemm_weight *w, int m, int *workgroups, int *waves_per_group,
@@ -257,8 +257,8 @@ int lutgemm_weight_plan_for(const lutgemm_weight *w, int m, int *workgroups, int
  * (1..12 wavefronts per workgroup, 1..min(k/512 rounded up, 128) k-splits). */
 int lutgemm_weight_set_plan(lutgemm_weight *w, int waves_per_group, int k_splits);
 
-/* Override the batch kernel's launch plan (calls with 3 to 16 rows; calls with more then go through the
- * batch kernel as well, 16 rows per pass): 8..16 wavefronts per
+/* Override the batch kernel's launch plan (calls with 3 to 16 rows, which then all take that kernel, and so do
+ * calls with more, 16 rows per pass): 8..16 wavefronts per
  * workgroup (exactly 8 for weights of more than four planes; fewer than 16 where four scale
  * groups per 128 k leave less LDS) and the k-splits; both 0: back to the automatic choice.
  * LUTGEMM_ERR_BAD_SHAPE if the request cannot be launched.  No launch on the handle may be in
@@ -268,8 +268,8 @@ int lutgemm_weight_set_batch_plan(lutgemm_weight *w, int waves_per_group, int k_
 /* Measure the most promising launch plans on the device (a few launches each, on `stream`, with
  * scratch activations of its own) and keep the fastest, separately for launches with one
  * activation row and for two-row passes (which keep the k-split of the one-row plan, so that
- * rows stay bit-identical to their own one-row launches), and, where the batch kernel takes the
- * shape, for its passes of up to 8 and of 9 to 16 rows.  Optional: the automatic plan is chosen
+ * rows stay bit-identical to their own one-row launches), and for calls of 3 to 8 and of 9 to 16
+ * rows with the kernel that takes them.  Optional: the automatic plan is chosen
  * from a model, this replaces it by a measurement.  The measurement streams the weight from
  * HBM as a decoder does: it rotates over temporary device copies of the packed weight (about
  * 1 GiB in total, at most 64 copies) so that no launch finds its weight in the memory-side

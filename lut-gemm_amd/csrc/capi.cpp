@@ -75,8 +75,12 @@ struct StreamSet {
     bool zeroed;                 // they are, for work behind the fill on the stream that first claimed the set
     void *xrows;                 // staging of column-batched activations: xrows_cols rows of k halves,
     int xrows_cols;              //   grown on demand
-    float *partials[kRoomSizes]; // room for the sums of launches of more than 16 rows that split k: [c] holds 2^c units,
+    float *few_partials;         // room for the sums of launches of 3 to 16 rows that split k: few_units units
+    size_t few_units;
+    float *partials[kRoomSizes]; // the same for launches of more rows, and where few_units are too few: [c] holds 2^c units,
     bool no_room;                //   from the first launch that needs it on; an allocation failed: none is tried again
+    void *block;                 // the allocation that holds accum, the first xrows and few_partials (null in set 0: the
+    bool xrows_grown;            //   tiles' block); xrows is an allocation of its own
     hipEvent_t done;             // recorded behind the set's latest launch (only while done_valid)
     bool done_valid;
     unsigned long long last_use;
@@ -87,7 +91,7 @@ struct lutgemm_weight {
     Shape shape;
     int device;
     int compute_units;
-    uint8_t *d_signs;
+    uint8_t *d_signs;             // one allocation: the sign tiles, the scale tiles, the memory of set 0
     uint16_t *d_scales;
     bool finite_scales;           // no infinity or NaN among the scales and offsets
     std::mutex slot_mutex;
@@ -447,6 +451,46 @@ int refuse_capture(void *stream, const char *what)
     return fail(LUTGEMM_ERR_UNSUPPORTED, "%s synchronises with the device and cannot run on a stream under graph capture", what);
 }
 
+// Units of partial sums that the handle's plans for 3 to 16 rows write (0: none does).
+size_t few_room(const lutgemm_weight *w)
+{
+    size_t units = 0;
+    for (int m = 3; few_shape(w->shape) && m <= kRowsPerPass; m++) {
+        const int splits = w->plan_few[m > 8].k_splits;
+        if (splits > 1 && !few_takes_atomics(w->shape, m, splits)) units = std::max(units, (size_t)w->shape.nb * splits);
+    }
+    return units;
+}
+
+// The memory of a set in one piece: split-k words, kStagedColumns staged columns, `units` units of partial sums; set 0 lies
+// behind the tiles in theirs.  Every hipMalloc costs 20 to 40 us and every hipFree, which waits for the device, about 80: with
+// one allocation instead of four, a 4096 x 16384 weight of four planes is made from host arrays, expanded and freed in 2190
+// instead of 2270 us, and as no room is allocated behind a launch the first call of 12 columns on a new 7168 x 28672 weight
+// takes 68 us instead of 124 (of 8 rows on the four weights of a 12288 block: 195 instead of 282).
+constexpr size_t aligned256(size_t bytes) { return (bytes + 255) / 256 * 256; }
+size_t words_bytes(const lutgemm_weight *w) { return aligned256(set_words(w) * sizeof(unsigned long long)); }
+size_t staging_bytes(const lutgemm_weight *w) { return aligned256((size_t)kStagedColumns * w->shape.k * sizeof(uint16_t)); }
+
+// `front` bytes and, behind them, the memory of a set.  Where the device cannot hold the partial sums too, the set is made without
+// (few_units 0): its launches then look for room one by one (partials_of).
+int alloc_block(const lutgemm_weight *w, size_t front, StreamSet *t, char **block)
+{
+    const size_t base = front + words_bytes(w) + staging_bytes(w);
+    t->few_units = few_room(w);
+    hipError_t e = hipMalloc((void **)block, base + t->few_units * kPartialUnitBytes);
+    if (e != hipSuccess && t->few_units) {
+        (void)hipGetLastError();
+        t->few_units = 0;
+        e = hipMalloc((void **)block, base);
+    }
+    if (e != hipSuccess) return hip_fail(e, front ? "hipMalloc(weight)" : "hipMalloc(split-k accumulators)");
+    t->accum = reinterpret_cast<unsigned long long *>(*block + front);
+    t->xrows = *block + front + words_bytes(w);
+    t->xrows_cols = kStagedColumns;
+    t->few_partials = reinterpret_cast<float *>(*block + base);
+    return LUTGEMM_OK;
+}
+
 // Device memory of set i (idempotent), its words zeroed on `stream`, which has to be the first to launch on the set: a
 // hipMemset would run on the null stream, with which a stream need not be synchronised, and might come behind the first
 // launches, whose counts it would clear.  Allocates: not for a stream that is being captured.
@@ -454,13 +498,9 @@ int alloc_set(lutgemm_weight *w, int i, void *stream)
 {
     StreamSet &t = w->set[i];
     if (!t.accum) {
-        hipError_t e = hipMalloc((void **)&t.accum, set_words(w) * sizeof(unsigned long long));
-        if (e != hipSuccess) return hip_fail(e, "hipMalloc(split-k accumulators)");
-    }
-    if (!t.xrows) {
-        hipError_t e = hipMalloc(&t.xrows, (size_t)kStagedColumns * w->shape.k * sizeof(uint16_t));
-        if (e != hipSuccess) return hip_fail(e, "hipMalloc(column staging)");
-        t.xrows_cols = kStagedColumns;
+        char *block = nullptr;
+        if (int st = alloc_block(w, 0, &t, &block)) return st;
+        t.block = block;
     }
     if (!t.zeroed) {
         hipError_t e = lutgemm_kernels::launch_fill_zero(t.accum, set_words(w), static_cast<hipStream_t>(stream));
@@ -501,14 +541,30 @@ float *partials_of(lutgemm_weight *w, int slot, size_t units)
     return t.partials[size];
 }
 
+// For a launch of 3 to 16 rows: the room that the set was made with, so that a first launch allocates nothing; another one
+// where the set's plans changed since (room_for_plans).
+float *few_partials_of(lutgemm_weight *w, int slot, size_t units)
+{
+    const StreamSet &t = w->set[slot];
+    return units <= t.few_units ? t.few_partials : partials_of(w, slot, units);
+}
+
+// Other plans than the sets were made for (measured, or a clone's): their room is looked for now.
+void room_for_plans(lutgemm_weight *w)
+{
+    const size_t units = few_room(w);
+    for (int i = 0; i < kStreamSlots; i++)
+        if (w->set[i].accum && units > w->set[i].few_units) (void)partials_of(w, i, units);
+}
+
 size_t workspace_bytes(const lutgemm_weight *w)
 {
     size_t bytes = 0;
     for (int i = 0; i < kStreamSlots; i++) {
-        if (w->set[i].accum) bytes += set_words(w) * sizeof(unsigned long long);
+        if (w->set[i].accum) bytes += words_bytes(w) + staging_bytes(w) + w->set[i].few_units * kPartialUnitBytes;
         for (int c = 0; c < kRoomSizes; c++)
             if (w->set[i].partials[c]) bytes += kPartialUnitBytes << c;
-        if (w->set[i].xrows) bytes += (size_t)w->set[i].xrows_cols * w->shape.k * sizeof(uint16_t);
+        if (w->set[i].xrows_grown) bytes += (size_t)w->set[i].xrows_cols * w->shape.k * sizeof(uint16_t);
     }
     return bytes;
 }
@@ -654,18 +710,16 @@ int new_handle(const Shape &s, lutgemm_weight **out)
     w->device = dev;
     w->compute_units = units > 0 ? units : 256;
 
-    int st = LUTGEMM_OK;
-    e = hipMalloc((void **)&w->d_signs, sign_bytes(s));
-    if (e != hipSuccess) st = hip_fail(e, "hipMalloc(signs)");
+    w->plan = w->plan2 = choose_plan(s, w->compute_units);
+    w->batch_measured[0] = w->batch_measured[1] = false;
+    if (few_shape(s))
+        for (int i = 0; i < 2; i++) w->plan_few[i] = choose_few_plan(s, w->compute_units, i ? kRowsPerPass : 8);
+    const size_t signs = aligned256(sign_bytes(s)), scales = aligned256(scale_bytes(s));
+    char *block = nullptr;
+    int st = alloc_block(w, signs + scales, &w->set[0], &block);
     if (st == LUTGEMM_OK) {
-        e = hipMalloc((void **)&w->d_scales, scale_bytes(s));
-        if (e != hipSuccess) st = hip_fail(e, "hipMalloc(scales)");
-    }
-    if (st == LUTGEMM_OK) {
-        w->plan = w->plan2 = choose_plan(s, w->compute_units);
-        w->batch_measured[0] = w->batch_measured[1] = false;
-        if (few_shape(s))
-            for (int i = 0; i < 2; i++) w->plan_few[i] = choose_few_plan(s, w->compute_units, i ? kRowsPerPass : 8);
+        w->d_signs = reinterpret_cast<uint8_t *>(block);
+        w->d_scales = reinterpret_cast<uint16_t *>(block + signs);
         st = alloc_set(w, 0, nullptr);   // check_scales waits for the null stream before any stream can launch on the handle
     }
     if (st != LUTGEMM_OK) {
@@ -781,14 +835,13 @@ int pack_on_device(lutgemm_weight *w, const uint32_t *bW, const void *alpha, con
     const Shape &s = w->shape;
     const size_t item = halves ? 2 : 4, words = (size_t)(s.k / 32) * s.q * s.n * sizeof(uint32_t);
     const size_t scales = (size_t)s.num_groups * s.q * s.n * item, offsets = q_bias ? (size_t)s.num_groups * s.n * item : 0;
-    auto aligned = [](size_t b) { return (b + 255) / 256 * 256; };
     char *raw = nullptr;
     *done = false;
-    if (hipMalloc((void **)&raw, aligned(words) + aligned(scales) + offsets) != hipSuccess) {
+    if (hipMalloc((void **)&raw, aligned256(words) + aligned256(scales) + offsets) != hipSuccess) {
         (void)hipGetLastError();
         return LUTGEMM_OK;
     }
-    char *d_alpha = raw + aligned(words), *d_offsets = d_alpha + aligned(scales);
+    char *d_alpha = raw + aligned256(words), *d_offsets = d_alpha + aligned256(scales);
     int st = LUTGEMM_OK;
     auto copy = [&](void *to, const void *from, size_t bytes) {
         if (st != LUTGEMM_OK) return;
@@ -1004,12 +1057,16 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
             hipError_t e = hipStreamSynchronize(st);
             if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
             std::lock_guard<std::mutex> lock(mw->slot_mutex);
-            if (t.xrows) (void)hipFree(t.xrows);
-            t.xrows = nullptr;
-            t.xrows_cols = 0;
-            e = hipMalloc(&t.xrows, (size_t)m * s.k * sizeof(uint16_t));
+            void *grown = nullptr;
+            if (t.xrows_grown) (void)hipFree(t.xrows);
+            t.xrows = t.accum + words_bytes(w) / sizeof(unsigned long long);   // the set's first rows
+            t.xrows_cols = kStagedColumns;
+            t.xrows_grown = false;
+            e = hipMalloc(&grown, (size_t)m * s.k * sizeof(uint16_t));
             if (e != hipSuccess) return hip_fail(e, "hipMalloc(column staging)");
+            t.xrows = grown;
             t.xrows_cols = m;
+            t.xrows_grown = true;
         }
         uint16_t *rows = static_cast<uint16_t *>(t.xrows);
         hipError_t e = lutgemm_kernels::launch_gather_columns(x, rows, s.k, m, st);
@@ -1036,7 +1093,7 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
         a.y_stride = cols ? m : 1;   // y [n][m] or [m][n]
         a.y_row_stride = cols ? 1 : s.n;
         if (a.k_splits > 1 && !few_takes_atomics(s, m, a.k_splits))   // without room for partial sums atomics it is
-            g.partials = static_ws ? static_partials : partials_of(mw, slot, (size_t)s.nb * a.k_splits);
+            g.partials = static_ws ? static_partials : few_partials_of(mw, slot, (size_t)s.nb * a.k_splits);
         g.bias = bias;
         g.columns = few_columns;
         g.wide_y = !cols && s.n % 4 == 0 && ((uintptr_t)y & 7u) == 0;
@@ -1315,6 +1372,7 @@ int lutgemm_weight_clone(const lutgemm_weight *w, lutgemm_weight **out)
         }
         (*out)->batch_set = w->batch_set;
         for (int i = 0; i < 2; i++) (*out)->plan_few[i] = w->plan_few[i];
+        room_for_plans(*out);
     }
     return st;
 }
@@ -1383,10 +1441,10 @@ int lutgemm_weight_destroy(lutgemm_weight *w)
 {
     if (!w) return LUTGEMM_OK;
     int st = LUTGEMM_OK;
-    std::vector<void *> ptrs = {w->d_signs, w->d_scales};
+    std::vector<void *> ptrs = {w->d_signs};
     for (StreamSet &t : w->set) {
-        ptrs.push_back(t.accum);
-        ptrs.push_back(t.xrows);
+        ptrs.push_back(t.block);
+        if (t.xrows_grown) ptrs.push_back(t.xrows);
         ptrs.insert(ptrs.end(), t.partials, t.partials + kRoomSizes);
         if (t.done) (void)hipEventDestroy(t.done);
     }
@@ -1924,6 +1982,7 @@ int lutgemm_weight_autotune(lutgemm_weight *w, void *stream)
         (few ? w->plan_few : w->plan_batch)[bi] = ok ? chosen_batch[bi] : before_batch[bi];
         w->batch_measured[bi] = ok ? !few : before_measured[bi];
     }
+    room_for_plans(w);
     if (status == LUTGEMM_OK && have_batch[1]) w->batch_set = false;   // the caller's plan is replaced
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
