@@ -92,11 +92,11 @@ int lutgemm_weight_info(const lutgemm_weight *w, lutgemm_weight_info_t *info);
  * dequantises the whole weight and calls a library GEMM (kernels.cu:73-79); here every
  * 1 <= m <= LUTGEMM_MAX_BATCH streams the packed weight: m == 1 and m == 2 through the table-lookup
  * kernels (a two-row pass gives each row bit-identical to its own one-row call), 3 to 16 rows in one
- * pass over the weight, contracted on the matrix cores while a tile is in registers (scale groups of a multiple of 128 k
- * through the kernel for few rows, finer ones and weights with an infinite or NaN scale through the batch kernel), and more
- * rows through a kernel that contracts a tile with up to 64 of them.  Partial sums of launches of 3 to 16 rows lie in memory that
- * a stream's set is made with (none where the device had none left: sums then go through the accumulators).  A launch of more than 16 rows that splits k keeps partial sums in memory of the stream's set,
- * allocated when a launch first needs as much (a power of two of bytes, 2 KiB to 16 MiB; mostly 1 to 4 MiB; also under graph
+ * pass over the weight, contracted on the matrix cores while a tile is in registers (through the kernel for few rows; weights
+ * with an infinite or NaN scale, or with a plan set for it, through the batch kernel), and more rows through a kernel that
+ * contracts a tile with up to 64 of them.  Partial sums of launches of 3 to 16 rows lie in memory that a stream's set is made
+ * with (where the device had none left, sums go through the accumulators).  A launch of more than 16 rows that splits k keeps
+ * partial sums in memory of the stream's set, allocated when a launch first needs as much (a power of two of bytes, 2 KiB to 16 MiB; mostly 1 to 4 MiB; also under graph
  * capture, so that a captured launch gives the bits of an eager one) and held until the handle is destroyed; where the
  * device has no such memory left, k is not split on that set from then on (until lutgemm_weight_reset_workspace) and a
  * result may differ in the last bit.  Batch results are deterministic and within

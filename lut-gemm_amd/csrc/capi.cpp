@@ -296,7 +296,7 @@ Plan choose_few_plan(const Shape &s, int cus, int rows)
 {
     Plan best{lutgemm_kernels::kFewWavesMin, div_up(s.nb, lutgemm_kernels::kFewWavesMin), s.ts, 1};
     double best_cost = 1e30;
-    for (int waves = lutgemm_kernels::kFewWavesMin; waves <= lutgemm_kernels::few_waves_max(s.qo); waves++)
+    for (int waves = lutgemm_kernels::kFewWavesMin; waves <= lutgemm_kernels::few_waves_max(s.qo, s.gsub); waves++)
         for (int ks = 1; ks <= s.ts && ks <= kMaxSplits; ks++) {
             Plan p;
             const double cost = few_plan_cost(s, cus, waves, ks, rows, &p);
@@ -419,7 +419,7 @@ RowsPlan choose_rows_plan(const Shape &s, int cus, int m, bool may_split)
 }
 
 // Shapes that the kernel for few rows takes: one scale group per row of a tile, and rows that 32 bits address.
-bool few_shape(const Shape &s) { return s.gsub == 1 && s.k <= kMaxRowsK; }
+bool few_shape(const Shape &s) { return s.k <= kMaxRowsK; }
 
 // A handle's device memory belongs to the device that was current when it was created.
 int check_device(const lutgemm_weight *w)
@@ -748,8 +748,9 @@ bool takes_rows_kernel(const lutgemm_weight *w, int m)
 }
 
 // The same for the kernel for few rows, which also contracts with the scales as matrix operand.  It is the faster one of the two
-// on every shape measured (0.72 to 1.0 of the batch kernel's time, 0.79 on average); that keeps weights with finer scale groups,
-// with non-finite scales, and calls for which the caller has set its plan.
+// on every shape measured (groups of 128 and more 0.72 to 1.0 of the batch kernel's time, 0.79 on average; groups of 32 and 64
+// 0.62 to 0.94, 0.79 on average, 42 points over 14 shapes); that keeps weights with non-finite scales, and calls for which the
+// caller has set its plan.
 bool takes_few_kernel(const lutgemm_weight *w, int m)
 {
     return m >= 3 && m <= kRowsPerPass && few_shape(w->shape) && w->finite_scales && !w->batch_measured[m > 8];
@@ -1096,6 +1097,7 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
             g.partials = static_ws ? static_partials : few_partials_of(mw, slot, (size_t)s.nb * a.k_splits);
         g.bias = bias;
         g.columns = few_columns;
+        g.gsub = s.gsub;
         g.wide_y = !cols && s.n % 4 == 0 && ((uintptr_t)y & 7u) == 0;
         hipError_t e = lutgemm_kernels::launch_few(s.q, s.has_offset, a, g, few_plan.waves, st);
         if (e != hipSuccess) return hip_fail(e, "launch lut_few_kernel");
@@ -1946,7 +1948,7 @@ int lutgemm_weight_autotune(lutgemm_weight *w, void *stream)
         struct Timed { float ms; double cost; Plan p; };
         std::vector<Timed> timed;
         const int wmin = few ? lutgemm_kernels::kFewWavesMin : lutgemm_kernels::kBatchWavesMin;
-        const int wmax = few ? lutgemm_kernels::few_waves_max(s.qo) : lutgemm_kernels::batch_waves_max(s.gsub, s.q, s.qo);
+        const int wmax = few ? lutgemm_kernels::few_waves_max(s.qo, s.gsub) : lutgemm_kernels::batch_waves_max(s.gsub, s.q, s.qo);
         for (int waves = wmin; waves <= wmax; waves++)
             for (int ks = 1; ks <= s.ts && ks <= kMaxSplits; ks++) {
                 Plan p;

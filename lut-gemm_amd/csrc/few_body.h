@@ -1,5 +1,4 @@
-// gfx950 kernel for small batches, 3 to 16 activation rows against a packed BCQ weight in one pass over its tiles, where a
-// scale group is a multiple of 128 k (one scale per row of a tile, layout.h).
+// gfx950 kernel for small batches, 3 to 16 activation rows against a packed BCQ weight in one pass over its tiles.
 //
 // The contraction is the batch kernel's (batch_body.h): v_smfmac_f32_16x16x64_f16 with every activation in LDS as the
 // pair (-x, +x) and the sign bits as the index registers.  What bounds both is instruction issue: a matrix instruction
@@ -11,13 +10,17 @@
 //    own 128 consecutive k each (kappa: row kappa of the tile), so a lane's scale words are those of its own output.  An
 //    offset is one more plane whose index always picks +x.
 //  * The index of step pair n + 1 is made while step pair n is contracted (sched_barrier keeps the order).
+//  * With scale groups of 32 and 64 k (FINE) a lane's operands change from word to word.  The scales of a tile are 1 KiB per plane;
+//    they go through LDS, loaded a k-block ahead, and an operand is made anew behind its last use.  Loaded word by word, a word
+//    ahead, they were waited for: 12288 x 12288, two planes, groups of 64, 8 rows 20.0 us, now 17.4.
 //  * Activations and tiles come by buffer loads: an offset beyond the weight's k reads zero, and addresses are scalar.
 //  * Sums of a k-split go through memory (sum_partials): eight 64-bit atomics per lane took 3.5 to 5 us of a launch.
 // Products of two fp16 numbers are exact in the fp32 sums, so a result differs from the batch kernel's by fp32 rounding.
 // What bounds it now: power.  With the weight stream taken away the loop runs at the 10.7 ns a matrix instruction takes when all
 // compute units issue nothing else (6.9 ns on a few of them); the stream comes on top.  Measured (us, batch kernel -> this one, the
 // better plan of each): 12288 x 12288, two planes, 8 rows 20.3 -> 18.3; n = 36864 45.2 -> 36.4; n = 49152 50.1 -> 45.8; k = 49152
-// 51.4 -> 45.9; 7168 x 28672, three planes, 12 rows 34.4 -> 28.8; 12288 x 12288, four planes, 16 rows 36.7 -> 32.1.
+// 51.4 -> 45.9; 7168 x 28672, three planes, 12 rows 34.4 -> 28.8; 12288 x 12288, four planes, 16 rows 36.7 -> 32.1; groups of 64, 12288 x 12288, two planes, 8 rows 22.9 -> 17.4;
+// groups of 32, 7168 x 7168, three planes, 16 rows 21.3 -> 16.0, 12288 x 36864, two planes, 8 rows 50.4 -> 45.5.
 // Tried: transposing the next tile's signs during the steps (two sets of sign registers, three activation buffers, the barrier in
 // the middle of a k-block): no faster, 30 to 100 more registers; two workgroups per compute unit: no faster.
 #ifndef LUTGEMM_FEW_BODY_H
@@ -69,10 +72,10 @@ __device__ __forceinline__ uint32_t minus_plus(uint32_t pair, uint32_t selector)
 }
 
 // the largest workgroup an instance is compiled for
-constexpr int few_waves(int planes, FewInput in) { return in == FewInput::kColumns ? kFewWavesMin : few_waves_max(planes); }
+constexpr int few_waves(int planes, FewInput in, bool fine) { return in == FewInput::kColumns ? kFewWavesMin : few_waves_max(planes, fine ? 2 : 1); }
 
-template <int Q, bool OFF, FewInput IN>
-__global__ __launch_bounds__(few_waves(Q + OFF, IN) * 64) void lut_few_kernel(MatvecArgs a, FewGrid g)
+template <int Q, bool OFF, FewInput IN, bool FINE>
+__global__ __launch_bounds__(few_waves(Q + OFF, IN, FINE) * 64) void lut_few_kernel(MatvecArgs a, FewGrid g)
 {
     constexpr int P = Q + (OFF ? 1 : 0);
     constexpr int PG = (P + 3) / 4;              // passes over the planes of a k-block
@@ -101,8 +104,9 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN) * 64) void lut_few_kernel(Ma
     lds_v2i *stage_r0 = reinterpret_cast<lds_v2i *>(stage + (r_off ^ ((kappa & 1) * 128)));
     lds_v2i *stage_r1 = reinterpret_cast<lds_v2i *>(stage + ((r_off + 128) ^ ((kappa & 1) * 128)));
 
+    const int gsub = FINE ? g.gsub : 1, subl = 16 / gsub, lh = 2 * gsub * P;   // scales of a lane of a tile
     const auto sign_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(a.signs + tile0 * (size_t)(2 * Q * kUnitBytes)), (short)0, -1, kBufferFlags);
-    const auto scale_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(a.scales + tile0 * (size_t)(kLanes * 2 * P)), (short)0, -1, kBufferFlags);
+    const auto scale_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(a.scales + tile0 * (size_t)(kLanes * lh)), (short)0, a.ts * 2 * kLanes * lh, kBufferFlags);
     u32x4 sign[NU];
     auto load_signs = [&](int kb, auto Pc) {
         static_for<NU>([&](auto U) {
@@ -110,8 +114,9 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN) * 64) void lut_few_kernel(Ma
                 sign[U] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(sign_rsrc, lane * 16, kb * (2 * Q * kUnitBytes) + (Pc * NU + U) * kUnitBytes, 2));
         });
     };
-    uint32_t scale[P];   // of the next k-block: number h P + b is the scale of plane b, output 16 h + j
+    uint32_t scale[FINE ? 1 : P];   // of the next k-block: number h P + b is the scale of plane b, output 16 h + j
     auto load_scales = [&](int kb) {
+        if constexpr (FINE) return;
         const int from = lane * (4 * P), tile = kb * (kLanes * 4 * P);
         static_for<(P + 3) / 4>([&](auto I) {
             constexpr int n = P - 4 * I < 4 ? P - 4 * I : 4;
@@ -128,6 +133,34 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN) * 64) void lut_few_kernel(Ma
                 scale[4 * I] = __builtin_amdgcn_raw_buffer_load_b32(scale_rsrc, from + 16 * I, tile, 2);
             }
         });
+    };
+
+    // FINE: the scales of a tile lie in LDS, from where a word's go into its operands; those of the next k-block are on their way
+    // while one is contracted, and take its place when its last word's have been read.
+    lds_byte *scale_area = lds + 2 * kFewBuf + waves * kFewStage + wave * few_scale_area(P);
+    u32x4 fine[FINE ? P : 1];
+    auto load_fine = [&](int kb) {
+        static_for<P>([&](auto I) {
+            if (4 * I < gsub * P) fine[I] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(scale_rsrc, lane * 16, kb * (2 * kLanes * lh) + I * 1024, 2));
+        });
+    };
+    auto store_fine = [&]() {
+        static_for<P>([&](auto I) {
+            if (4 * I < gsub * P) *reinterpret_cast<lds_u32x4 *>(scale_area + I * 1024 + lane * 16) = fine[I];
+        });
+    };
+    const lds_byte *scale_at = scale_area + 2 * ((kappa * 16 + j % subl) * lh + (j / subl) * P);
+    uint32_t word_scale[FINE ? NU : 1];   // of word w for the units of pass Pc
+    auto read_word_scales = [&](int w, auto Pc) {
+        static_for<NU>([&](auto U) {
+            constexpr int b = Pc * QP + U / 2, h = U % 2;
+            if constexpr (b < P) word_scale[U] = *reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>(scale_at + (w * gsub / 4) * (2 * subl * lh) + h * lh + 2 * b);
+        });
+    };
+    half8 A[NU];
+    auto make_word_operand = [&](auto U) {
+        const uint32_t s = __builtin_amdgcn_perm(word_scale[U], word_scale[U], 0x01000100u);
+        A[U] = __builtin_bit_cast(half8, u32x4{s, s, s, s});
     };
 
     // Activations.  Rows: a wavefront moves one row (and the one `waves` further on) of a k-block, a lane one chunk of 16 bytes,
@@ -199,6 +232,7 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN) * 64) void lut_few_kernel(Ma
 
     load_pieces();
     load_scales(ts0);
+    if constexpr (FINE) load_fine(ts0);
     load_signs(ts0, std::integral_constant<int, 0>{});
     {
         constexpr int slots = 4 * (kFewPitch / 16);   // of a row, all lane groups
@@ -209,13 +243,21 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN) * 64) void lut_few_kernel(Ma
         }
     }
     store_pieces(0);
+    if constexpr (FINE) {
+        store_fine();
+        read_word_scales(0, std::integral_constant<int, 0>{});
+        static_for<NU>([&](auto U) {
+            if constexpr (U / 2 < P) make_word_operand(U);
+        });
+    }
     __syncthreads();
     int buf = 0;
     for (int kb = ts0; kb < ts1; kb++) {
         const int next = kb + 1 < ts1 ? kb + 1 : ts0;   // past the end a tile that is there
         load_pieces();
-        uint32_t sc[P];
-        static_for<P>([&](auto I) { sc[I] = scale[I]; });
+        uint32_t sc[FINE ? 1 : P];
+        if constexpr (!FINE) static_for<P>([&](auto I) { sc[I] = scale[I]; });
+        else load_fine(next);
         static_for<PG>([&](auto Pc) {
             constexpr int b0 = Pc * QP;
             u32x4 R[NU];   // sign bits of output j: word w are the 32 k 128 kappa + 32 w
@@ -227,10 +269,9 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN) * 64) void lut_few_kernel(Ma
                     R[U] = u32x4{(uint32_t)lo.x, (uint32_t)lo.y, (uint32_t)hi.x, (uint32_t)hi.y};
                 }
             });
-            half8 A[NU];
             static_for<NU>([&](auto U) {
                 constexpr int b = b0 + U / 2, number = (U % 2) * P + b;
-                if constexpr (b < P) {
+                if constexpr (b < P && !FINE) {
                     const uint32_t s = __builtin_amdgcn_perm(sc[number / 2], sc[number / 2], number % 2 ? 0x03020302u : 0x01000100u);
                     A[U] = __builtin_bit_cast(half8, u32x4{s, s, s, s});
                 }
@@ -259,6 +300,11 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN) * 64) void lut_few_kernel(Ma
             __builtin_amdgcn_sched_barrier(0);
             static_for<16>([&](auto Gc) {
                 constexpr int step = Gc, w = step / 4, p = (step / 2) % 2, hh = step % 2, pair = step / 2;
+                constexpr int pass_next = w == 3 ? (Pc + 1) % PG : (int)Pc;   // whose word comes behind this one
+                if constexpr (FINE && step % 4 == 0) {
+                    if constexpr (w == 3 && Pc + 1 == PG) store_fine();
+                    read_word_scales((w + 1) % 4, std::integral_constant<int, pass_next>{});
+                }
                 if constexpr (step + AHEAD < 16) read_step(std::integral_constant<int, (step + AHEAD < 16 ? step + AHEAD : 0)>{});
                 __builtin_amdgcn_sched_barrier(0);
                 static_for<NU>([&](auto U) {
@@ -279,6 +325,7 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN) * 64) void lut_few_kernel(Ma
                     } else if constexpr (w < 3 && slot < NU) {
                         if constexpr (b0 + slot / 2 < Q) index[(pair + 1) % 2][slot] = (R[slot % NU][(w + 1) % 4] & mask55) | high88;
                     }
+                    if constexpr (FINE && step % 4 == 3 && pass_next * QP + U / 2 < P) make_word_operand(U);   // its last use was this one
                     __builtin_amdgcn_sched_barrier(0);
                 });
             });
@@ -348,29 +395,30 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN) * 64) void lut_few_kernel(Ma
     });
 }
 
-template <int Q, bool OFF, FewInput IN>
+template <int Q, bool OFF, FewInput IN, bool FINE>
 hipError_t launch_few_one(const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t stream)
 {
-    constexpr int W = few_waves(Q + OFF, IN);
+    constexpr int W = few_waves(Q + OFF, IN, FINE);
     static std::atomic<unsigned long long> allowed{0};
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     const unsigned long long bit = 1ull << (dev & 63);
     if (!(allowed.load(std::memory_order_relaxed) & bit)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&lut_few_kernel<Q, OFF, IN>), hipFuncAttributeMaxDynamicSharedMemorySize, few_lds_bytes(W));
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&lut_few_kernel<Q, OFF, IN, FINE>), hipFuncAttributeMaxDynamicSharedMemorySize, few_lds_bytes(W) + (FINE ? W * few_scale_area(Q + OFF) : 0));
         if (e != hipSuccess) return e;
         allowed.fetch_or(bit, std::memory_order_relaxed);
     }
-    hipLaunchKernelGGL((lut_few_kernel<Q, OFF, IN>), dim3((unsigned)(a.ntiles * a.k_splits)), dim3(waves * kLanes), few_lds_bytes(waves), stream, a, g);
+    hipLaunchKernelGGL((lut_few_kernel<Q, OFF, IN, FINE>), dim3((unsigned)(a.ntiles * a.k_splits)), dim3(waves * kLanes),
+                       few_lds_bytes(waves) + (FINE ? waves * few_scale_area(Q + OFF) : 0), stream, a, g);
     return hipGetLastError();
 }
 
-template <FewInput IN>
+template <FewInput IN, bool FINE>
 hipError_t launch_few_input(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t s)
 {
     auto by_offset = [&](auto Qc) -> hipError_t {
-        return has_offset ? launch_few_one<Qc, true, IN>(a, g, waves, s) : launch_few_one<Qc, false, IN>(a, g, waves, s);
+        return has_offset ? launch_few_one<Qc, true, IN, FINE>(a, g, waves, s) : launch_few_one<Qc, false, IN, FINE>(a, g, waves, s);
     };
     switch (q) {
         case 1: return by_offset(std::integral_constant<int, 1>{});

@@ -5,7 +5,7 @@ namespace lutgemm_kernels {
 
 hipError_t launch_few_columns(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, hipStream_t s)
 {
-    return launch_few_input<FewInput::kColumns>(q, has_offset, a, g, kFewWavesMin, s);
+    return launch_few_input<FewInput::kColumns, false>(q, has_offset, a, g, kFewWavesMin, s);
 }
 
 }  // namespace lutgemm_kernels

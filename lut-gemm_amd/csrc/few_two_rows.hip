@@ -6,7 +6,7 @@ namespace lutgemm_kernels {
 
 hipError_t launch_few_two_rows(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t s)
 {
-    return launch_few_input<FewInput::kTwoRows>(q, has_offset, a, g, waves, s);
+    return launch_few_input<FewInput::kTwoRows, false>(q, has_offset, a, g, waves, s);
 }
 
 }  // namespace lutgemm_kernels

@@ -100,25 +100,36 @@ hipError_t launch_batch(int q, int has_offset, int gsub, const MatvecArgs &a, in
 hipError_t launch_batch_multi(int q, int has_offset, int gsub, const MultiMatvecArgs &m, int workgroups, int waves,
                               hipStream_t stream);
 
-// 3 to kBatchRows activation rows where a scale group is a multiple of 128 k (few_body.h): kFewWavesMin .. few_waves_max
-// wavefronts per workgroup (two planes and fewer take 128 registers per lane, three 168, more up to 256), one output batch
+// 3 to kBatchRows activation rows (few_body.h): kFewWavesMin .. few_waves_max
+// wavefronts per workgroup (two planes and fewer take 128 registers per lane, three 168, more up to 256; one plane less each with
+// scale groups of 32 and 64 k), one output batch
 // each; with activations as columns (x [k][rows]) exactly kFewWavesMin.
 constexpr int kFewWavesMin = 8;
-constexpr int few_waves_max(int planes) { return planes <= 2 ? 16 : planes == 3 ? 12 : 8; }
+constexpr int few_waves_max(int planes, int gsub)
+{
+    return gsub == 1 ? (planes <= 2 ? 16 : planes == 3 ? 12 : 8) : planes == 1 ? 16 : planes == 2 ? 12 : 8;
+}
 // a quarter of an activation row of a k-block, every value as the pair (-x, +x), with 16 bytes of padding; the sign staging of
 // a wavefront; two activation blocks and the staging of all wavefronts
 constexpr int kFewPitch = 4 * 128 + 16, kFewStage = 1024;
 constexpr int few_lds_bytes(int waves) { return 2 * 4 * kBatchRows * kFewPitch + waves * kFewStage; }
-static_assert(few_lds_bytes(16) <= 160 * 1024, "LDS of a compute unit");
+// and, for scale groups of 32 and 64 k, the scales of a wavefront's tile
+constexpr int few_scale_area(int planes) { return 1024 * planes; }
+static_assert(few_lds_bytes(16) + 16 * few_scale_area(1) <= 160 * 1024 && few_lds_bytes(12) + 12 * few_scale_area(2) <= 160 * 1024 &&
+              few_lds_bytes(8) + 8 * few_scale_area(kBatchMaxPlanes + 1) <= 160 * 1024, "LDS of a compute unit");
 struct FewGrid {
     const void *bias;  // fp16 [n] added to the rounded sum of an output, which is rounded again; null for none
     float *partials;   // k_splits > 1: 512 floats per (output batch, split) (no initial value); counts in accum[batch]
     int columns;       // x is [k][rows]
     int wide_y;        // four neighbouring outputs of a row are 8-byte aligned in y
+    int gsub;          // scale groups per 128 k: 1, 2 or 4
 };
 hipError_t launch_few(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t stream);
 hipError_t launch_few_two_rows(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t stream);   // rows > waves
 hipError_t launch_few_columns(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, hipStream_t stream);
+hipError_t launch_few_fine(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t stream);   // gsub > 1
+hipError_t launch_few_fine_two_rows(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t stream);
+hipError_t launch_few_fine_columns(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, hipStream_t stream);
 
 // Many activation rows in one launch (rows_body.h): a workgroup of kRowsWaves wavefronts takes 16 rt rows and
 // kRowsWaves / kw output batches, its wavefronts in kw groups that share out the k-blocks; row_chunks workgroups share

@@ -1,4 +1,4 @@
-// Every instance of the kernel for 3 to 16 rows (launch_few): planes, with and without an offset, activations as rows (at most
+// Every instance of the kernel for 3 to 16 rows (launch_few): planes, with and without an offset, scale groups of 128, 64 and 32 k, activations as rows (at most
 // one and two per wavefront) and as columns, with and without splits along k, their sums by atomics and through memory, with a
 // partial output batch, group of batches and k-block; results in rows of 8-byte and of 2-byte stores and in columns, with
 // and without bias.  Results against double precision within the tolerance of the path (oracle/oracle.py), the same launch
@@ -30,7 +30,6 @@ namespace {
 
 constexpr int kK = 1664, kN = 300, kTs = 4, kNb = 10;   // the last k-block is a quarter, the last batch 12 outputs
 constexpr int kMaxRows = lutgemm_kernels::kBatchRows;
-constexpr int kGroup = 128;
 constexpr int kGuard = 4096;                            // halves behind the results
 
 uint16_t bits(_Float16 v) { uint16_t b; memcpy(&b, &v, 2); return b; }
@@ -79,11 +78,11 @@ std::vector<_Float16> launch(int q, bool offset, int waves, bool atomics, lutgem
     return out;
 }
 
-void run_weight(int q, bool offset, int *variant)
+void run_weight(int q, bool offset, int group, int *variant)
 {
     std::mt19937 rng(q * 2 + offset);
     std::normal_distribution<float> normal;
-    const int planes = q + offset, group = kGroup, groups = kK / group;
+    const int planes = q + offset, groups = kK / group;
     std::vector<uint32_t> words((size_t)kK / 32 * q * kN);
     for (auto &w : words) w = rng();
     std::vector<_Float16> alpha((size_t)groups * q * kN), z((size_t)groups * kN), x((size_t)kMaxRows * kK), bias(kN);
@@ -115,7 +114,7 @@ void run_weight(int q, bool offset, int *variant)
     void *signs = nullptr, *scales = nullptr;
     lutgemm_weight_device_ptrs(w, &signs, &scales, nullptr);
     _Float16 *xd = to_device(x), *bd = to_device(bias);
-    const int wmax = lutgemm_kernels::few_waves_max(planes);
+    const int wmax = lutgemm_kernels::few_waves_max(planes, 128 / group);
     uint16_t *xc = nullptr;   // the first rows of x as columns
     HIP_OK(hipMalloc((void **)&xc, (size_t)kK * kMaxRows * 2));
     for (int rows : {3, 8, 9, 16}) {
@@ -141,8 +140,9 @@ void run_weight(int q, bool offset, int *variant)
                 a.x_row_stride = kK;
                 lutgemm_kernels::FewGrid g{};
                 g.wide_y = v % 3 == 0;
+                g.gsub = 128 / group;
                 const bool y_cols = v % 3 == 2;
-                printf("case few rows instance planes %d offset %d rows %d wavefronts %d splits %d %s\n", planes, offset, rows, waves, a.k_splits,
+                printf("case few rows instance planes %d offset %d groups of %d rows %d wavefronts %d splits %d %s\n", planes, offset, group, rows, waves, a.k_splits,
                        end ? "atomics" : "memory");
                 fflush(stdout);
                 const std::vector<_Float16> y = launch(q, offset, waves, end, a, g, y_cols), again = launch(q, offset, waves, end, a, g, y_cols);
@@ -179,7 +179,8 @@ int main()
 {
     int variant = 0;
     for (int q = 1; q <= 8; q++)
-        for (int offset = 0; offset < 2; offset++) run_weight(q, offset, &variant);
+        for (int offset = 0; offset < 2; offset++)
+            for (int group : {128, 64, 32}) run_weight(q, offset, group, &variant);
     printf("FEW OK %d\n", variant);
     return 0;
 }
