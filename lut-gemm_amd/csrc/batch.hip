@@ -1,5 +1,6 @@
 // The batch kernel for one batch: 3..16 activation rows against a packed BCQ weight in one pass
-// over its tiles (workgroup body and description: batch_body.h).
+// over its tiles (workgroup body and description: batch_body.h).  It takes the weights with a non-finite scale, which the
+// kernels that contract with the scales cannot (few_body.h, rows_body.h), and calls for which its plan was set.
 #include "batch_body.h"
 
 namespace lutgemm_kernels {

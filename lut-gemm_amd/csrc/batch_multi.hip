@@ -1,8 +1,9 @@
 // The batch kernel as a work list, like lut_matvec_multi_kernel: up to kMaxFused independent
 // batches (same planes, offset and scale layout, same wavefronts per workgroup; each with its own
 // weight, rows and k-split) share one grid, entry i owning the workgroups first_block[i] ..
-// first_block[i + 1] - 1 (workgroup body: batch_body.h).  A kernel of its own beside the one for a
-// single batch: the larger kernel arguments cost a launch one to two microseconds.
+// first_block[i + 1] - 1 (workgroup body: batch_body.h); weights with a
+// non-finite scale come here, few_multi.hip takes the others.  A kernel of its own beside the one for a single batch: the
+// larger kernel arguments cost a launch one to two microseconds.
 #include "batch_body.h"
 
 namespace lutgemm_kernels {

@@ -359,6 +359,46 @@ FusedPlan choose_fused_batch_plan(const Shape *const *shapes, const int *rows, i
     return best;
 }
 
+// The same for the kernel for few rows, with the terms of few_plan_cost: rounds of workgroups, one per compute unit, against the
+// stream of all weights, and the atomics of a k-split (a list's sums always go through the accumulators).  On the 39 lists that
+// lutgemm_matvec_many_autotune was tried on, its choice is within 5 % of the fastest candidate.
+FusedPlan choose_fused_few_plan(const Shape *const *shapes, const int *rows, int count, int cus,
+                                std::vector<FusedCandidate> *all = nullptr)
+{
+    const double round_us = 1.5, tile_us = 0.0745, two_rows = 1.1212, block_us = 0.169, block_floor = 0.6, bytes_per_us = 7.135e6;
+    const double atomics_us = 2.34, atomic_us = 5.07e-6;
+    int max_ts = 1;
+    double stream = 0.0;
+    for (int e = 0; e < count; e++) {
+        max_ts = std::max(max_ts, shapes[e]->ts);
+        stream += (double)(sign_bytes(*shapes[e]) + scale_bytes(*shapes[e])) / bytes_per_us;
+    }
+    const int wmax = lutgemm_kernels::few_waves_max(shapes[0]->qo, shapes[0]->gsub);   // the entries have one kernel instance
+    FusedPlan best{wmax, max_ts};
+    double best_cost = 1e300;
+    for (int waves = lutgemm_kernels::kFewWavesMin; waves <= wmax; waves++)
+        for (int bpg = div_up(max_ts, kMaxSplits); bpg <= max_ts; bpg++) {
+            long groups = 0;
+            double work = 0.0, atomics = 0.0;
+            for (int e = 0; e < count; e++) {
+                const Shape &s = *shapes[e];
+                const int b = bpg < s.ts ? bpg : s.ts, ks = div_up(s.ts, b);
+                const long g = (long)div_up(s.nb, waves) * ks;
+                groups += g;
+                work += (double)g * b * std::max(waves * s.qo * tile_us * (rows[e] > 8 ? two_rows : 1.0) + block_us, block_floor);
+                if (ks > 1) atomics += (double)s.n * rows[e] * ks;
+            }
+            const double rounds = (double)((groups + cus - 1) / cus), busy = rounds * work / (double)groups;
+            const double cost = rounds * round_us + std::sqrt(busy * busy + stream * stream) + (atomics > 0.0 ? atomics_us + atomic_us * atomics : 0.0);
+            if (all) all->push_back(FusedCandidate{cost, FusedPlan{waves, bpg}});
+            if (cost < best_cost - 1e-9) {
+                best_cost = cost;
+                best = FusedPlan{waves, bpg};
+            }
+        }
+    return best;
+}
+
 // Launch plan of the kernel for more than 16 rows (rows_body.h): output batches per workgroup (8, or 4 with the
 // wavefronts in two groups along k), row tiles of 16 per workgroup, workgroups along the rows and along k.
 struct RowsPlan {
@@ -1204,6 +1244,14 @@ int fused_kind(int m)
     return 0;
 }
 
+// kind 4: the kernel for few rows takes the batches (39 lists of 2 to 12 entries, k and n 512 to 49152, one to eight planes, 3 to 16
+// rows: 0.68 to 1.04 of the batch kernel's time, 0.89 on average)
+int fused_kind(const lutgemm_weight *w, int m)
+{
+    const int kind = fused_kind(m);
+    return kind == 2 && few_shape(w->shape) && w->finite_scales ? 4 : kind;
+}
+
 // Longest run of entries starting at i that one launch can take: the same kind and kernel
 // instance, no handle twice (its split-k words would be shared), and no output overlapping an
 // input or output of another entry of the run, so that their order does not matter.  Returns the
@@ -1217,10 +1265,10 @@ int form_run(const lutgemm_weight *const *ws, const void *const *xs, void *const
     run->multi = lutgemm_kernels::MultiMatvecArgs{};
     int j = i;
     const lutgemm_weight *w0 = ws[i];
-    const int kind = w0 && xs[i] && ys[i] ? fused_kind(ms[i]) : 0;
+    const int kind = w0 && xs[i] && ys[i] ? fused_kind(w0, ms[i]) : 0;
     for (; kind != 0 && j < count && j - i < lutgemm_kernels::kMaxFused; j++) {
         const lutgemm_weight *w = ws[j];
-        if (!w || !xs[j] || !ys[j] || ((uintptr_t)xs[j] & 15u) != 0 || fused_kind(ms[j]) != kind) break;
+        if (!w || !xs[j] || !ys[j] || ((uintptr_t)xs[j] & 15u) != 0 || fused_kind(w, ms[j]) != kind) break;
         const Shape &s = w->shape;
         if (s.q != w0->shape.q || s.has_offset != w0->shape.has_offset || s.gsub != w0->shape.gsub ||
             w->device != w0->device)
@@ -1258,8 +1306,9 @@ int form_run(const lutgemm_weight *const *ws, const void *const *xs, void *const
 FusedPlan model_fused_plan(const FusedRun &run, std::vector<FusedCandidate> *all)
 {
     const int cus = run.handle[0]->compute_units;
-    return run.kind == 2 ? choose_fused_batch_plan(run.shape, run.rows, run.count, cus, all)
-                         : choose_fused_plan(run.shape, run.count, cus, run.kind == 1 ? 1 : 2, all);
+    return run.kind == 4   ? choose_fused_few_plan(run.shape, run.rows, run.count, cus, all)
+         : run.kind == 2   ? choose_fused_batch_plan(run.shape, run.rows, run.count, cus, all)
+                           : choose_fused_plan(run.shape, run.count, cus, run.kind == 1 ? 1 : 2, all);
 }
 
 // two plans that give every entry of the run the same grid
@@ -1330,11 +1379,25 @@ int launch_run(FusedRun &run, const FusedPlan &fp, void *stream)
         a.accum = we->set[slots[e]].accum;
     }
     run.multi.count = run.count;
-    hipError_t e = run.kind != 2 ? lutgemm_kernels::launch_matvec_multi(s0.q, s0.has_offset, s0.gsub, run.multi, blocks, fp.waves,
-                                                                       static_cast<hipStream_t>(stream))
-                                 : lutgemm_kernels::launch_batch_multi(s0.q, s0.has_offset, s0.gsub, run.multi, blocks, fp.waves,
-                                                                       static_cast<hipStream_t>(stream));
-    if (e != hipSuccess) return hip_fail(e, run.kind != 2 ? "launch lut_matvec_multi_kernel" : "launch lut_batch_multi_kernel");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    hipError_t e;
+    const char *what;
+    if (run.kind == 4) {
+        lutgemm_kernels::FewGrid g{};
+        g.gsub = s0.gsub;
+        g.wide_y = 1;
+        for (int en = 0; en < run.count; en++)
+            if (run.shape[en]->n % 4 != 0 || ((uintptr_t)run.multi.entry[en].y & 7u) != 0) g.wide_y = 0;
+        e = lutgemm_kernels::launch_few_multi(s0.q, s0.has_offset, run.multi, g, blocks, fp.waves, st);
+        what = "launch lut_few_multi_kernel";
+    } else if (run.kind == 2) {
+        e = lutgemm_kernels::launch_batch_multi(s0.q, s0.has_offset, s0.gsub, run.multi, blocks, fp.waves, st);
+        what = "launch lut_batch_multi_kernel";
+    } else {
+        e = lutgemm_kernels::launch_matvec_multi(s0.q, s0.has_offset, s0.gsub, run.multi, blocks, fp.waves, st);
+        what = "launch lut_matvec_multi_kernel";
+    }
+    if (e != hipSuccess) return hip_fail(e, what);
     for (int en = 0; en < run.count; en++) leases[en].launched = true;
     return LUTGEMM_OK;
 }

@@ -74,8 +74,9 @@ __device__ __forceinline__ uint32_t minus_plus(uint32_t pair, uint32_t selector)
 // the largest workgroup an instance is compiled for
 constexpr int few_waves(int planes, FewInput in, bool fine) { return in == FewInput::kColumns ? kFewWavesMin : few_waves_max(planes, fine ? 2 : 1); }
 
+// workgroup `block` of a launch of a.ntiles * a.k_splits
 template <int Q, bool OFF, FewInput IN, bool FINE>
-__global__ __launch_bounds__(few_waves(Q + OFF, IN, FINE) * 64) void lut_few_kernel(MatvecArgs a, FewGrid g)
+__device__ __forceinline__ void few_workgroup(const MatvecArgs &a, const FewGrid &g, unsigned block)
 {
     constexpr int P = Q + (OFF ? 1 : 0);
     constexpr int PG = (P + 3) / 4;              // passes over the planes of a k-block
@@ -90,7 +91,7 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN, FINE) * 64) void lut_few_ker
     const int tid = threadIdx.x, lane = tid & 63, waves = blockDim.x >> 6;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kappa = lane >> 4, j = lane & 15;
-    const int ntile = (int)(blockIdx.x % (unsigned)a.ntiles), ks = (int)(blockIdx.x / (unsigned)a.ntiles);
+    const int ntile = (int)(block % (unsigned)a.ntiles), ks = (int)(block / (unsigned)a.ntiles);
     const int nb = ntile * waves + wave;
     const bool active = nb < a.nb;
     const int ts0 = ks * a.blocks_per_split, ts1 = min(ts0 + a.blocks_per_split, a.ts);
@@ -114,7 +115,7 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN, FINE) * 64) void lut_few_ker
                 sign[U] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(sign_rsrc, lane * 16, kb * (2 * Q * kUnitBytes) + (Pc * NU + U) * kUnitBytes, 2));
         });
     };
-    uint32_t scale[FINE ? 1 : P];   // of the next k-block: number h P + b is the scale of plane b, output 16 h + j
+    uint32_t scale[P];   // of the next k-block: number h P + b is the scale of plane b, output 16 h + j
     auto load_scales = [&](int kb) {
         if constexpr (FINE) return;
         const int from = lane * (4 * P), tile = kb * (kLanes * 4 * P);
@@ -138,7 +139,7 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN, FINE) * 64) void lut_few_ker
     // FINE: the scales of a tile lie in LDS, from where a word's go into its operands; those of the next k-block are on their way
     // while one is contracted, and take its place when its last word's have been read.
     lds_byte *scale_area = lds + 2 * kFewBuf + waves * kFewStage + wave * few_scale_area(P);
-    u32x4 fine[FINE ? P : 1];
+    u32x4 fine[P];
     auto load_fine = [&](int kb) {
         static_for<P>([&](auto I) {
             if (4 * I < gsub * P) fine[I] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(scale_rsrc, lane * 16, kb * (2 * kLanes * lh) + I * 1024, 2));
@@ -150,7 +151,7 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN, FINE) * 64) void lut_few_ker
         });
     };
     const lds_byte *scale_at = scale_area + 2 * ((kappa * 16 + j % subl) * lh + (j / subl) * P);
-    uint32_t word_scale[FINE ? NU : 1];   // of word w for the units of pass Pc
+    uint32_t word_scale[NU];   // of word w for the units of pass Pc
     auto read_word_scales = [&](int w, auto Pc) {
         static_for<NU>([&](auto U) {
             constexpr int b = Pc * QP + U / 2, h = U % 2;
@@ -255,7 +256,7 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN, FINE) * 64) void lut_few_ker
     for (int kb = ts0; kb < ts1; kb++) {
         const int next = kb + 1 < ts1 ? kb + 1 : ts0;   // past the end a tile that is there
         load_pieces();
-        uint32_t sc[FINE ? 1 : P];
+        uint32_t sc[P];
         if constexpr (!FINE) static_for<P>([&](auto I) { sc[I] = scale[I]; });
         else load_fine(next);
         static_for<PG>([&](auto Pc) {
@@ -396,30 +397,63 @@ __global__ __launch_bounds__(few_waves(Q + OFF, IN, FINE) * 64) void lut_few_ker
 }
 
 template <int Q, bool OFF, FewInput IN, bool FINE>
-hipError_t launch_few_one(const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t stream)
+__global__ __launch_bounds__(few_waves(Q + OFF, IN, FINE) * 64) void lut_few_kernel(MatvecArgs a, FewGrid g)
+{
+    few_workgroup<Q, OFF, IN, FINE>(a, g, blockIdx.x);
+}
+
+// A work list (like lut_matvec_multi_kernel): entry i owns the workgroups first_block[i] .. first_block[i + 1] - 1.  A kernel of its
+// own beside the one for a single batch, since the larger kernel arguments cost a launch one to two microseconds.
+template <int Q, bool OFF, FewInput IN, bool FINE>
+__global__ __launch_bounds__(few_waves(Q + OFF, IN, FINE) * 64) void lut_few_multi_kernel(MultiMatvecArgs m, FewGrid g)
+{
+    int i = 0;
+    while (i + 1 < m.count && (int)blockIdx.x >= m.first_block[i + 1]) i++;   // scalar: at most 31 steps
+    few_workgroup<Q, OFF, IN, FINE>(m.entry[i], g, blockIdx.x - (unsigned)m.first_block[i]);
+}
+
+template <int Q, bool OFF, FewInput IN, bool FINE>
+hipError_t allow_few_lds(const void *kernel, std::atomic<unsigned long long> &allowed)
 {
     constexpr int W = few_waves(Q + OFF, IN, FINE);
-    static std::atomic<unsigned long long> allowed{0};
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     const unsigned long long bit = 1ull << (dev & 63);
-    if (!(allowed.load(std::memory_order_relaxed) & bit)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&lut_few_kernel<Q, OFF, IN, FINE>), hipFuncAttributeMaxDynamicSharedMemorySize, few_lds_bytes(W) + (FINE ? W * few_scale_area(Q + OFF) : 0));
-        if (e != hipSuccess) return e;
-        allowed.fetch_or(bit, std::memory_order_relaxed);
-    }
+    if (allowed.load(std::memory_order_relaxed) & bit) return hipSuccess;
+    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, few_lds_bytes(W) + (FINE ? W * few_scale_area(Q + OFF) : 0));
+    if (e == hipSuccess) allowed.fetch_or(bit, std::memory_order_relaxed);
+    return e;
+}
+
+template <int Q, bool OFF, FewInput IN, bool FINE>
+hipError_t launch_few_one(const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t stream)
+{
+    static std::atomic<unsigned long long> allowed{0};
+    const hipError_t e = allow_few_lds<Q, OFF, IN, FINE>(reinterpret_cast<const void *>(&lut_few_kernel<Q, OFF, IN, FINE>), allowed);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL((lut_few_kernel<Q, OFF, IN, FINE>), dim3((unsigned)(a.ntiles * a.k_splits)), dim3(waves * kLanes),
                        few_lds_bytes(waves) + (FINE ? waves * few_scale_area(Q + OFF) : 0), stream, a, g);
     return hipGetLastError();
 }
 
-template <FewInput IN, bool FINE>
-hipError_t launch_few_input(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t s)
+// `workgroups`: of all entries
+template <int Q, bool OFF, FewInput IN, bool FINE>
+hipError_t launch_few_list(const MultiMatvecArgs &m, const FewGrid &g, int workgroups, int waves, hipStream_t stream)
 {
-    auto by_offset = [&](auto Qc) -> hipError_t {
-        return has_offset ? launch_few_one<Qc, true, IN, FINE>(a, g, waves, s) : launch_few_one<Qc, false, IN, FINE>(a, g, waves, s);
-    };
+    static std::atomic<unsigned long long> allowed{0};
+    const hipError_t e = allow_few_lds<Q, OFF, IN, FINE>(reinterpret_cast<const void *>(&lut_few_multi_kernel<Q, OFF, IN, FINE>), allowed);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((lut_few_multi_kernel<Q, OFF, IN, FINE>), dim3((unsigned)workgroups), dim3(waves * kLanes),
+                       few_lds_bytes(waves) + (FINE ? waves * few_scale_area(Q + OFF) : 0), stream, m, g);
+    return hipGetLastError();
+}
+
+// launch(planes, offset) for the weight's
+template <typename Launch>
+hipError_t by_planes(int q, int has_offset, Launch launch)
+{
+    auto by_offset = [&](auto Qc) -> hipError_t { return has_offset ? launch(Qc, std::true_type{}) : launch(Qc, std::false_type{}); };
     switch (q) {
         case 1: return by_offset(std::integral_constant<int, 1>{});
         case 2: return by_offset(std::integral_constant<int, 2>{});
@@ -431,6 +465,18 @@ hipError_t launch_few_input(int q, int has_offset, const MatvecArgs &a, const Fe
         case 8: return by_offset(std::integral_constant<int, 8>{});
         default: return hipErrorInvalidValue;
     }
+}
+
+template <FewInput IN, bool FINE>
+hipError_t launch_few_input(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t s)
+{
+    return by_planes(q, has_offset, [&](auto Qc, auto Off) { return launch_few_one<Qc, Off, IN, FINE>(a, g, waves, s); });
+}
+
+template <FewInput IN, bool FINE>
+hipError_t launch_few_list_input(int q, int has_offset, const MultiMatvecArgs &m, const FewGrid &g, int workgroups, int waves, hipStream_t s)
+{
+    return by_planes(q, has_offset, [&](auto Qc, auto Off) { return launch_few_list<Qc, Off, IN, FINE>(m, g, workgroups, waves, s); });
 }
 
 }  // namespace

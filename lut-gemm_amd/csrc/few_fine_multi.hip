@@ -1,0 +1,11 @@
+// The kernel for 3 to 16 activation rows (few_body.h) over a work list: instances for scale groups of 32 and 64 k, at most one row per wavefront.
+#include "few_body.h"
+
+namespace lutgemm_kernels {
+
+hipError_t launch_few_fine_multi(int q, int has_offset, const MultiMatvecArgs &m, const FewGrid &g, int workgroups, int waves, hipStream_t s)
+{
+    return launch_few_list_input<FewInput::kOneRow, true>(q, has_offset, m, g, workgroups, waves, s);
+}
+
+}  // namespace lutgemm_kernels

@@ -129,6 +129,12 @@ hipError_t launch_few_two_rows(int q, int has_offset, const MatvecArgs &a, const
 hipError_t launch_few_columns(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, hipStream_t stream);
 hipError_t launch_few_fine(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t stream);   // gsub > 1
 hipError_t launch_few_fine_two_rows(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, int waves, hipStream_t stream);
+// A work list of independent batches in one launch, as launch_batch_multi; sums of a k-split go through the accumulators
+// (g.partials null), and activations come as rows.
+hipError_t launch_few_multi(int q, int has_offset, const MultiMatvecArgs &m, const FewGrid &g, int workgroups, int waves, hipStream_t stream);
+hipError_t launch_few_multi_two_rows(int q, int has_offset, const MultiMatvecArgs &m, const FewGrid &g, int workgroups, int waves, hipStream_t stream);
+hipError_t launch_few_fine_multi(int q, int has_offset, const MultiMatvecArgs &m, const FewGrid &g, int workgroups, int waves, hipStream_t stream);
+hipError_t launch_few_fine_multi_two_rows(int q, int has_offset, const MultiMatvecArgs &m, const FewGrid &g, int workgroups, int waves, hipStream_t stream);
 hipError_t launch_few_fine_columns(int q, int has_offset, const MatvecArgs &a, const FewGrid &g, hipStream_t stream);
 
 // Many activation rows in one launch (rows_body.h): a workgroup of kRowsWaves wavefronts takes 16 rt rows and

@@ -65,6 +65,42 @@ def test_few_rows_non_finite_activations(lutgemm, device, q, g, offset):
     W.close()
 
 
+@pytest.mark.parametrize("q,g,offset,rows", [(1, 128, False, (3, 8, 5)), (2, 256, True, (16, 3, 9)), (3, 32, False, (8, 7, 4)),
+                                             (6, 64, True, (4, 16, 12)), (8, 128, False, (9, 16, 3))])
+def test_few_rows_work_list(lutgemm, oracle, device, q, g, offset, rows):
+    """Independent batches in one launch, with and without splits along k, one of odd width; a weight with an infinite scale
+    among them, which the batch kernel keeps, divides the list and has the results of its own call."""
+    import torch
+    from lutgemm import synth
+    shapes = [(1024, 300), (3072, 96), (512, 2049)]
+    made = [make(lutgemm, synth, k, n, q, g, offset=offset, seed=k + i) for i, (k, n) in enumerate(shapes)]
+    w_inf, _ = made[0]
+    alpha = np.array(w_inf["alpha"], dtype=np.float32)
+    alpha[0, 0, 5] = np.inf
+    W_inf = lutgemm.BCQWeight(w_inf["bW"], alpha, 1024, 300, q, 1024 // g, w_inf["q_bias"])
+    xs = [synth.make_x(m, k, seed=m) for (k, n), m in zip(shapes, rows)]
+    for with_inf in (False, True):
+        items = list(zip([W for _, W in made], xs, [n for _, n in shapes]))
+        if with_inf:
+            items.insert(1, (W_inf, xs[0], 300))
+        xd = [torch.from_numpy(x).to(device) for _, x, _ in items]
+        yd = [torch.zeros((x.shape[0], n), dtype=torch.float16, device=device) for _, x, n in items]
+        seq = lutgemm.MatvecSequence([(W, x.data_ptr(), y.data_ptr(), x.shape[0]) for (W, _, _), x, y in zip(items, xd, yd)])
+        say("case few rows list", q, g, offset, rows, "inf", with_inf, seq.fused_plan())
+        assert seq.fused_plan()["entries"] == (1 if with_inf else 3)
+        for _ in range(2):
+            seq.launch(torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            got = [y.cpu().numpy() for y in yd]
+            if with_inf:
+                assert np.array_equal(got[1].view(np.uint16), run_matvec(lutgemm, W_inf, xs[0], device).view(np.uint16))
+                del got[1]
+            for (w, _), x, y in zip(made, xs, got):
+                assert_within_tolerance(y, truth_of(oracle, w, x), "list, m=%d" % x.shape[0])
+    for W in [W for _, W in made] + [W_inf]:
+        W.close()
+
+
 def test_every_few_rows_instance(lutgemm):
     """Planes, inputs, wavefronts, splits along k and their sums that the plans of the sizes above do not reach."""
     program = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "few_test")
