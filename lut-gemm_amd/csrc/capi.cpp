@@ -506,7 +506,9 @@ size_t few_room(const lutgemm_weight *w)
 // behind the tiles in theirs.  Every hipMalloc costs 20 to 40 us and every hipFree, which waits for the device, about 80: with
 // one allocation instead of four, a 4096 x 16384 weight of four planes is made from host arrays, expanded and freed in 2190
 // instead of 2270 us, and as no room is allocated behind a launch the first call of 12 columns on a new 7168 x 28672 weight
-// takes 68 us instead of 124 (of 8 rows on the four weights of a 12288 block: 195 instead of 282).
+// takes 68 us instead of 124 (of 8 rows on the four weights of a 12288 block: 195 instead of 282).  Small weights lose a little, as
+// one piece of some MiB is no longer cut from the runtime's own chunks: 2048 x 2048, three planes, made and freed 147 -> 185 us;
+// 7168 x 7168 885 -> 830.
 constexpr size_t aligned256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 size_t words_bytes(const lutgemm_weight *w) { return aligned256(set_words(w) * sizeof(unsigned long long)); }
 size_t staging_bytes(const lutgemm_weight *w) { return aligned256((size_t)kStagedColumns * w->shape.k * sizeof(uint16_t)); }

@@ -253,7 +253,7 @@ class BCQWeight:
         return info
 
     def plan(self, m=1):
-        """Launch plan of calls with m activation rows (one-row, two-row or batch kernel)."""
+        """Launch plan of calls with m activation rows (the kernel that takes them)."""
         v = [ctypes.c_int() for _ in range(4)]
         _check(load().lutgemm_weight_plan_for(self._h, m, *[ctypes.byref(x) for x in v]))
         return dict(workgroups=v[0].value, waves=v[1].value, k_splits=v[2].value, k_blocks=v[3].value)

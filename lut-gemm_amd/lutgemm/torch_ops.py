@@ -13,7 +13,7 @@ lutGEMM/src/nQWeight_fp16.cu:93-99), the dense weight is rebuilt per call in a s
 by all layers (one per device and stream), so a layer never holds more than its packed weight;
 `keep_dense=True` keeps a private dense copy instead (2 k n bytes) and skips the rebuild.  Up to
 the threshold the library streams the packed weight
-(one or two rows through the table-lookup kernels, 3 to 16 through the batch kernel, more through the kernel
+(one or two rows through the table-lookup kernels, 3 to 16 through the kernel for few rows, more through the kernel
 for many rows).  The default threshold depends on the weight and on keep_dense (default_dense_threshold):
 it is where the two routes met when measured on MI355X.
 """
@@ -31,7 +31,7 @@ def default_dense_threshold(weight, keep_dense=False):
     (keep_dense) pays the GEMM alone: 32 rows for one or two planes, 16 for three to seven, and
     eight planes leave the packed route from three rows on (57 against 50 us).
 
-    More than 16 rows no longer take passes of 16, so the packed route would stay ahead for longer (12288 x 12288,
+    3 to 16 rows take less by now (kernel for few rows) and more no longer take passes of 16, so the packed route would stay ahead for longer (12288 x 12288,
     three planes, 160 rows: 130 against 192 us).  The lines are kept all the same (those of layers
     with a dense copy rest on passes of 16 rows as well), because the routes are not
     interchangeable: the dense one passes gradients to x, follows autocast, can be captured on a stream that has not
