@@ -79,8 +79,8 @@ struct StreamSet {
     size_t few_units;
     float *partials[kRoomSizes]; // the same for launches of more rows, and where few_units are too few: [c] holds 2^c units,
     bool no_room;                //   from the first launch that needs it on; an allocation failed: none is tried again
-    void *block;                 // the allocation that holds accum, the first xrows and few_partials (null in set 0: the
-    bool xrows_grown;            //   tiles' block); xrows is an allocation of its own
+    void *block;                 // the allocation that holds accum, the first xrows and few_partials (null in set 0 if
+    bool xrows_grown;            //   they lie behind the sign tiles); xrows is an allocation of its own
     hipEvent_t done;             // recorded behind the set's latest launch (only while done_valid)
     bool done_valid;
     unsigned long long last_use;
@@ -91,7 +91,8 @@ struct lutgemm_weight {
     Shape shape;
     int device;
     int compute_units;
-    uint8_t *d_signs;             // one allocation: the sign tiles, the scale tiles, the memory of set 0
+    uint8_t *d_signs;             // one allocation: the sign tiles, the scale tiles, the memory of set 0; small sign tiles have
+                                  // one of their own, and the rest is set 0's block (new_handle)
     uint16_t *d_scales;
     bool finite_scales;           // no infinity or NaN among the scales and offsets
     std::mutex slot_mutex;
@@ -506,9 +507,10 @@ size_t few_room(const lutgemm_weight *w)
 // behind the tiles in theirs.  Every hipMalloc costs 20 to 40 us and every hipFree, which waits for the device, about 80: with
 // one allocation instead of four, a 4096 x 16384 weight of four planes is made from host arrays, expanded and freed in 2190
 // instead of 2270 us, and as no room is allocated behind a launch the first call of 12 columns on a new 7168 x 28672 weight
-// takes 68 us instead of 124 (of 8 rows on the four weights of a 12288 block: 195 instead of 282).  Small weights lose a little, as
-// one piece of some MiB is no longer cut from the runtime's own chunks: 2048 x 2048, three planes, made and freed 147 -> 185 us;
-// 7168 x 7168 885 -> 830.
+// takes 68 us instead of 124 (of 8 rows on the four weights of a 12288 block: 195 instead of 282).  Pieces below
+// kRuntimeChunk cost next to nothing, as the runtime cuts them from chunks of its own: sign tiles that are such a piece stay
+// one where all together would not be (2048 x 2048, three planes, made, expanded and freed: 185 us, in one allocation 227, in four 187).
+constexpr size_t kRuntimeChunk = (size_t)2 << 20;
 constexpr size_t aligned256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 size_t words_bytes(const lutgemm_weight *w) { return aligned256(set_words(w) * sizeof(unsigned long long)); }
 size_t staging_bytes(const lutgemm_weight *w) { return aligned256((size_t)kStagedColumns * w->shape.k * sizeof(uint16_t)); }
@@ -757,11 +759,19 @@ int new_handle(const Shape &s, lutgemm_weight **out)
     if (few_shape(s))
         for (int i = 0; i < 2; i++) w->plan_few[i] = choose_few_plan(s, w->compute_units, i ? kRowsPerPass : 8);
     const size_t signs = aligned256(sign_bytes(s)), scales = aligned256(scale_bytes(s));
+    const size_t set0 = words_bytes(w) + staging_bytes(w) + few_room(w) * kPartialUnitBytes;
+    const bool apart = signs < kRuntimeChunk && signs + scales + set0 >= kRuntimeChunk;
     char *block = nullptr;
-    int st = alloc_block(w, signs + scales, &w->set[0], &block);
+    int st = LUTGEMM_OK;
+    if (apart) {
+        e = hipMalloc((void **)&w->d_signs, signs);
+        if (e != hipSuccess) st = hip_fail(e, "hipMalloc(signs)");
+    }
+    if (st == LUTGEMM_OK) st = alloc_block(w, (apart ? 0 : signs) + scales, &w->set[0], &block);
     if (st == LUTGEMM_OK) {
-        w->d_signs = reinterpret_cast<uint8_t *>(block);
-        w->d_scales = reinterpret_cast<uint16_t *>(block + signs);
+        if (apart) w->set[0].block = block;
+        else w->d_signs = reinterpret_cast<uint8_t *>(block);
+        w->d_scales = reinterpret_cast<uint16_t *>(block + (apart ? 0 : signs));
         st = alloc_set(w, 0, nullptr);   // check_scales waits for the null stream before any stream can launch on the handle
     }
     if (st != LUTGEMM_OK) {
