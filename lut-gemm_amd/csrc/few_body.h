@@ -15,7 +15,11 @@
 //    ahead, they were waited for: 12288 x 12288, two planes, groups of 64, 8 rows 20.0 us, now 17.4.
 //  * Activations and tiles come by buffer loads: an offset beyond the weight's k reads zero, and addresses are scalar.
 //  * Sums of a k-split go through memory (sum_partials): eight 64-bit atomics per lane took 3.5 to 5 us of a launch.
-// Products of two fp16 numbers are exact in the fp32 sums, so a result differs from the batch kernel's by fp32 rounding.
+// Products of two fp16 numbers are exact in the fp32 sums, so a result differs from the batch kernel's by fp32 rounding.  All planes
+// of an output share one accumulator: codes off the middle of their range and activations with a mean make plane sums that only
+// cancel together.  With an accumulator per plane parity both grew over a workgroup's k and lost the bits of their difference (k = 49152,
+// four planes and offset, codes around 4 of 15, x around 1: 33 % of the results not the nearest fp16 number, 1.3 % now, 2.9 % in the
+// batch kernel), and the distance of two uses that it gave was not needed (block of 12288 at 8 rows 134.7 us, now 133.9).
 // What bounds it now: power.  With the weight stream taken away the loop runs at the 10.7 ns a matrix instruction takes when all
 // compute units issue nothing else (6.9 ns on a few of them); the stream comes on top.  Measured (us, batch kernel -> this one, the
 // better plan of each): 12288 x 12288, two planes, 8 rows 20.3 -> 18.3; n = 36864 45.2 -> 36.4; n = 49152 50.1 -> 45.8; k = 49152
@@ -223,8 +227,8 @@ __device__ __forceinline__ void few_workgroup(const MatvecArgs &a, const FewGrid
         });
     };
 
-    float4v acc[2][2];   // output half, plane % 2
-    static_for<4>([&](auto I) { acc[I % 2][I / 2] = float4v{0.f, 0.f, 0.f, 0.f}; });
+    float4v acc[2];   // output half: every plane's products, so that they cancel where the planes do (the top of this file)
+    static_for<2>([&](auto H) { acc[H] = float4v{0.f, 0.f, 0.f, 0.f}; });
     const lds_byte *xlane = lds + kappa * kFewGroup + j * kFewPitch;
     uint32_t mask55 = 0x55555555u, high88 = 0x88888888u;   // in registers, so that the mask and the OR are one v_and_or_b32
     asm("" : "+s"(mask55));
@@ -312,7 +316,7 @@ __device__ __forceinline__ void few_workgroup(const MatvecArgs &a, const FewGrid
                     constexpr int b = b0 + U / 2;
                     if constexpr (b < P) {
                         const int picks = b < Q ? (int)index[pair % 2][U] : kAlwaysPlus;
-                        acc[U % 2][b % 2] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(A[U], B[step % (AHEAD + 1)], acc[U % 2][b % 2], picks, 0, hh);
+                        acc[U % 2] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(A[U], B[step % (AHEAD + 1)], acc[U % 2], picks, 0, hh);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                     // behind it one instruction of the next pair's indices: two per unit for odd k, one for even k
@@ -336,19 +340,18 @@ __device__ __forceinline__ void few_workgroup(const MatvecArgs &a, const FewGrid
         buf ^= 1;
     }
 
-    static_for<2>([&](auto H) { acc[H][0] += acc[H][1]; });
     __half *y = reinterpret_cast<__half *>(a.y);
     const __half *bias = static_cast<const __half *>(g.bias);
     if (a.k_splits > 1 && !g.partials) {
         // One atomic per value.  Each 16 x 16 tile is turned through the staging area first, so that the lanes hold the outputs of
-        // a row side by side (one cache line per row): acc[h][0][v] becomes activation row 4 kappa + v, output 16 h + j.
+        // a row side by side (one cache line per row): acc[h][v] becomes activation row 4 kappa + v, output 16 h + j.
         typedef __attribute__((address_space(3))) float lds_float;
         lds_float *turn = reinterpret_cast<lds_float *>(stage);
         static_for<2>([&](auto H) {
             asm volatile("" ::: "memory");   // the reads before are done with (LDS operations of a wavefront execute in order)
-            static_for<4>([&](auto V) { turn[(4 * kappa + V) * 16 + j] = acc[H][0][(int)V]; });
+            static_for<4>([&](auto V) { turn[(4 * kappa + V) * 16 + j] = acc[H][(int)V]; });
             asm volatile("" ::: "memory");
-            acc[H][0] = *reinterpret_cast<__attribute__((address_space(3))) float4v *>(turn + j * 16 + 4 * kappa);
+            acc[H] = *reinterpret_cast<__attribute__((address_space(3))) float4v *>(turn + j * 16 + 4 * kappa);
         });
         Arrival arrival[8];
         bool valid[8];
@@ -357,7 +360,7 @@ __device__ __forceinline__ void few_workgroup(const MatvecArgs &a, const FewGrid
             const int row = 4 * kappa + I % 4, out = nb * kBatch + 16 * (I / 4) + j;
             valid[I] = active && row < a.rows && out < a.n;
             word[I] = a.accum + (size_t)row * a.accum_row_stride + out;
-            arrival[I] = arrive_output(acc[I / 4][0][I % 4], valid[I], word[I]);
+            arrival[I] = arrive_output(acc[I / 4][I % 4], valid[I], word[I]);
         });
         // all answers are looked at before the first output is stored: a wait behind a store would wait for the store as well
         unsigned last = 0;
@@ -371,15 +374,15 @@ __device__ __forceinline__ void few_workgroup(const MatvecArgs &a, const FewGrid
         });
         return;
     }
-    // acc[h][0][v]: activation row j, output nb * 32 + 16 h + 4 kappa + v
+    // acc[h][v]: activation row j, output nb * 32 + 16 h + 4 kappa + v
     if (!active || j >= a.rows) return;
     if (a.k_splits > 1 &&
         !sum_partials<2>(g.partials + (size_t)nb * a.k_splits * 512, reinterpret_cast<unsigned *>(a.accum + nb), ks, a.k_splits, lane,
-                         [&](auto I) -> float4v & { return acc[I][0]; }))
+                         [&](auto I) -> float4v & { return acc[I]; }))
         return;
     static_for<2>([&](auto H) {
         const int out = nb * kBatch + 16 * H + 4 * kappa;
-        float4v &v = acc[H][0];
+        float4v &v = acc[H];
         if (bias)
             static_for<4>([&](auto V) {
                 if (out + V < a.n) v[(int)V] = plus_bias(v[(int)V], __half2float(bias[out + V]));

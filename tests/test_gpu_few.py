@@ -65,6 +65,36 @@ def test_few_rows_non_finite_activations(lutgemm, device, q, g, offset):
     W.close()
 
 
+@pytest.mark.parametrize("k,n,q,g", [(12288, 32768, 4, 128), (12288, 32768, 3, 128), (12288, 32768, 4, 64), (12288, 32768, 4, 32),
+                                     (12288, 16384, 6, 128)])
+def test_few_rows_planes_that_cancel(lutgemm, device, k, n, q, g):
+    """Every code is the weight zero (uniform codes around an offset), the activations have a mean: the planes' sums are large and
+    cancel exactly, so a result is the rounding of the sums.  A matrix instruction rounds its 64 products and the sum so far,
+    which is at most what all planes add up to between two cancellations: a step of 64 k, or a k-block of 512 where five
+    planes and more take two passes over it.  A rounding is within half a unit in the last place (2^-24 of that), its deviation
+    1 / sqrt(3) of it, and 1 / 3 as the sum grows from nothing; independent ones add up by the root of their number.  The bound is
+    six of these deviations, for 16 n results."""
+    step, code = 2.0 ** -7, 4
+    signs = [code >> b & 1 for b in range(q)]
+    alpha = np.array([step * 2 ** b / 2 for b in range(q)], dtype=np.float32)
+    offset = -sum(a if s else -a for a, s in zip(alpha, signs))
+    bW = np.empty((k // 32, q, n), dtype=np.uint32)
+    for b in range(q):
+        bW[:, b] = 0xffffffff if signs[b] else 0
+    W = lutgemm.BCQWeight(bW, np.broadcast_to(alpha[None, :, None], (k // g, q, n)).copy(), k, n, q, k // g,
+                          np.full((k // g, n), offset, dtype=np.float32))
+    x = (np.random.default_rng(k + q).standard_normal((16, k)) + 1).astype(np.float16)
+    window = 64 if q + 1 <= 4 else 512
+    most = float(alpha.sum() + abs(offset)) * np.abs(x.astype(np.float64)).reshape(16, -1, window).sum(2).max()
+    bound = 2 * 2.0 ** -24 * most * np.sqrt(k / 64 * (q + 1))
+    for m in (8, 16):
+        say("case few rows planes that cancel", k, n, q, g, "m", m, W.plan(m), "bound", bound)
+        worst = float(np.abs(run_matvec(lutgemm, W, x[:m], device).astype(np.float64)).max())
+        say("largest", worst)
+        assert worst <= bound, (m, worst, bound)
+    W.close()
+
+
 @pytest.mark.parametrize("q,g,offset,rows", [(1, 128, False, (3, 8, 5)), (2, 256, True, (16, 3, 9)), (3, 32, False, (8, 7, 4)),
                                              (6, 64, True, (4, 16, 12)), (8, 128, False, (9, 16, 3))])
 def test_few_rows_work_list(lutgemm, oracle, device, q, g, offset, rows):
