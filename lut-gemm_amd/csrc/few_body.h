@@ -13,7 +13,9 @@
 //  * With scale groups of 32 and 64 k (FINE) a lane's operands change from word to word.  The scales of a tile are 1 KiB per plane;
 //    they go through LDS, loaded a k-block ahead, and an operand is made anew behind its last use.  Loaded word by word, a word
 //    ahead, they were waited for: 12288 x 12288, two planes, groups of 64, 8 rows 20.0 us, now 17.4.
-//  * Activations and tiles come by buffer loads: an offset beyond the weight's k reads zero, and addresses are scalar.
+//  * Activations and tiles come by buffer loads: an offset beyond the weight's k reads zero, and addresses are scalar.  The bounds
+//    check covers the vector and the immediate offset and is not promised for the scalar one, so what may lie beyond k has no scalar
+//    offset (12 columns of 7168 x 28672: 29.6 us with and without it).
 //  * Sums of a k-split go through memory (sum_partials): eight 64-bit atomics per lane took 3.5 to 5 us of a launch.
 // Products of two fp16 numbers are exact in the fp32 sums, so a result differs from the batch kernel's by fp32 rounding.  All planes
 // of an output share one accumulator: codes off the middle of their range and activations with a mean make plane sums that only
@@ -205,7 +207,7 @@ __device__ __forceinline__ void few_workgroup(const MatvecArgs &a, const FewGrid
     auto load_pieces = [&]() {
         if constexpr (COLS) {
             static_for<NP>([&](auto I) {
-                if (I < a.rows) half_of[I] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(x_rsrc, (int)x_off, I * 1024, 0);
+                if (I < a.rows) half_of[I] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(x_rsrc, (int)x_off + I * 1024, 0, 0);
             });
             x_off += (uint32_t)(kBlockK * 2) * (uint32_t)a.rows;
         } else {

@@ -65,6 +65,27 @@ def test_few_rows_non_finite_activations(lutgemm, device, q, g, offset):
     W.close()
 
 
+@pytest.mark.parametrize("k,n,q,g,offset", [(1120, 4104, 2, 32, True), (640, 300, 3, 128, False), (4160, 96, 4, 64, False), (32, 40, 6, 32, True)])
+def test_few_columns_end_at_k(lutgemm, device, k, n, q, g, offset):
+    """k ends within a k-block and NaNs follow the last column of x: they must not be read, neither as part of the block nor as what
+    the zero scales of the tile's padding are multiplied with."""
+    import torch
+    from lutgemm import synth
+    _, W = make(lutgemm, synth, k, n, q, g, offset=offset, seed=k)
+    x = synth.make_x(16, k, seed=n)
+    for m in (3, 7, 8, 12, 16):
+        say("case few columns end at k", k, n, q, g, offset, "m", m, W.plan(m))
+        assert W.plan(m)["waves"] == 8   # read as they are
+        rows = run_matvec(lutgemm, W, x[:m], device)
+        xd = torch.full((k * m + 16384,), float("nan"), dtype=torch.float16, device=device)
+        xd[:k * m] = torch.from_numpy(np.ascontiguousarray(x[:m].T).reshape(-1)).to(device)
+        yd = torch.zeros((n, m), dtype=torch.float16, device=device)
+        W.matvec_cols(xd.data_ptr(), yd.data_ptr(), m, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert np.array_equal(yd.cpu().numpy().T.view(np.uint16), rows.view(np.uint16))
+    W.close()
+
+
 @pytest.mark.parametrize("k,n,q,g", [(12288, 32768, 4, 128), (12288, 32768, 3, 128), (12288, 32768, 4, 64), (12288, 32768, 4, 32),
                                      (12288, 16384, 6, 128)])
 def test_few_rows_planes_that_cancel(lutgemm, device, k, n, q, g):
