@@ -1238,8 +1238,8 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
 }
 
 // ---- runs of independent entries that share one launch (lutgemm_matvec_many) ----------------
-// kind: 1 one-row entries, 3 two-row entries (table-lookup kernels), 2 batches of 3 to 16 rows (the
-// batch kernel); an entry of more than 16 rows is launched on its own.
+// kind: 1 one-row entries, 3 two-row entries (table-lookup kernels), 4 and 2 batches of 3 to 16 rows (the
+// kernel for few rows and the batch kernel); an entry of more than 16 rows is launched on its own.
 struct FusedRun {
     int kind, count;
     lutgemm_kernels::MultiMatvecArgs multi;
@@ -1256,12 +1256,12 @@ int fused_kind(int m)
     return 0;
 }
 
-// kind 4: the kernel for few rows takes the batches (39 lists of 2 to 12 entries, k and n 512 to 49152, one to eight planes, 3 to 16
-// rows: 0.68 to 1.04 of the batch kernel's time, 0.89 on average)
+// kind 4: the kernel for few rows takes the batches that it takes as single calls (39 lists of 2 to 12 entries, k and n 512 to
+// 49152, one to eight planes, 3 to 16 rows: 0.68 to 1.04 of the batch kernel's time, 0.89 on average).  The batch kernel keeps the
+// others: a list of weights with non-finite scales or with plans that the caller has set for it.
 int fused_kind(const lutgemm_weight *w, int m)
 {
-    const int kind = fused_kind(m);
-    return kind == 2 && few_shape(w->shape) && w->finite_scales ? 4 : kind;
+    return takes_few_kernel(w, m) ? 4 : fused_kind(m);
 }
 
 // Longest run of entries starting at i that one launch can take: the same kind and kernel

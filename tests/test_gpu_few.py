@@ -152,6 +152,55 @@ def test_few_rows_work_list(lutgemm, oracle, device, q, g, offset, rows):
         W.close()
 
 
+@pytest.mark.parametrize("infinite", [False, True])
+@pytest.mark.parametrize("q,g,offset,rows", [(1, 128, True, (3, 8, 16)), (2, 64, False, (16, 5, 9)), (3, 32, False, (8, 9, 4)), (4, 32, True, (4, 16, 12)),
+                                             (6, 128, True, (9, 3, 16)), (8, 64, False, (12, 4, 7)), (5, 32, True, (3, 16, 8))])
+def test_work_list_of_the_batch_kernel(lutgemm, oracle, device, q, g, offset, rows, infinite):
+    """Weights with a plan set for the batch kernel, and weights with infinite scales, share launches of it: results are those of
+    single calls with the list's split along k bit for bit, so that a NaN or an infinity stays with its output."""
+    import torch
+    from lutgemm import synth
+    st = torch.cuda.current_stream().cuda_stream
+    items = []
+    for i, ((k, n), m) in enumerate(zip([(1024, 300), (4096, 96), (512, 2049)], rows)):
+        w = synth.make_weight(k, n, q, g, offset=offset, seed=k + i)
+        alpha = np.array(w["alpha"], dtype=np.float32)
+        if infinite:
+            alpha[0, q - 1, 5] = np.inf if i else -np.inf
+        W = lutgemm.BCQWeight(w["bW"], alpha, k, n, q, k // g, w["q_bias"])
+        if not infinite:
+            W.set_batch_plan(8, 1)
+        x = synth.make_x(m, k, seed=m)
+        items.append((w, W, x, torch.from_numpy(x).to(device), torch.zeros((m, n), dtype=torch.float16, device=device)))
+    seq = lutgemm.MatvecSequence([(W, xd.data_ptr(), yd.data_ptr(), xd.shape[0]) for _, W, _, xd, yd in items])
+    plan = seq.fused_plan()
+    say("case list of the batch kernel", q, g, offset, rows, infinite, plan)
+    assert plan["entries"] == 3
+    seq.launch(st)
+    torch.cuda.synchronize()
+    first = [yd.cpu().numpy() for *_, yd in items]
+    seq.launch(st)
+    torch.cuda.synchronize()
+    for (w, W, x, _, yd), y in zip(items, first):
+        n = y.shape[1]
+        assert np.array_equal(yd.cpu().numpy().view(np.uint16), y.view(np.uint16))
+        blocks = -(-W.kSize // 512)
+        per_split = min(plan["k_blocks"], blocks)
+        splits = -(-blocks // per_split)
+        assert -(-blocks // splits) == per_split, "a split that single calls can be given"
+        W.set_batch_plan(8, splits)
+        single = run_matvec(lutgemm, W, x, device)
+        finite = np.delete(np.arange(n), 5) if infinite else np.arange(n)
+        assert np.array_equal(y[:, finite].view(np.uint16), single[:, finite].view(np.uint16))
+        assert_within_tolerance(y[:, finite], truth_of(oracle, w, x)[:, finite], "list, m=%d" % x.shape[0])
+        if infinite:
+            assert not np.isfinite(y[:, 5]).any()
+            assert np.array_equal(np.isnan(y[:, 5]), np.isnan(single[:, 5]))
+            whole = ~np.isnan(single[:, 5])
+            assert np.array_equal(y[whole, 5], single[whole, 5])
+        W.close()
+
+
 def test_every_few_rows_instance(lutgemm):
     """Planes, inputs, wavefronts, splits along k and their sums that the plans of the sizes above do not reach."""
     program = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "few_test")
