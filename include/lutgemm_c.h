@@ -150,7 +150,9 @@ int lutgemm_matvec_static(const lutgemm_weight *w, const void *x, void *y, int m
  * Replaces lutGEMM::matmul(void* output, nQWeight_fp16&, void* input, int n, int algo)
  * (lutGEMM/include/kernels.h:26, lutGEMM/src/kernels.cu:56-63).  For m == 1 it is the same
  * operation as lutgemm_matvec.  For m > 1 the columns are first gathered into staging rows owned
- * by the handle (one buffer per launching stream).  Up to m = 16 nothing is allocated; a larger m
+ * by the handle (one buffer per launching stream), or, 3 to 16 of them with plans of 8 wavefronts per workgroup
+ * (lutgemm_weight_plan_for), read where they lie.  y may overlap x for m > 1: such a call always gathers.
+ * Up to m = 16 nothing is allocated; a larger m
  * grows the stream's buffer the first time it occurs (synchronises that stream, frees, allocates). */
 int lutgemm_matvec_cols(const lutgemm_weight *w, const void *x, void *y, int m, void *stream);
 

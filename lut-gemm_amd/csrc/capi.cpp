@@ -1093,10 +1093,13 @@ int run_matvec(const lutgemm_weight *w, const void *x, void *y, int m, void *str
         lease.stream = stream;
         a.accum = mw->set[slot].accum;
     }
-    // few rows (few_body.h); workgroups of kFewWavesMin wavefronts read columns as they are
+    // few rows (few_body.h); workgroups of kFewWavesMin wavefronts read columns as they are, unless y lies over x: some workgroups
+    // store results while others still read, and a call in place needs all of x gathered first
     const bool few = takes_few_kernel(w, m);
     const Plan few_plan = few ? w->plan_few[m > 8] : Plan{};
-    const bool few_columns = few && cols && few_plan.waves == lutgemm_kernels::kFewWavesMin;
+    const uintptr_t x0 = (uintptr_t)x, y0 = (uintptr_t)y;
+    const bool in_place = x0 < y0 + (size_t)m * s.n * sizeof(uint16_t) && y0 < x0 + (size_t)m * s.k * sizeof(uint16_t);
+    const bool few_columns = few && cols && few_plan.waves == lutgemm_kernels::kFewWavesMin && !in_place;
     if (cols && m > 1 && !few_columns) {
         // gather the m columns into contiguous rows first (the kernel reads 16 bytes per lane); the
         // staging rows belong to the stream's set, or, for the allocation-free entry point, to set 0

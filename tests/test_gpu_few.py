@@ -86,6 +86,32 @@ def test_few_columns_end_at_k(lutgemm, device, k, n, q, g, offset):
     W.close()
 
 
+@pytest.mark.parametrize("k,n,q,g,offset", [(4096, 4096, 3, 128, False), (2048, 8192, 2, 64, True), (7168, 1024, 4, 32, False)])
+def test_columns_in_place(lutgemm, device, k, n, q, g, offset):
+    """y over x: the results of a call into another buffer, bit for bit, however the two overlap."""
+    import torch
+    from lutgemm import synth
+    _, W = make(lutgemm, synth, k, n, q, g, offset=offset, seed=k)
+    st = torch.cuda.current_stream().cuda_stream
+    direct = 0
+    for m in (2, 3, 8, 16, 20):
+        direct += 3 <= m <= 16 and W.plan(m)["waves"] == 8   # read where they lie into another buffer
+        x = torch.from_numpy(np.ascontiguousarray(synth.make_x(m, k, seed=m).T)).to(device).reshape(-1)
+        apart = torch.zeros(n * m, dtype=torch.float16, device=device)
+        W.matvec_cols(x.data_ptr(), apart.data_ptr(), m, st)
+        for x_at, y_at in ((0, 0), (0, 128 * m), (64 * m, 0), (0, (k - 1) * m + m - 1), ((n - 8) * m, 0)):
+            say("case columns in place", k, n, q, g, offset, "m", m, "x at", x_at, "y at", y_at, W.plan(m))
+            both = torch.zeros(max(x_at + k * m, y_at + n * m), dtype=torch.float16, device=device)
+            xv, yv = both[x_at:x_at + k * m], both[y_at:y_at + n * m]
+            assert xv.data_ptr() % 16 == 0
+            xv.copy_(x)
+            W.matvec_cols(xv.data_ptr(), yv.data_ptr(), m, st)
+            torch.cuda.synchronize()
+            assert torch.equal(yv.view(torch.int16), apart.view(torch.int16))
+    assert direct
+    W.close()
+
+
 @pytest.mark.parametrize("k,n,q,g", [(12288, 32768, 4, 128), (12288, 32768, 3, 128), (12288, 32768, 4, 64), (12288, 32768, 4, 32),
                                      (12288, 16384, 6, 128)])
 def test_few_rows_planes_that_cancel(lutgemm, device, k, n, q, g):
