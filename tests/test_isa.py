@@ -1,5 +1,5 @@
-"""What the compiler made of the batch kernel and of the kernel for many rows, checked on the generated gfx950 assembly of the
-library's own translation units (no GPU needed: hipcc cross-compiles; about a minute).  The hot
+"""What the compiler made of the batch kernel and of the kernels for few and for many rows, checked on the generated gfx950 assembly
+of the library's own translation units (no GPU needed: hipcc cross-compiles; three minutes on eight cores).  The hot
 loop and the end of a workgroup depend on properties the source can only ask for: the
 transposition done by the LDS, the matrix instructions present, the index and the scale
 multiply-add in one instruction each, no packed fp32 forms, no register used while an LDS read
@@ -10,6 +10,7 @@ launch 1.5 to 2 microseconds when the compiler once arranged the code that way).
 import os
 import re
 import subprocess
+from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 
@@ -18,24 +19,28 @@ CSRC = os.path.join(ROOT, "lut-gemm_amd", "csrc")
 
 
 ROWS_SOURCES = [("rows.hip", 1), ("rows_two_groups.hip", 2)]   # k groups
+FEW_SOURCES = [("few%s%s%s.hip" % (fine, multi, way), "lut_few%s_kernel" % multi, inputs, bool(fine))   # inputs: FewInput (few_body.h)
+               for fine in ("", "_fine") for multi in ("", "_multi") for inputs, way in enumerate(("", "_two_rows", "_columns"))
+               if not (multi and way == "_columns")]
 SOURCES = [("batch.hip", "lut_batch_kernel", "10MatvecArgs"), ("batch_multi.hip", "lut_batch_multi_kernel", "15MultiMatvecArgs")]
 
 
 @pytest.fixture(scope="module")
 def assembly(tmp_path_factory):
-    """gfx950 assembly of the translation units of the two kernels, compiled side by side."""
+    """gfx950 assembly of the translation units of these kernels, compiled side by side."""
     out_dir = tmp_path_factory.mktemp("isa")
-    jobs = {}
-    for source in [s[0] for s in SOURCES + ROWS_SOURCES]:
+
+    def compiled(source):
         out = os.path.join(str(out_dir), source + ".s")
         cmd = ["/opt/rocm/bin/hipcc", "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-Xclang", "-target-feature",
                "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument", "-I", CSRC, "-S", "--cuda-device-only",
                "-o", out, os.path.join(CSRC, source)]
-        jobs[source] = (subprocess.Popen(cmd, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL), out)
-    texts = {}
-    for source, (proc, out) in jobs.items():
-        assert proc.wait() == 0, source
-        texts[source] = open(out).read()
+        assert subprocess.run(cmd, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL).returncode == 0, source
+        return open(out).read()
+
+    sources = [s[0] for s in SOURCES + ROWS_SOURCES + FEW_SOURCES]
+    with ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
+        texts = dict(zip(sources, pool.map(compiled, sources)))
     return texts
 
 
@@ -154,9 +159,9 @@ def test_batch_kernel_assembly(assembly, source, kernel, args):
     assert re.search(r"\.amdhsa_private_segment_fixed_size 0\b", meta)
 
 
-# register spills of the kernel for many rows (scratch memory per lane, bytes): only with four row tiles (96 registers
-# of sums and activations) and six planes or more
-MAX_ROWS_SCRATCH_BYTES = {(8, 4, 1): 40, (6, 4, 2): 12, (7, 4, 2): 88, (8, 4, 2): 144, (9, 4, 2): 80}
+# register spills of the kernel for many rows (scratch memory per lane, bytes): one instance of eight planes and four row tiles
+# (96 registers of sums and activations)
+MAX_ROWS_SCRATCH_BYTES = {(8, 4, 2): 36}
 
 
 @pytest.mark.parametrize("source,groups", ROWS_SOURCES)
@@ -177,3 +182,25 @@ def test_rows_kernel_assembly(assembly, source, groups):
         assert not any(op.startswith(("v_pk_add_f32", "v_pk_mul_f32", "v_pk_fma_f32")) for op in ops), instance
         scratch = int(re.search(r"\.amdhsa_private_segment_fixed_size (\d+)", meta).group(1))
         assert scratch <= MAX_ROWS_SCRATCH_BYTES.get(instance, 0), (instance, scratch)
+
+
+@pytest.mark.parametrize("source,kernel,inputs,fine", FEW_SOURCES)
+def test_few_kernel_assembly(assembly, source, kernel, inputs, fine):
+    text = assembly[source]
+    names = re.findall(r"^(_ZN\S*%sILi(\d)ELb(\d)ELNS0_8FewInputE(\d)ELb(\d)E\S*):" % kernel, text, re.M)
+    assert sorted(tuple(int(v) for v in n[1:]) for n in names) == [(q, o, inputs, fine) for q in range(1, 9) for o in (0, 1)]
+    for name, *args in names:
+        q, offset, _, _ = instance = tuple(int(v) for v in args)
+        planes = q + offset
+        body = text[text.index("\n%s:" % name):]
+        ops = [ln.split()[0] for ln in body[:body.index(".Lfunc_end")].splitlines() if re.match(r"\t[a-z]", ln)]
+        meta = text[text.index(".amdhsa_kernel " + name):]
+        meta = meta[:meta.index(".end_amdhsa_kernel")]
+        # up to 16, 12 or 8 wavefronts per workgroup (few_waves_max in kernels.h; columns: 8), a quarter of them on a SIMD of 512 registers
+        waves = 8 if inputs == 2 else {1: 16, 2: 12 if fine else 16, 3: 8 if fine else 12}.get(planes, 8)
+        assert int(re.search(r"\.amdhsa_next_free_vgpr (\d+)", meta).group(1)) <= {16: 128, 12: 168, 8: 256}[waves], instance
+        assert ops.count("ds_read_b64_tr_b8") == 4 * q, instance
+        assert ops.count("v_smfmac_f32_16x16x64_f16") == 32 * planes, instance
+        assert ops.count("v_and_or_b32") >= 16 * q, instance   # the index of a step pair: one instruction per sign word and parity
+        assert not any(op.startswith(("v_pk_add_f32", "v_pk_mul_f32", "v_pk_fma_f32")) for op in ops), instance
+        assert re.search(r"\.amdhsa_private_segment_fixed_size 0\b", meta), instance
