@@ -1,9 +1,9 @@
-// Every instance of the kernel for 3 to 16 rows (launch_few): planes, with and without an offset, scale groups of 128, 64 and 32 k, activations as rows (at most
+// Every instance of the kernel for 3 to 16 rows (launch_few, and launch_few_multi as a list of two batches): planes, with and without an offset, scale groups of 128, 64 and 32 k, activations as rows (at most
 // one and two per wavefront) and as columns, with and without splits along k, their sums by atomics and through memory, with a
 // partial output batch, group of batches and k-block; results in rows of 8-byte and of 2-byte stores and in columns, with
 // and without bias.  Results against double precision within the tolerance of the path (oracle/oracle.py), the same launch
 // twice bit for bit, the bias as an addition to the fp16 result bit for bit, nothing written behind the results, the words for
-// the splits back at zero, and columns with the bits of rows.
+// the splits back at zero, columns with the bits of rows, and the batches of a list with the bits of launches of their own.
 #include <hip/hip_runtime_api.h>
 
 #include <cmath>
@@ -43,39 +43,73 @@ T *to_device(const std::vector<T> &v)
     return p;
 }
 
-// y of one launch, element (row, output) at [row * n + output] whatever the layout on the device
+// device memory of a batch's results and sums
+struct Batch {
+    size_t count;
+    uint16_t *y;
+    unsigned long long *words;
+    float *partials;
+
+    Batch(lutgemm_kernels::MatvecArgs *a, bool y_cols) : count((size_t)a->rows * kN)
+    {
+        y = to_device(std::vector<uint16_t>(count + kGuard, 0x7e01));
+        words = to_device(std::vector<unsigned long long>((size_t)kMaxRows * kNb * 32));
+        HIP_OK(hipMalloc((void **)&partials, (size_t)kNb * a->k_splits * 512 * sizeof(float)));
+        a->y = y;
+        a->accum = words;
+        a->accum_row_stride = kNb * 32;
+        a->y_stride = y_cols ? a->rows : 1;
+        a->y_row_stride = y_cols ? 1 : kN;
+    }
+
+    // element (row, output) at [row * n + output] whatever the layout on the device; frees the memory
+    std::vector<_Float16> results(int rows, bool y_cols)
+    {
+        std::vector<uint16_t> filled(count + kGuard);
+        std::vector<unsigned long long> counts((size_t)kMaxRows * kNb * 32);
+        HIP_OK(hipMemcpy(filled.data(), y, filled.size() * 2, hipMemcpyDeviceToHost));
+        HIP_OK(hipMemcpy(counts.data(), words, counts.size() * 8, hipMemcpyDeviceToHost));
+        HIP_OK(hipFree(y));
+        HIP_OK(hipFree(words));
+        HIP_OK(hipFree(partials));
+        for (size_t i = count; i < filled.size(); i++)
+            if (filled[i] != 0x7e01) { printf("FAIL written behind the results\n"); exit(1); }
+        for (unsigned long long c : counts)
+            if (c) { printf("FAIL a word is not back at zero\n"); exit(1); }
+        std::vector<_Float16> out(count);
+        for (int r = 0; r < rows; r++)
+            for (int j = 0; j < kN; j++)
+                memcpy(&out[(size_t)r * kN + j], &filled[y_cols ? (size_t)j * rows + r : (size_t)r * kN + j], 2);
+        return out;
+    }
+};
+
+// y of one launch
 std::vector<_Float16> launch(int q, bool offset, int waves, bool atomics, lutgemm_kernels::MatvecArgs a, lutgemm_kernels::FewGrid g, bool y_cols)
 {
-    const size_t count = (size_t)a.rows * kN;
-    std::vector<uint16_t> filled(count + kGuard, 0x7e01);
-    uint16_t *y = to_device(filled);
-    std::vector<unsigned long long> zeros((size_t)kMaxRows * kNb * 32);
-    unsigned long long *words = to_device(zeros);
-    float *partials = nullptr;
-    HIP_OK(hipMalloc((void **)&partials, (size_t)kNb * a.k_splits * 512 * sizeof(float)));
-    a.y = y;
-    a.accum = words;
-    a.accum_row_stride = kNb * 32;
-    a.y_stride = y_cols ? a.rows : 1;
-    a.y_row_stride = y_cols ? 1 : kN;
-    g.partials = atomics ? nullptr : partials;
+    Batch batch(&a, y_cols);
+    g.partials = atomics ? nullptr : batch.partials;
     HIP_OK(hipDeviceSynchronize());
     HIP_OK(lutgemm_kernels::launch_few(q, offset, a, g, waves, nullptr));
     HIP_OK(hipDeviceSynchronize());
-    HIP_OK(hipMemcpy(filled.data(), y, filled.size() * 2, hipMemcpyDeviceToHost));
-    HIP_OK(hipMemcpy(zeros.data(), words, zeros.size() * 8, hipMemcpyDeviceToHost));
-    HIP_OK(hipFree(y));
-    HIP_OK(hipFree(words));
-    HIP_OK(hipFree(partials));
-    for (size_t i = count; i < filled.size(); i++)
-        if (filled[i] != 0x7e01) { printf("FAIL written behind the results\n"); exit(1); }
-    for (unsigned long long c : zeros)
-        if (c) { printf("FAIL a word is not back at zero\n"); exit(1); }
-    std::vector<_Float16> out(count);
-    for (int r = 0; r < a.rows; r++)
-        for (int j = 0; j < kN; j++)
-            memcpy(&out[(size_t)r * kN + j], &filled[y_cols ? (size_t)j * a.rows + r : (size_t)r * kN + j], 2);
-    return out;
+    return batch.results(a.rows, y_cols);
+}
+
+// A launch of a batch of `other` rows and one of a.rows as a list (sums by atomics); y of both, one behind the other
+std::vector<_Float16> launch_list(int q, bool offset, int waves, lutgemm_kernels::MatvecArgs a, const lutgemm_kernels::FewGrid &g, int other)
+{
+    lutgemm_kernels::MultiMatvecArgs list{};
+    list.count = 2;
+    list.entry[0] = list.entry[1] = a;
+    list.entry[0].rows = other;
+    list.first_block[1] = a.ntiles * a.k_splits;
+    Batch first(&list.entry[0], false), second(&list.entry[1], false);
+    HIP_OK(hipDeviceSynchronize());
+    HIP_OK(lutgemm_kernels::launch_few_multi(q, offset, list, g, 2 * a.ntiles * a.k_splits, waves, nullptr));
+    HIP_OK(hipDeviceSynchronize());
+    std::vector<_Float16> y = first.results(other, false), more = second.results(a.rows, false);
+    y.insert(y.end(), more.begin(), more.end());
+    return y;
 }
 
 void run_weight(int q, bool offset, int group, int *variant)
@@ -154,6 +188,20 @@ void run_weight(int q, bool offset, int group, int *variant)
                 g.bias = nullptr;
                 g.columns = 1;
                 const std::vector<_Float16> from_columns = launch(q, offset, lutgemm_kernels::kFewWavesMin, end, ac, g, y_cols);
+                if (end || a.k_splits == 1) {
+                    g.columns = 0;
+                    const int other = rows == 3 ? 8 : 24 - rows;   // lists with one row per wavefront at most and with two
+                    lutgemm_kernels::MatvecArgs alone = a;
+                    alone.rows = other;
+                    std::vector<_Float16> each = launch(q, offset, waves, true, alone, g, false);
+                    const std::vector<_Float16> last = y_cols ? launch(q, offset, waves, true, a, g, false) : y;
+                    each.insert(each.end(), last.begin(), last.end());
+                    const std::vector<_Float16> list = launch_list(q, offset, waves, a, g, other);
+                    if (list.size() != each.size() || memcmp(list.data(), each.data(), each.size() * 2)) {
+                        printf("FAIL the batches of a list are not those of launches of their own\n");
+                        exit(1);
+                    }
+                }
                 for (size_t i = 0; i < y.size(); i++) {
                     const double t = truth[i], m = std::fmax(std::fabs(t), std::ldexp(1.0, -14));
                     const double bound = 2 * std::ldexp(1.0, (int)std::floor(std::log2(m)) - 10) + 1e-3;
