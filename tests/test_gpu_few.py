@@ -235,3 +235,13 @@ def test_every_few_rows_instance(lutgemm):
     sys.stdout.write(r.stdout)
     sys.stderr.write(r.stderr)
     assert r.returncode == 0 and "FEW OK 960" in r.stdout
+
+
+def test_without_memory_for_partial_sums(lutgemm):
+    """Handles whose device refuses the room for the partial sums of 3 to 16 rows (room_test.cpp)."""
+    program = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "room_test")
+    assert os.path.exists(program), "build the C++ tests first (make -C tests/cpp, or __graft_entry__.build())"
+    r = subprocess.run([program], capture_output=True, text=True, timeout=110)
+    sys.stdout.write(r.stdout)
+    sys.stderr.write(r.stderr)
+    assert r.returncode == 0 and "ROOM OK" in r.stdout
