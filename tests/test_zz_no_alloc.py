@@ -1,7 +1,8 @@
 """The allocation-free entry point lutgemm_matvec_static (split-k words in a static device array)
 against lutgemm_matvec on the same inputs, through the C ABI: bit for bit, on calls in a row
-(three, two, one and nine activation rows: batch, two-row and one-row kernels), the second on a
-smaller weight than the first, so that words left behind by a call would show in the next."""
+(three, two, one and nine activation rows: the kernel for few rows, the two-row and the one-row kernel; the batch kernel where
+weights or plans choose it), the second on a smaller weight than the first, so that words left behind by a call would show in the
+next."""
 import ctypes
 import sys
 
@@ -76,4 +77,26 @@ def test_static_workspace_entry_point_matches_matvec_for_many_rows(lutgemm, devi
         want = run(lutgemm, W, x[:rows], device, static=False)
         got = run(lutgemm, W, x[:rows], device, static=True)
         assert np.array_equal(got.view(np.uint16), want.view(np.uint16)), rows
+    W.close()
+
+
+@pytest.mark.parametrize("infinite", [False, True])
+@pytest.mark.parametrize("k,n,q,g,off", [(8192, 500, 3, 128, True), (4096, 2080, 2, 32, False), (2048, 700, 6, 64, True)])
+def test_static_workspace_entry_point_matches_matvec_for_the_batch_kernel(lutgemm, device, k, n, q, g, off, infinite):
+    """Weights with an infinite scale, and a plan set for the batch kernel: 3 to 16 rows and passes of 16, bit for bit."""
+    from lutgemm import synth
+    w = synth.make_weight(k, n, q, g, offset=off, seed=k + n)
+    alpha = w["alpha"].copy()
+    if infinite:
+        alpha[0, 0, 5] = np.inf
+    W = lutgemm.BCQWeight(w["bW"], alpha, k, n, q, k // g, w["q_bias"])
+    if not infinite:
+        W.set_batch_plan(8, 4)
+    x = synth.make_x(40, k, seed=n)
+    for rows in (3, 9, 40, 16):
+        print("case static batch kernel", k, n, q, g, off, infinite, rows, W.plan(rows), flush=True)
+        want = run(lutgemm, W, x[:rows], device, static=False)
+        got = run(lutgemm, W, x[:rows], device, static=True)
+        assert np.array_equal(got.view(np.uint16), want.view(np.uint16)), rows
+        assert np.isfinite(np.delete(want, 5, axis=1)).all() and np.isfinite(want[:, 5]).all() != infinite
     W.close()
