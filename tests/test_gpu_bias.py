@@ -9,8 +9,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("k,n,q,g,offset", [(512, 40, 3, 128, False), (4096, 70, 2, 64, True), (1024, 1001, 5, 32, False)])
 def test_bias_on_every_kernel(lutgemm, oracle, device, k, n, q, g, offset):
-    """One row, two rows, the batch kernel (17 and 40 rows too where its plan is set) and the kernel for many rows, with
-    and without splits along k: the result without bias plus the bias in fp16, bit for bit; with weights of zero, the bias."""
+    """One row, two rows, the kernels for few and for many rows, and the batch kernel for all from 3 rows on where its plan is
+    set, with and without splits along k: the result without bias plus the bias in fp16, bit for bit; with weights of zero, the bias."""
     import torch
     from lutgemm import synth
     w, W = make(lutgemm, synth, k, n, q, g, offset=offset, seed=k + n)

@@ -141,8 +141,8 @@ def test_cfg4_full_size_all_batches(lutgemm, oracle, device, layer):
     (64, 70000, 8, 64, True),
 ])
 def test_extreme_aspect_ratios(lutgemm, oracle, device, k, n, q, g, offset):
-    """Very wide and very deep weights, every kernel family (one row, two rows, the batch kernel in
-    one and in two passes), rows and columns entry; the whole output is compared with the oracle."""
+    """Very wide and very deep weights, every kernel family (one row, two rows, 3 to 16, more), rows and
+    columns entry; the whole output is compared with the oracle."""
     from lutgemm import synth
     w = synth.make_weight(k, n, q, g, offset=offset, seed=k % 1000 + n % 1000)
     W = lutgemm.BCQWeight(w["bW"], w["alpha"], k, n, q, k // g, w["q_bias"])

@@ -142,8 +142,8 @@ def test_batched_rows_and_columns(lutgemm, oracle, device, m):
 def test_row_pairs_equal_single_rows_bit_for_bit(lutgemm, oracle, device, k, n, q, g, offset):
     """A two-row pass must give each row exactly as a one-row launch with the same plan produces
     it (same tables, same order of accumulation), for every scale layout (g % 128, % 64, % 32),
-    with and without offset, for several plans.  Five rows go through the batch kernel in one pass,
-    within the tolerance."""
+    with and without offset, for several plans.  Five rows go through the weight in one pass on the
+    matrix cores, within the tolerance."""
     from lutgemm import synth
     m = 5
     w, W = make(lutgemm, synth, k, n, q, g, offset=offset, seed=k + q)
@@ -201,7 +201,7 @@ def test_batch_kernel_shapes(lutgemm, oracle, device, k, n, q, g, offset):
     eight) and every scale-group layout (one, two or four groups per 128 k), with and
     without offset, k that ends inside a k-block, n that ends inside a batch, one to many k-splits,
     row counts below, at and above the 16 rows of a pass; deterministic; row- and column-batched
-    forms agree."""
+    forms agree.  Each with the kernel that takes the call by itself and with the batch kernel, by a plan set for it."""
     from lutgemm import synth
     w, W = make(lutgemm, synth, k, n, q, g, offset=offset, seed=k + 5 * q)
     ts = (k + 511) // 512
@@ -210,20 +210,25 @@ def test_batch_kernel_shapes(lutgemm, oracle, device, k, n, q, g, offset):
         x = synth.make_x(m, k, seed=n + m)
         truth = truth_of(oracle, w, x)
         W.set_plan(waves, min(ks, ts))
-        y = run_matvec(lutgemm, W, x, device)
-        assert_within_tolerance(y, truth, "m=%d plan=%s" % (m, W.plan()))
-        assert np.array_equal(y.view(np.uint16), run_matvec(lutgemm, W, x, device).view(np.uint16))
-        yc = run_matvec(lutgemm, W, x, device, cols=True)
-        assert np.array_equal(y.view(np.uint16), yc.view(np.uint16))
+        per_split = -(-ts // max(1, ks))
+        for batch_plan in ((0, 0), (8, -(-ts // per_split))):
+            W.set_batch_plan(*batch_plan)
+            y = run_matvec(lutgemm, W, x, device)
+            assert_within_tolerance(y, truth, "m=%d plan=%s" % (m, W.plan(m)))
+            assert np.array_equal(y.view(np.uint16), run_matvec(lutgemm, W, x, device).view(np.uint16))
+            yc = run_matvec(lutgemm, W, x, device, cols=True)
+            assert np.array_equal(y.view(np.uint16), yc.view(np.uint16))
     # unit activations in a batch: rows of the dequantised weight, bit for bit (sums of a few fp16 numbers are exact)
     e = np.zeros((5, k), np.float16)
     rows = [0, 7, k // 2 + 3, k - 1, 129 % k]
     for i, r in enumerate(rows):
         e[i, r] = 1
-    ye = run_matvec(lutgemm, W, e, device)
     dense = oracle.dense_weight_f64(w["bW"], w["alpha"].astype(np.float16),
                                     w["q_bias"].astype(np.float16) if offset else None)
-    assert np.array_equal(ye.view(np.uint16), dense[rows].astype(np.float16).view(np.uint16))
+    for batch_plan in ((0, 0), (8, 1), (8, ts)):
+        W.set_batch_plan(*batch_plan)
+        ye = run_matvec(lutgemm, W, e, device)
+        assert np.array_equal(ye.view(np.uint16), dense[rows].astype(np.float16).view(np.uint16))
     W.close()
 
 
@@ -303,8 +308,8 @@ def test_autotune_keeps_results_and_picks_a_valid_plan(lutgemm, oracle, device):
     # two-row passes keep a measured plan of their own; their rows must still equal the one-row launches
     y = run_matvec(lutgemm, W, x[:2], device)
     assert np.array_equal(y.view(np.uint16), singles[:2].view(np.uint16))
-    # the batch kernel (measured plans for passes of up to 8 and of 9..16 rows): another order
-    # of additions, same tolerance
+    # 3 to 16 rows (measured plans for up to 8 and for 9..16 of them): another order of additions,
+    # same tolerance
     for m in (3, 5, 12):
         bp = W.plan(m)
         assert 8 <= bp["waves"] <= 16 and bp["workgroups"] == -(-(n // 32) // bp["waves"]) * bp["k_splits"], bp
@@ -367,7 +372,7 @@ def test_device_round_trip_and_dequantize(lutgemm, oracle, device):
 def test_random_shapes_plans_and_batches(lutgemm, oracle, device):
     """Sixty seeded random problems: ragged k (any multiple of 32, so the last k-block and the
     last scale group are partial), odd n, every q, group sizes with all three scale layouts,
-    with / without offset, 1..33 rows (one-row, two-row and batch kernels, more than one pass),
+    with / without offset, 1..33 rows (the kernels for one, two, 3 to 16 and more rows),
     random launch plans."""
     from lutgemm import synth
     rng = np.random.default_rng(20240607)
@@ -499,7 +504,7 @@ def test_matvec_many_shares_launches_and_keeps_every_result(lutgemm, oracle, dev
 
 
 def test_matvec_many_fuses_batches(lutgemm, oracle, device):
-    """Independent batches of 3 to 16 rows share one launch of the batch kernel, whatever their
+    """Independent batches of 3 to 16 rows share one launch, whatever their
     shapes and row counts (more rows than the launch has wavefronts per workgroup included); runs
     are cut where the kind of entry changes (one row, two rows, more than 16, another plane count),
     where a handle repeats and where an entry reads an earlier output.  Every entry meets the
@@ -845,7 +850,7 @@ def test_one_handle_from_many_host_threads(lutgemm, oracle, device):
     """Eight host threads, each with a stream of its own, launch on one handle at the same time (the
     binding releases the interpreter lock during a call): a set that one thread has claimed and is
     launching on is not handed to another thread's stream in between, so every result equals the
-    same launch issued alone, whatever the row count (table-lookup, two-row and batch kernels)."""
+    same launch issued alone, whatever the row count (the kernels for one, two and 3 to 16 rows)."""
     import threading
     import torch
     from lutgemm import synth

@@ -70,7 +70,7 @@ def test_large_batches_take_the_dense_route(lutgemm, oracle, device):
     assert np.abs(y_dense.cpu().double().numpy() - truth).max() <= 3e-2   # fp16 weight + library GEMM
 
 
-@pytest.mark.parametrize("rows", [2, 5])   # the two-row table kernel and the batch kernel
+@pytest.mark.parametrize("rows", [2, 5])   # the two-row table kernel and the kernel for 3 to 16 rows
 def test_operator_replays_from_a_hip_graph(lutgemm, device, rows):
     from lutgemm import quantize, torch_ops
     lin, gen = _layer(3, bias=False)
