@@ -40,8 +40,8 @@ typedef enum lutgemm_status {
 
 /* Opaque packed weight: device-resident sign tiles, scales and offsets plus the launch plan
  * and the workspace of the launching streams (split-k accumulators: 64-bit words, one per output and
- * activation row of a pass; staging rows of the column-batched form; partial sums of calls of more than 16 rows).  Stands in for class lutGEMM::nQWeight_fp16
- * (lutGEMM/include/nQWeight_fp16.h:27-52). */
+ * activation row of a pass; staging rows of the column-batched form; partial sums of calls of 3 and more rows).
+ * Stands in for class lutGEMM::nQWeight_fp16 (lutGEMM/include/nQWeight_fp16.h:27-52). */
 typedef struct lutgemm_weight lutgemm_weight;
 
 /* Shape record returned by lutgemm_weight_info(); field meanings follow the public data
@@ -56,8 +56,8 @@ typedef struct lutgemm_weight_info_t {
     size_t sign_bytes;   /* k*n*q/8: packed sign bytes streamed per matvec (unpadded) */
     size_t scale_bytes;  /* num_groups*q*n*2 (unpadded) */
     size_t offset_bytes; /* num_groups*n*2 or 0 (unpadded) */
-    size_t device_bytes; /* bytes of device memory held by the handle: tiles, split-k accumulators and
-                            staging rows of every stream set allocated so far */
+    size_t device_bytes; /* bytes of device memory held by the handle: tiles, split-k accumulators, staging rows
+                            and room for partial sums of every stream set allocated so far */
 } lutgemm_weight_info_t;
 
 /* Build a packed weight from HOST arrays in the layout above (floats are rounded to fp16,
@@ -119,9 +119,10 @@ int lutgemm_weight_info(const lutgemm_weight *w, lutgemm_weight_info_t *info);
  * the caller, as for any stream.
  * Non-finite values follow IEEE arithmetic whatever the launch plan: a NaN activation gives NaN
  * outputs, infinite partial sums give an infinity of their sign, or NaN if both signs occur.  With
- * more than one k-split the partial sums are added as fixed-point integers (2^-24 resolution);
- * a finite partial sum beyond +-4.1e6 (64 times binary16's range) counts as an infinity (up to 16 rows; launches of more
- * add the fp32 partial sums themselves).  From three rows on an infinite scale multiplies sums of 128 or 64 activations
+ * more than one k-split the partial sums of one and two rows are added as fixed-point integers (2^-24 resolution);
+ * a finite partial sum beyond +-4.1e6 (64 times binary16's range) counts as an infinity.  The same holds for 3 to 16 rows where
+ * they go through the accumulators (few outputs, no memory for partial sums, the batch kernel, lists); other launches of 3 and
+ * more rows add the fp32 partial sums themselves, in fp32 and in the order of k.  From three rows on an infinite scale multiplies sums of 128 or 64 activations
  * where the group size is a multiple of that, and single activations where it is not: infinities of both signs give NaN.
  * More than 16 rows against a weight with non-finite scales or offsets are taken 16 per pass, with the results of such
  * passes. */
@@ -135,7 +136,8 @@ int lutgemm_matvec_bias(const lutgemm_weight *w, const void *x, void *y, const v
 
 /* lutgemm_matvec without any allocation, for callers that cannot allocate: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the
- * reference.  Same arguments, same kernels and bit-identical results; the only difference is where
+ * reference.  Same arguments, same kernels and bit-identical results (but where the device has no memory for the partial sums of
+ * a set: that changes the results of lutgemm_matvec, see there); the only difference is where
  * the split-k accumulators and partial sums live: not in the handle's allocation but in static device arrays of
  * the library (24 MiB on every device the library runs on, held until the process ends), whose
  * addresses are looked up once per device.  Limit: n <= 65,536 outputs (LUTGEMM_ERR_UNSUPPORTED
@@ -160,8 +162,8 @@ int lutgemm_matvec_cols(const lutgemm_weight *w, const void *x, void *y, int m, 
  * computes ys[i] = xs[i] * ws[i] with batch ms[i] exactly as lutgemm_matvec would, and the results
  * are those of the entries executed in order.  Consecutive entries that do not depend on each other
  * share ONE kernel launch (up to 32 per launch): entries that all have one activation row, that all
- * have two, or that all have 3 to 16 rows (the batch kernel), with the same q /
- * offset / group layout, distinct handles, and no output overlapping an input or output of another
+ * have two, or that all have 3 to 16 rows and are taken by the same kernel (the kernel for few rows, or the batch kernel), with
+ * the same q / offset / group layout, distinct handles, and no output overlapping an input or output of another
  * entry of the launch.  The workgroups of such entries follow each other in one grid, so the memory
  * system stays busy while single workgroups start and finish, and the launch overhead is paid
  * once.  Such a launch has a shape of its own (wavefronts per workgroup, split along k) chosen for
@@ -254,7 +256,8 @@ int lutgemm_weight_plan_for(const lutgemm_weight *w, int m, int *workgroups, int
                             int *k_splits, int *k_blocks_per_group);
 
 /* Override the launch plan of the table-lookup kernels, for one-row and two-row launches alike (0
- * keeps the automatic choice for that field; the batch kernel has lutgemm_weight_set_batch_plan);
+ * keeps the automatic choice for that field; the batch kernel has lutgemm_weight_set_batch_plan, the kernels for few and for
+ * many rows choose for themselves);
  * synchronises the device first.  Returns LUTGEMM_ERR_BAD_SHAPE if the request cannot be launched
  * (1..12 wavefronts per workgroup, 1..min(k/512 rounded up, 128) k-splits). */
 int lutgemm_weight_set_plan(lutgemm_weight *w, int waves_per_group, int k_splits);

@@ -459,7 +459,7 @@ RowsPlan choose_rows_plan(const Shape &s, int cus, int m, bool may_split)
     return best;
 }
 
-// Shapes that the kernel for few rows takes: one scale group per row of a tile, and rows that 32 bits address.
+// Shapes that the kernel for few rows takes: 16 rows of activations that 32 bits address in bytes.
 bool few_shape(const Shape &s) { return s.k <= kMaxRowsK; }
 
 // A handle's device memory belongs to the device that was current when it was created.
@@ -504,10 +504,12 @@ size_t few_room(const lutgemm_weight *w)
 }
 
 // The memory of a set in one piece: split-k words, kStagedColumns staged columns, `units` units of partial sums; set 0 lies
-// behind the tiles in theirs.  Every hipMalloc costs 20 to 40 us and every hipFree, which waits for the device, about 80: with
-// one allocation instead of four, a 4096 x 16384 weight of four planes is made from host arrays, expanded and freed in 2190
-// instead of 2270 us, and as no room is allocated behind a launch the first call of 12 columns on a new 7168 x 28672 weight
-// takes 68 us instead of 124 (of 8 rows on the four weights of a 12288 block: 195 instead of 282).  Pieces below
+// behind the tiles in theirs.  Every hipMalloc costs 20 to 40 us and every hipFree, which waits for the device, about 80, which a
+// 4096 x 16384 weight of four planes, made from host arrays, expanded and freed in 2100 us, does not show beyond its noise; but as
+// no room is allocated behind a launch the first call of 12 columns on a new 7168 x 28672 weight
+// takes 68 us instead of 124 (of 8 rows on the four weights of a 12288 block: 195 instead of 282).  The price is memory: the room
+// is there from creation, also for a program that never passes three rows (4096 x 4096, three planes: 2.0 MiB beside 6.75 of
+// tiles; 12288 x 12288: 3.75 beside 60.75).  Pieces below
 // kRuntimeChunk cost next to nothing, as the runtime cuts them from chunks of its own: sign tiles that are such a piece stay
 // one where all together would not be (2048 x 2048, three planes, made, expanded and freed: 185 us, in one allocation 227, in four 187).
 constexpr size_t kRuntimeChunk = (size_t)2 << 20;

@@ -23,11 +23,11 @@ struct MatvecArgs {
     int y_stride;           // output j goes to y[j * y_stride]
     // rows == 2: a second activation row at x + x_row_stride goes to y + y_row_stride in the
     // same pass (strides in fp16 elements), with its accumulators at accum + accum_row_stride
-    int rows;               // 1 or 2 activation rows (0 selects the read probe); 1..kBatchRows for launch_batch
+    int rows;               // 1 or 2 activation rows (0 selects the read probe); 1..kBatchRows for launch_few and launch_batch
     long long x_row_stride, y_row_stride, accum_row_stride;
 };
 
-// Activation rows the batch kernel takes in one pass over the weight (rows r at x + r * x_row_stride
+// Activation rows the kernel for few rows and the batch kernel take in one pass over the weight (rows r at x + r * x_row_stride
 // go to y + r * y_row_stride, with split-k accumulators at accum + r * accum_row_stride).
 constexpr int kBatchRows = 16;
 

@@ -15,7 +15,7 @@
 //  * A matrix instruction holds the vector unit of its SIMD for 16 cycles and takes one other vector instruction for nothing,
 //    every further one in 4 cycles (few_body.h), so indices and activations are made one instruction behind each matrix
 //    instruction, and addresses are scalar (buffer loads).
-// What bounds it: power.  7168 x 7168, 3 planes, 256 rows (RT = 2, KW = 1): 4.8 million matrix instructions in 77 us; a loop of
+// What bounds it: power.  7168 x 7168, 3 planes, 256 rows (RT = 2, KW = 1): 4.8 million matrix instructions in 73 to 75 us; a loop of
 // nothing but them with such operands takes 50 us on the whole device (10.7 ns each and SIMD, 6.9 on a few compute units), and
 // the compute units that the plan leaves idle, start and end the rest.  Before the instructions were spread: 82 to 89 us; 12288 x
 // 12288, 3 planes, 48 rows (RT = 3, five splits): 58 -> 49 us.  The launch replaced 16 of the batch kernel: 257 us.

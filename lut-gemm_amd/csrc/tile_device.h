@@ -1,4 +1,4 @@
-// Device-side pieces shared by the matvec kernels (kernels.hip) and the batch kernel (batch.hip):
+// Device-side pieces shared by the matvec kernels (kernels.hip) and the kernels for 3 and more rows (*_body.h):
 // the registers of one weight tile with their loads, and the split-k completion of an output.
 #ifndef LUTGEMM_TILE_DEVICE_H
 #define LUTGEMM_TILE_DEVICE_H

@@ -23,18 +23,17 @@ def default_dense_threshold(weight, keep_dense=False):
     """Rows up to which the packed route beats dequantised weight + library GEMM (measured on MI355X
     at k = n = 12288 and at k = 7168, n = 28672; LutLinear(dense_threshold=...) overrides).
 
-    A pass of the batch kernel over up to 16 rows costs 22 / 24 / 30 / 36 us for one to four planes
-    and 41 / 43 / 50 / 57 us for five to eight (k = n = 12288).  The dense route costs the
+    The lines come from passes of the batch kernel, which layers took when they were drawn: up to 16 rows at
+    22 / 24 / 30 / 36 us for one to four planes and 41 / 43 / 50 / 57 us for five to eight (k = n = 12288).  The dense route costs the
     dequantisation (75 us up to four planes, 97-130 us for five to eight) plus the GEMM (50-56 us up
     to 32 rows), so by default it only pays from the number of passes on that costs as much:
     80 rows for one or two planes, 64 for three, 48 beyond.  A layer that keeps its dense copy
     (keep_dense) pays the GEMM alone: 32 rows for one or two planes, 16 for three to seven, and
     eight planes leave the packed route from three rows on (57 against 50 us).
 
-    3 to 16 rows take less by now (kernel for few rows) and more no longer take passes of 16, so the packed route would stay ahead for longer (12288 x 12288,
-    three planes, 160 rows: 130 against 192 us).  The lines are kept all the same (those of layers
-    with a dense copy rest on passes of 16 rows as well), because the routes are not
-    interchangeable: the dense one passes gradients to x, follows autocast, can be captured on a stream that has not
+    3 to 16 rows take the kernel for few rows by now (12288 x 12288, two planes, 8 rows 18 us; four planes, 16 rows 32) and more
+    no longer take passes of 16, so the packed route would stay ahead for longer (12288 x 12288, three planes, 160 rows: 130
+    against 192 us).  The lines are kept all the same, because the routes are not interchangeable: the dense one passes gradients to x, follows autocast, can be captured on a stream that has not
     launched on the handle, and rounds the weight to fp16, so its results differ by some 4e-4 of their norm."""
     q = weight.nb
     if keep_dense:
